@@ -44,8 +44,8 @@ const int CXH[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
 // means, J (their x-fluxes), 2 unused; and per row nb block records of
 // BLK_STRIDE floats, X over each 64-node block of the row
 constexpr int kRefStride = 8;
+constexpr int kDftLds = 32768;             // LDS bytes of a narrow rows' direct-DFT tile
 constexpr int kMaxTriChunks = TRI_WG / 2;  // the plan keeps G = TRI_WG / C >= 2 modes per work-group
-constexpr int kDftLds = 32768;             // LDS bytes of a direct-DFT tile
 
 // stored value + ref[d][y][x] = population (FP32 storage; 0 for FP64)
 std::vector<double> ref_offsets(ekpnp_ctx* c, int channel, int species, hipError_t* err);
@@ -366,10 +366,14 @@ hipError_t apply_lbm_tiles(ekpnp_ctx* c, int wrows) {
   return hipSuccess;
 }
 
+// x-transform of a channel, in the order of the FFT tile table: 0 power-of-two
+// FFT, 1 matrix-core direct DFT, 2 direct DFT of narrow rows
+int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2; }
+
 // Poisson work decomposition.  x-FFT: a work-group transforms whole rows,
-// up to fft_elems complex values (power-of-two channels; the direct DFT of
-// other widths takes one row per work-group); power-of-two tiles come first
-// in the table.  Tridiagonal: each column is cut into C = 2^k chunks of at
+// up to fft_elems complex values (power-of-two channels and narrow others; the
+// matrix-core direct DFT takes 16 or 32 rows per work-group); the tiles are
+// sorted by family (x_family).  Tridiagonal: each column is cut into C = 2^k chunks of at
 // most about tri_rows rows (8 <= C <= 128), G = TRI_WG / C modes per
 // work-group.  Rebuilding drops the cached graphs (their grids change).
 hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft_persist) {
@@ -377,7 +381,8 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
   c->tri_tiles.clear();
   unsigned lds_pow2 = 16, lds_dft = 16, lds_pow2_tw = 16;  // rows; rows + quadrant table
   unsigned lds_pow2_t2 = 16;                                 // rows + two-level table
-  int n_fft_pow2 = 0;
+  int n_fft_pow2 = 0, n_fft_dft = 0, groups_fwd = 1, groups_inv = 1;
+  unsigned dft_lds = 16;
   // wide row-pair kernels: every power-of-two channel has rows of
   // N = FFT_PAIR_WIDE_S * FFT_WG_ROWS complex values (nx = 8192), asked for
   // as fft_elems = N with the row-pair family; tiles of two rows, one row
@@ -393,12 +398,12 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
   wide = wide && n_pow2_chan > 0;
   const unsigned wide_lds = (unsigned)((kWideN + tw2_count(2 * kWideN)) * sizeof(double2));
   wide = wide && wide_lds <= (unsigned)c->max_lds;
-  for (int pass = 0; pass < 2; ++pass) {
+  for (int pass = 0; pass < 3; ++pass) {
     for (int i = 0; i < c->nchan; ++i) {
       ChanDesc& d = c->desc[i];
-      if ((pass == 0) != (d.pow2 == 1)) continue;
+      if (pass != x_family(d)) continue;
       const int M = d.ny - 2;
-      int rows = 1;
+      int rows = 1, dft_wr = 0;
       if (d.pow2) {
         const int N = d.nx / 2;
         rows = wide ? 2 : std::max(1, std::min(std::min(M, FFT_MAX_ROWS), fft_elems / N));
@@ -408,8 +413,17 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
         lds_pow2_tw = std::max<unsigned>(lds_pow2_tw, (unsigned)((padded + d.nx / 4) * sizeof(double2)));
         const int t2 = tw2_count(d.nx);  // the kernels' two-level twiddle table
         lds_pow2_t2 = std::max<unsigned>(lds_pow2_t2, (unsigned)((padded + t2) * sizeof(double2)));
+      } else if (d.nx >= DFT_MIN_NX) {
+        // matrix-core direct DFT: 16 rows per row tile, the four waves of a
+        // work-group split between rows and columns by the width (k_dft_fwd)
+        dft_wr = d.nx <= 32 ? 2 : 1;
+        rows = 16 * dft_wr;
+        dft_lds = std::max(dft_lds, dft_lds_bytes(d.nx));
+        const int cols = 64 / dft_wr;
+        groups_fwd = std::max(groups_fwd, (d.nk + cols - 1) / cols);
+        groups_inv = std::max(groups_inv, (d.nx + cols - 1) / cols);
       } else {
-        // direct-DFT tiles: as many whole rows as fit fft_elems values and
+        // narrow rows: as many whole rows as fit fft_elems values and
         // kDftLds bytes of LDS (a row of nx | 1 right-hand-side values, or
         // its nk spectrum values)
         const int per_row = (int)std::max((d.nx | 1) * sizeof(double), d.nk * sizeof(double2));
@@ -419,10 +433,11 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
       d.fft_rows = rows;
       c->ctiles[i].fft_first = (int)c->fft_tiles.size();
       for (int y0 = 1; y0 <= M; y0 += rows)
-        c->fft_tiles.push_back(make_int4(i, y0, std::min(rows, M + 1 - y0), 0));
+        c->fft_tiles.push_back(make_int4(i, y0, std::min(rows, M + 1 - y0), dft_wr));
       c->ctiles[i].fft_count = (int)c->fft_tiles.size() - c->ctiles[i].fft_first;
     }
     if (pass == 0) n_fft_pow2 = (int)c->fft_tiles.size();
+    if (pass == 1) n_fft_dft = (int)c->fft_tiles.size() - n_fft_pow2;
   }
   int tri_lmax = 1;
   for (int i = 0; i < c->nchan; ++i) {
@@ -466,7 +481,11 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
                       fft_one_tile_blocks_per_cu(true, lds_pow2_tw) >= fft_one_tile_blocks_per_cu(false, lds_pow2_t2))
                          ? 1 : 0;
   c->sb.fft_lds_pow2 = c->sb.fft_tw_lds ? lds_pow2_tw : lds_pow2_t2;
+  c->sb.n_fft_dft = n_fft_dft;
+  c->sb.dft_lds = dft_lds;
   c->sb.fft_lds_dft = lds_dft;
+  c->sb.dft_groups_fwd = groups_fwd;
+  c->sb.dft_groups_inv = groups_inv;
   c->sb.tri_lmax = tri_lmax;
   // the persistent kernels take tiles of <= FFT_PERSIST_ELEMS values and keep
   // twiddles in LDS
@@ -533,7 +552,8 @@ hipError_t enqueue_poisson(ekpnp_ctx* c, int only_channel) {
     const ChannelTiles& t = c->ctiles[only_channel];
     b.fft_tiles = c->d_fft_tiles + t.fft_first;
     b.n_fft_tiles = t.fft_count;
-    b.n_fft_pow2 = c->desc[only_channel].pow2 ? t.fft_count : 0;
+    b.n_fft_pow2 = x_family(c->desc[only_channel]) == 0 ? t.fft_count : 0;
+    b.n_fft_dft = x_family(c->desc[only_channel]) == 1 ? t.fft_count : 0;
     b.tri_tiles = c->d_tri_tiles + t.tri_first;
     b.n_tri_tiles = t.tri_count;
   }

@@ -37,6 +37,18 @@ constexpr unsigned FFT_LDS_PERSIST = (FFT_PERSIST_ELEMS + FFT_PERSIST_ELEMS / 2)
 constexpr int TRI_WG = 256;       // lanes of a tridiagonal work-group (modes x chunks)
 constexpr int MAX_NX = 8192;      // LDS-resident x-rows (64 KiB of complex FP64)
 constexpr int MAX_NX_DFT = 2048;  // non-power-of-two rows use a direct DFT
+// Narrower rows that are no power of two (and 2, 4) take the one-output-per-lane
+// direct DFT, wider ones the matrix-core one: at 10 x 101 the Poisson stages
+// take the same time either way, and 512 channels of nx = 4 run 10 % faster
+// on the former (their 16 x 16 tiles would be mostly padding); from 24 nodes on
+// the matrix-core kernels are faster (nx = 48: forward 10.7 -> 8.2 us)
+constexpr int DFT_MIN_NX = 24;
+constexpr int DFT_WG = 256;       // lanes of a matrix-core direct-DFT work-group
+constexpr int DFT_CHUNK = 2048;   // FP64 values of a staged chunk: 16 wr rows x columns (or modes, two values each)
+// LDS of a direct-DFT work-group: the twiddle table, then one chunk, its rows
+// padded by at most two values
+__host__ __device__ constexpr int dft_tw_len(int nx) { return (nx + 3) & ~3; }
+__host__ __device__ constexpr unsigned dft_lds_bytes(int nx) { return dft_tw_len(nx) * 16 + DFT_CHUNK * 8 + 1024; }
 constexpr int TRI_LMAX = 16;              // rows per tridiagonal chunk (one lane)
 constexpr int MAX_INTERIOR_ROWS = 2048;  // 128 chunks x 16 rows per tridiagonal column
 // FP32 storage references along x: one record of BLK_STRIDE floats (rho,
@@ -96,7 +108,7 @@ struct StepBuffers {
   const int2* lbm_gen_tiles;
   int n_lbm_gen_tiles;
   int lbm_wrows;                // row-kernel interior tiles: 0 consecutive blocks, else rows per tile (2, 4)
-  const int4* fft_tiles;        // (channel, first row, rows, 0) per FFT work-group
+  const int4* fft_tiles;        // (channel, first row, rows, matrix-core DFT: row tiles) per FFT work-group
   int n_fft_tiles;
   int n_fft_pow2;               // the first n_fft_pow2 tiles are power-of-two rows
   int fft_persist;              // power-of-two tiles by the persistent kernels
@@ -105,7 +117,10 @@ struct StepBuffers {
                                 //   buffer, the second row in registers, the two-level table)
   int fft_grid;                 // work-groups of the persistent kernels
   unsigned fft_lds_pow2;        // dynamic LDS bytes of the Stockham kernels
-  unsigned fft_lds_dft;         // dynamic LDS bytes of the direct-DFT kernels
+  int n_fft_dft;                // then come the tiles of the matrix-core direct DFT, then the narrow rows'
+  unsigned dft_lds;             // dynamic LDS bytes of the matrix-core direct-DFT kernels
+  int dft_groups_fwd, dft_groups_inv;  // column groups of the widest such channel: modes, nodes
+  unsigned fft_lds_dft;         // dynamic LDS bytes of the narrow rows' direct-DFT kernels
   int fft_tw_lds;               // the power-of-two kernels stage twiddles in LDS
   const int2* tri_tiles;        // (channel, first mode) per tridiagonal work-group
   int n_tri_tiles;

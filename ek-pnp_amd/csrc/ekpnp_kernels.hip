@@ -1658,6 +1658,323 @@ __global__ __launch_bounds__(FFT_WG_ROWS) void k_fft_inv(StepBuffers b, const in
 }
 
 // ---------------------------------------------------------------------------
+// Direct real DFT of rows of at least DFT_MIN_NX nodes whose width is no power
+// of two, on the FP64 matrix cores.  v_mfma_f64_16x16x4 adds its four products to the
+// accumulator one after the other, k = 0, 1, 2, 3, each a fused multiply-add
+// (checked bit for bit against an fma chain), so a 16 x 16 tile of outputs
+// accumulated over n = 0..nx-1 is the plain sum
+//   X[k] = sum_n v[n] W^{kn}, acc = fma(v[n], W^{kn}, acc) in that order,
+// for 16 rows and 16 modes at once.  The forward transform is such a product;
+// the inverse adds 2 (Re z Re w + Im z Im w) mode by mode, one instruction
+// forming 256 of these terms (two of its four products used) and a vector
+// fma each adding them to the outputs.
+// Bound: the matrix pipe, 64 clocks per instruction (two per 16 x 16 x 4 products
+// forward, one per mode and 16 x 16 nodes inverse), and the vector instructions
+// between them, which the FP64 matrix instructions do not overlap: the
+// twiddles come from an LDS table through index chains of three instructions.
+// One output per lane with every twiddle read through the cache, the narrow
+// rows' kernel, was bound by those reads.  Forward + inverse, us, before and
+// after: 100 x 101 18 + 16 -> 9.5 + 9.3, 500 x 201 61 + 61 -> 19.5 + 21.2,
+// 1000 x 401 262 + 262 -> 33 + 59, 1999 x 1001 2204 + 2223 -> 163 + 399.  A
+// chirp-z transform (two padded FFTs) would take 18 + 15 at 1000 x 401, but it
+// changes the rounding of psi, and with FP32 storage a change in psi's last
+// bits re-draws the roundings of the populations: u differs by 4e-9 after 100
+// steps, where the sums in this order keep every bit.
+//
+// Work-group: 4 waves, wr row tiles x 4 / wr column tiles of 16 (t.w = wr: 2
+// for nx <= 32, else 1); blockIdx.y walks the groups of
+// column tiles (modes forward, nodes inverse), groups past the channel's
+// last column return.  Operands pass through LDS in chunks, the next chunk's
+// loads in flight while the current one is multiplied.
+// ---------------------------------------------------------------------------
+typedef double d4 __attribute__((ext_vector_type(4)));
+constexpr int DFT_LD_PAD = 2;               // row padding of a forward chunk (bank spread)
+constexpr int DFT_MODES = DFT_CHUNK / 32;   // modes of an inverse chunk, over wr
+
+// a - b, never contracted with the product that made a (the right-hand side
+// rounds -pc rho_e before the wall lift is taken off, as rhs_at's branches do)
+__device__ __forceinline__ double sub_pinned(double a, double b) {
+#pragma clang fp contract(off)
+  return a - b;
+}
+
+// (i + d) mod n for i, d < n: one of the two candidates wraps below zero
+__device__ __forceinline__ unsigned wrap_add(unsigned i, unsigned d, unsigned n) { return min(i + d, i + d - n); }
+
+// tw[i] = src[i], i < nx <= MAX_NX_DFT, every load issued before the first use
+__device__ __forceinline__ void dft_load_table(double2* tw, const double2* __restrict__ src, int nx) {
+  constexpr int SLOTS = MAX_NX_DFT / DFT_WG;
+  double2 t[SLOTS];
+#pragma unroll
+  for (int c = 0; c < SLOTS; ++c) t[c] = src[min((int)threadIdx.x + c * DFT_WG, nx - 1)];
+#pragma unroll
+  for (int c = 0; c < SLOTS; ++c) {
+    const int i = threadIdx.x + c * DFT_WG;
+    if (i < nx) tw[i] = t[c];
+  }
+}
+
+// interleave n matrix instructions with valu vector and ds LDS-read
+// instructions each (scheduling hint for the enclosing block)
+template <int N, int VALU, int DS>
+__device__ __forceinline__ void interleave_mfma() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, DS, 0);
+  }
+}
+
+__global__ __launch_bounds__(DFT_WG) __attribute__((amdgpu_waves_per_eu(2))) void k_dft_fwd(StepBuffers b, const int4* __restrict__ tiles,
+                                                    const ChanDesc* __restrict__ chans) {
+  extern __shared__ double2 lds[];
+  const int4 t = tiles[blockIdx.x];
+  const ChanDesc* __restrict__ cd = chans + t.x;
+  const int nx = cd->nx, nk = cd->nk, y0 = t.y, rows = t.z, wr = t.w;
+  const int cols = 64 / wr;  // modes of this work-group
+  if (!cd->active || (int)blockIdx.y * cols >= nk) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave & (4 / wr - 1), rt = wave / (4 / wr);  // column tile, row tile
+  const int k = (int)blockIdx.y * cols + 16 * wm + (lane & 15), q = lane >> 4;
+  const bool work = (int)blockIdx.y * cols + 16 * wm < nk && 16 * rt < rows;
+  double2* tw = lds;
+  double* v = reinterpret_cast<double*>(lds + dft_tw_len(nx));
+  const double2* __restrict__ twg = b.tw + cd->tw_off;
+  const double* __restrict__ re = b.rho_e + cd->fld_off;
+  const double* __restrict__ Wl = b.walls + cd->wall_off;
+  const long long ws = b.walls_stride;
+  const double neg_pc = -cd->pc_dy2;
+  // chunk: 16 wr rows x 2^lgc columns (at least one group of 16)
+  int lgc = 4;
+  while ((1 << lgc) < nx && (32 * wr << lgc) <= DFT_CHUNK) ++lgc;
+  const int CH = 1 << lgc, total = 16 * wr * CH, ld = CH + DFT_LD_PAD;
+  constexpr int SLOTS = DFT_CHUNK / DFT_WG;
+  // A lane stages column nl of every 256 >> lgc -th row.  Raw charge and wall
+  // potentials at clamped places, unconditionally: nothing waits for a load
+  // before the chunk is written to LDS, where the right-hand side (rhs_at)
+  // is formed.
+  const int nl = tid & (CH - 1), r0 = tid >> lgc, dr = DFT_WG >> lgc;
+  const bool lo = y0 == 1, hi = y0 + rows - 1 == cd->ny - 2;
+  double pf[SLOTS], wlo = 0.0, whi = 0.0;
+  auto prefetch = [&](int n0) {
+    const int n = min(n0 + nl, nx - 1);
+    const double* __restrict__ col = re + (long long)y0 * nx + n;
+#pragma unroll
+    for (int c = 0; c < SLOTS; ++c) pf[c] = col[min(r0 + c * dr, rows - 1) * nx];
+    if (lo) wlo = Wl[W_PSI_LO * ws + n];
+    if (hi) whi = Wl[W_PSI_HI * ws + n];
+  };
+  prefetch(0);
+  dft_load_table(tw, twg, nx);
+  // lane (row = lane % 16, q): value n = 4 s + q; (mode = lane % 16, q): its
+  // twiddle.  Four steps at a time, the next group's operands on their way
+  // from LDS during the current group's products; columns past nx hold 0.
+  d4 ar = {0.0, 0.0, 0.0, 0.0}, ai = {0.0, 0.0, 0.0, 0.0};
+  const int kk = work && k < nk ? k : 0;
+  const unsigned step = 16u * (unsigned)((16LL * kk) % nx), wrap = 16u * nx;
+  unsigned idx[4];  // 16 (n k mod nx) of the next group's steps
+#pragma unroll
+  for (int u = 0; u < 4; ++u) idx[u] = 16u * (unsigned)((long long)(4 * u + q) * kk % nx);
+  const char* twb = reinterpret_cast<const char*>(tw);
+  const double* va = v + (16 * rt + (lane & 15)) * ld + q;
+  double2 w[2][4];
+  double a[2][4];
+  auto load = [&](int s, double2(&wg)[4], double(&ag)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ag[u] = va[4 * (s + u)];
+      wg[u] = *reinterpret_cast<const double2*>(twb + idx[u]);
+      idx[u] = wrap_add(idx[u], step, wrap);
+    }
+  };
+  auto mul = [&](const double2(&wg)[4], const double(&ag)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ar = __builtin_amdgcn_mfma_f64_16x16x4f64(ag[u], wg[u].x, ar, 0, 0, 0);
+      ai = __builtin_amdgcn_mfma_f64_16x16x4f64(ag[u], wg[u].y, ai, 0, 0, 0);
+    }
+  };
+  for (int n0 = 0; n0 < nx; n0 += CH) {
+    __syncthreads();  // the previous chunk has been read
+#pragma unroll
+    for (int c = 0; c < SLOTS; ++c) {
+      const int r = r0 + c * dr;
+      double rhs = neg_pc * pf[c];
+      if (lo && r == 0) rhs = sub_pinned(rhs, wlo);
+      if (hi && r == rows - 1) rhs = sub_pinned(rhs, whi);
+      if (c * DFT_WG < total) v[r * ld + nl] = r < rows && n0 + nl < nx ? rhs : 0.0;
+    }
+    if (n0 + CH < nx) prefetch(n0 + CH);
+    __syncthreads();
+    if (work) {
+      const int steps = (min(CH, nx - n0) + 3) >> 2;
+      load(0, w[0], a[0]);
+      int s = 0;
+      for (; s + 8 < steps; s += 8) {
+        load(s + 4, w[1], a[1]);
+        mul(w[0], a[0]);
+        load(s + 8, w[0], a[0]);
+        mul(w[1], a[1]);
+        interleave_mfma<16, 3, 1>();
+      }
+      if (s + 4 < steps) {
+        load(s + 4, w[1], a[1]);
+        mul(w[0], a[0]);
+        mul(w[1], a[1]);
+      } else {
+        mul(w[0], a[0]);
+      }
+    }
+  }
+  // result i of a lane: row lane / 16 + 4 i, column lane % 16
+  if (work && k < nk) {
+    double2* __restrict__ spec = b.spec + cd->spec_off;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * rt + q + 4 * i;
+      if (r < rows) spec[spec_idx(cd->ny, y0 + r, k)] = make_double2(ar[i], ai[i]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(DFT_WG) __attribute__((amdgpu_waves_per_eu(2))) void k_dft_inv(
+    StepBuffers b, const int4* __restrict__ tiles, const ChanDesc* __restrict__ chans) {
+  extern __shared__ double2 lds[];
+  const int4 t = tiles[blockIdx.x];
+  const ChanDesc* __restrict__ cd = chans + t.x;
+  const int nx = cd->nx, nk = cd->nk, ny = cd->ny, y0 = t.y, rows = t.z, wr = t.w;
+  const int cols = 64 / wr, c0 = (int)blockIdx.y * cols;  // nodes c0 .. c0 + cols - 1
+  if (!cd->active || c0 >= nx) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave & (4 / wr - 1), rt = wave / (4 / wr);
+  const int n = c0 + 16 * wm + (lane & 15), q = lane >> 4;
+  const bool work = c0 + 16 * wm < nx && 16 * rt < rows;
+  double2* tw = lds;
+  double2* z = lds + dft_tw_len(nx);
+  __shared__ double2 zeros[DFT_MODES];
+  __shared__ double ends[64];
+  const double2* __restrict__ twg = b.tw + cd->tw_off;
+  const double2* __restrict__ spec = b.spec + cd->spec_off;
+  double* __restrict__ ps = b.psi + cd->fld_off;
+  // rows and modes per chunk, odd row stride
+  const int lgr = 3 + wr, R = 1 << lgr, KB = DFT_MODES / wr, ld = KB + 1;
+  constexpr int SLOTS = 16 * DFT_MODES / DFT_WG;
+  // chunk: modes k0 .. k0 + KB - 1 of every row, in the order of the spectrum
+  // layout (rows past the tile's last repeat it and are not stored)
+  double2 pf[SLOTS];
+  auto prefetch = [&](int k0) {
+#pragma unroll
+    for (int c = 0; c < SLOTS; ++c) {
+      const int e = tid + c * DFT_WG, kb = e >> (3 + lgr), r = (e >> 3) & (R - 1), k = k0 + 8 * kb + (e & 7);
+      pf[c] = spec[spec_idx(ny, y0 + min(r, rows - 1), min(k, nk - 1))];
+    }
+  };
+  prefetch(0);
+  dft_load_table(tw, twg, nx);
+  if (tid < DFT_MODES) zeros[tid] = make_double2(0.0, 0.0);
+  // modes 1 .. kmax are counted twice; the constant and (nx even) the Nyquist
+  // mode once: their real parts go to ends[], 0 to their places in the chunk
+  const int kmax = (nx - 1) / 2;
+  const bool nyq = (nx & 1) == 0;
+  // operands of lane (row or node = lane % 16, q): q = 0 the imaginary parts,
+  // q = 1 the real parts, 2 and 3 zeros.  Four modes at a time: the next
+  // group's operands are on their way from LDS and the previous group's terms
+  // are added while the current group's are formed.
+  const double* zp = reinterpret_cast<const double*>(q < 2 ? z + (16 * rt + (lane & 15)) * ld : zeros) + (q == 0 ? 1 : 0);
+  const char* twb = reinterpret_cast<const char*>(tw) + (q == 0 ? 8 : 0);
+  const int nn = work && n < nx ? n : 0;
+  const unsigned wrap = 16u * nx, step = 16u * (unsigned)((4LL * nn) % nx);
+  unsigned idx[4];  // 16 (k nn mod nx) of the next group's modes
+#pragma unroll
+  for (int u = 0; u < 4; ++u) idx[u] = 16u * (unsigned)((long long)u * nn % nx);
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+  double a[2][4], w[2][4];
+  d4 term[2][4];
+  auto load = [&](int kk, double(&ag)[4], double(&wg)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ag[u] = zp[2 * (kk + u)];
+      wg[u] = *reinterpret_cast<const double*>(twb + idx[u]);
+      idx[u] = wrap_add(idx[u], step, wrap);
+    }
+  };
+  auto form = [&](const double(&ag)[4], const double(&wg)[4], d4(&tg)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      tg[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ag[u], wg[u], (d4){0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+  };
+  auto add = [&](const d4(&tg)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = __builtin_fma(2.0, tg[u][i], acc[i]);
+  };
+  for (int k0 = 0; k0 < nk; k0 += KB) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < SLOTS; ++c) {
+      const int e = tid + c * DFT_WG, kb = e >> (3 + lgr), r = (e >> 3) & (R - 1), k = k0 + 8 * kb + (e & 7);
+      const bool once = k == 0 || k > kmax;
+      if (k == 0) ends[r] = pf[c].x;
+      if (k == nk - 1) ends[32 + r] = pf[c].x;
+      z[r * ld + 8 * kb + (e & 7)] = make_double2(once ? 0.0 : pf[c].x, once ? 0.0 : pf[c].y);
+    }
+    if (k0 + KB < nk) prefetch(k0 + KB);
+    __syncthreads();
+    if (!work) continue;
+    if (k0 == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = ends[16 * rt + q + 4 * i];
+    }
+    const int m = min(KB, kmax + 1 - k0);  // modes of this chunk, in groups of 4
+    if (m <= 0) continue;
+    load(0, a[0], w[0]);
+    if (m > 4) load(4, a[1], w[1]);
+    form(a[0], w[0], term[0]);
+    int kk = 0;
+    for (; kk + 12 < m; kk += 8) {
+      load(kk + 8, a[0], w[0]);
+      form(a[1], w[1], term[1]);
+      add(term[0]);
+      load(kk + 12, a[1], w[1]);
+      form(a[0], w[0], term[0]);
+      add(term[1]);
+    }
+    // one to three groups are left: term[0] formed, a[1] loaded if there is a second
+    if (kk + 4 < m) {
+      if (kk + 8 < m) load(kk + 8, a[0], w[0]);
+      form(a[1], w[1], term[1]);
+      add(term[0]);
+      if (kk + 8 < m) form(a[0], w[0], term[0]);
+      add(term[1]);
+      if (kk + 8 < m) add(term[0]);
+    } else {
+      add(term[0]);
+    }
+  }
+  if (work && n < nx) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * rt + q + 4 * i;
+      double v = acc[i];
+      if (nyq) {
+        const double zn = ends[32 + r];
+        v += (n & 1) ? -zn : zn;
+      }
+      if (r < rows) ps[(long long)(y0 + r) * nx + n] = v / (double)nx;
+    }
+  }
+  // Dirichlet rows (odd_extract, poisson.cu:297-303), this work-group's nodes
+  const double* __restrict__ Wl = b.walls + cd->wall_off;
+  const long long ws = b.walls_stride;
+  if (tid < cols && c0 + tid < nx) {
+    if (y0 == 1) ps[c0 + tid] = Wl[W_PSI_LO * ws + c0 + tid];
+    if (y0 + rows - 1 == ny - 2) ps[(long long)(ny - 1) * nx + c0 + tid] = Wl[W_PSI_HI * ws + c0 + tid];
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Row-pair x-FFTs.  A work-group takes the rows A = y0 and B = y0 + 1 of a
 // tile (a channel's last tile may hold A only) and transforms them one after
 // the other.  Every load of both rows is issued before the first is used,
@@ -2579,7 +2896,7 @@ hipError_t launch_lbm(int precision, bool compute64, bool from_q, bool macro, co
 }
 
 // The FFT tile table holds the power-of-two tiles first (n_fft_pow2 of them),
-// then the direct-DFT tiles.
+// then the matrix-core direct DFT's (n_fft_dft), then the narrow rows'.
 hipError_t launch_poisson_fwd(const StepBuffers& b, hipStream_t s) {
   if (b.n_fft_pow2 > 0 && b.fft_pair_s > 0) {
     const dim3 grid(b.n_fft_pow2), block(FFT_WG_ROWS);
@@ -2597,9 +2914,12 @@ hipError_t launch_poisson_fwd(const StepBuffers& b, hipStream_t s) {
     else
       hipLaunchKernelGGL((k_fft_fwd<true, false>), dim3(b.n_fft_pow2), dim3(FFT_WG_ROWS), b.fft_lds_pow2, s, b, b.fft_tiles, b.chans, 0);
   }
-  if (b.n_fft_tiles > b.n_fft_pow2)
-    hipLaunchKernelGGL((k_fft_fwd<false, false>), dim3(b.n_fft_tiles - b.n_fft_pow2), dim3(FFT_WG_ROWS),
-                       b.fft_lds_dft, s, b, b.fft_tiles, b.chans, b.n_fft_pow2);
+  if (b.n_fft_dft > 0)
+    hipLaunchKernelGGL(k_dft_fwd, dim3(b.n_fft_dft, b.dft_groups_fwd), dim3(DFT_WG), b.dft_lds, s, b,
+                       b.fft_tiles + b.n_fft_pow2, b.chans);
+  if (b.n_fft_tiles > b.n_fft_pow2 + b.n_fft_dft)
+    hipLaunchKernelGGL((k_fft_fwd<false, false>), dim3(b.n_fft_tiles - b.n_fft_pow2 - b.n_fft_dft), dim3(FFT_WG_ROWS),
+                       b.fft_lds_dft, s, b, b.fft_tiles, b.chans, b.n_fft_pow2 + b.n_fft_dft);
   return hipGetLastError();
 }
 
@@ -2635,9 +2955,12 @@ hipError_t launch_poisson_inv(const StepBuffers& b, hipStream_t s) {
     else
       hipLaunchKernelGGL((k_fft_inv<true, false>), dim3(b.n_fft_pow2), dim3(FFT_WG_ROWS), b.fft_lds_pow2, s, b, b.fft_tiles, b.chans, 0);
   }
-  if (b.n_fft_tiles > b.n_fft_pow2)
-    hipLaunchKernelGGL((k_fft_inv<false, false>), dim3(b.n_fft_tiles - b.n_fft_pow2), dim3(FFT_WG_ROWS),
-                       b.fft_lds_dft, s, b, b.fft_tiles, b.chans, b.n_fft_pow2);
+  if (b.n_fft_dft > 0)
+    hipLaunchKernelGGL(k_dft_inv, dim3(b.n_fft_dft, b.dft_groups_inv), dim3(DFT_WG), b.dft_lds, s, b,
+                       b.fft_tiles + b.n_fft_pow2, b.chans);
+  if (b.n_fft_tiles > b.n_fft_pow2 + b.n_fft_dft)
+    hipLaunchKernelGGL((k_fft_inv<false, false>), dim3(b.n_fft_tiles - b.n_fft_pow2 - b.n_fft_dft), dim3(FFT_WG_ROWS),
+                       b.fft_lds_dft, s, b, b.fft_tiles, b.chans, b.n_fft_pow2 + b.n_fft_dft);
   return hipGetLastError();
 }
 
