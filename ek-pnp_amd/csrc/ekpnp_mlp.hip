@@ -6,15 +6,19 @@
 // last layer is linear.  Backward (loss = mean (y - t)^2):
 //   g_{L+1} = 2 (y - t) / (B n_out)
 //   dW_l = g_l^T a_{l-1},  db_l = sum_b g_l,  g_{l-1} = (g_l W_l) * GELU'(z_{l-1})
-// with g_l rounded to BF16 before it enters a product.  One GEMM kernel does
-// all three product shapes: C[M][N] = sum_k A(m,k) B(n,k) with arbitrary
-// strides, 64x64 tiles, four waves of 2x2 v_mfma_f32_16x16x32_bf16.
+// with g_l rounded to BF16 before it enters a product.  Every product is
+// C[M][N] = sum_k A[m][k] B[n][k] with k contiguous in both operands
+// (k_gemm, k_wgrad): the epilogues that write a_l and g_l also write their
+// transposes, and the BF16 weight shadow is kept in both orders, so a lane
+// loads its MFMA fragment (8 consecutive k of one row) straight from memory.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <algorithm>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/ekpnp_mlp.h"
@@ -24,10 +28,13 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int TM = 64, TN = 64, TK = 32, KPAD = 8;  // LDS rows padded to 80 bytes
-constexpr int GEMM_THREADS = 256;
+constexpr int TILE = 16;     // MFMA tile edge
+constexpr int KSTEP = 32;    // k of one v_mfma_f32_16x16x32_bf16
+constexpr int MLP_WG = 256;  // lanes of a work-group, four waves
+constexpr int KGROUP = 8;    // k steps whose loads are in flight together
 
 // round-to-nearest-even FP32 -> BF16 bits
 __host__ __device__ inline uint16_t f2bf(float f) {
@@ -44,164 +51,234 @@ __device__ inline float dgelu(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-enum Epi { EPI_HIDDEN = 0, EPI_OUT = 1, EPI_DGELU = 2, EPI_WGRAD = 3 };
+// Accumulates C(m0.., n0..) = sum_k A[m][k] B[n][k] of one 16 x 16 tile, k in
+// steps of 32 from 0 up (K a multiple of 32, rows 16-byte aligned).
+// Lane layout of v_mfma_f32_16x16x32_bf16: A / B row = lane % 16, k = 8 (lane /
+// 16) + 0..7; C column = lane % 16, rows 4 (lane / 16) + 0..3.
+__device__ __forceinline__ floatx4 tile_product(const uint16_t* __restrict__ A, long long lda,
+                                                const uint16_t* __restrict__ B, long long ldb, int m0, int n0, int K) {
+  const int lane = threadIdx.x & 63;
+  const u16x8* pa = reinterpret_cast<const u16x8*>(A + (m0 + (lane & 15)) * lda) + (lane >> 4);
+  const u16x8* pb = reinterpret_cast<const u16x8*>(B + (n0 + (lane & 15)) * ldb) + (lane >> 4);
+  constexpr int STEP = KSTEP / 8;  // 16-byte values per k step and row
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  u16x8 va[KGROUP], vb[KGROUP];
+  const int steps = K / KSTEP;
+  for (int s0 = 0; s0 < steps; s0 += KGROUP) {
+#pragma unroll
+    for (int u = 0; u < KGROUP; ++u)
+      if (s0 + u < steps) {
+        va[u] = pa[(s0 + u) * STEP];
+        vb[u] = pb[(s0 + u) * STEP];
+      }
+#pragma unroll
+    for (int u = 0; u < KGROUP; ++u)
+      if (s0 + u < steps)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va[u]),
+                                                      __builtin_bit_cast(bf16x8, vb[u]), acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+enum Epi { EPI_HIDDEN = 0, EPI_OUT = 1, EPI_LOSS = 2, EPI_DGELU = 3 };
 
 struct GemmArgs {
-  const uint16_t* A;
-  long long sam, sak;
-  const uint16_t* B;
-  long long sbn, sbk;
-  int M, N, K;
-  const float* bias;   // [N]            (EPI_HIDDEN, EPI_OUT)
-  float* Cf;           // FP32 out [M][ldc]
-  uint16_t* Cb;        // BF16 out [M][ldc] (EPI_HIDDEN, EPI_DGELU)
-  const float* zaux;   // pre-activation [M][ldc] (EPI_DGELU)
-  long long ldc;
+  const uint16_t* A;   // [rows][K], rows a multiple of 32
+  const uint16_t* B;   // [N][K]
+  int M, N, K;         // M: rows that count; the transposes hold 0 from row M up to the next multiple of 32
+  const float* bias;   // [N]                       (HIDDEN, OUT, LOSS)
+  float* z;            // pre-activation [M][N]: written (HIDDEN, OUT), read (DGELU)
+  const float* t;      // targets [M][N]            (LOSS)
+  float* g;            // FP32 gradient [M][N]      (LOSS, DGELU)
+  uint16_t* c;         // BF16 a_l or g_l [rows][N] (HIDDEN, LOSS, DGELU)
+  uint16_t* ct;        // its transpose [N][ldt]    (HIDDEN while training, LOSS, DGELU; may be null)
+  long long ldt;
+  float* partial;      // squared-error sum of each work-group (LOSS)
+  float scale;         // 1 / (M N)                 (LOSS)
 };
 
-// Loads a 64 x 32 tile of X(r, k) = X[r*sr + k*sk] into LDS as [r][k].
-__device__ inline void load_tile(uint16_t (*T)[TK + KPAD], const uint16_t* X, long long sr,
-                                 long long sk, int r0, int k0, int R, int K) {
-  const int t = threadIdx.x;
-  if (sk == 1) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {  // consecutive lanes walk k
-      const int idx = t * 8 + e, r = idx >> 5, kk = idx & 31;
-      const int gr = r0 + r, gk = k0 + kk;
-      T[r][kk] = (gr < R && gk < K) ? X[(long long)gr * sr + gk] : (uint16_t)0;
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {  // consecutive lanes walk r
-      const int idx = t + e * GEMM_THREADS, kk = idx >> 6, r = idx & 63;
-      const int gr = r0 + r, gk = k0 + kk;
-      T[r][kk] = (gr < R && gk < K) ? X[(long long)gr * sr + (long long)gk * sk] : (uint16_t)0;
-    }
-  }
-}
-
+// One 16 x 16 tile per wave.  A layer of the warm-start network (256 x 256 at a
+// batch of 256) is 256 waves, one per CU, each with all its loads in flight:
+// latency bounds it.  64 x 64 tiles staged through LDS two bytes at a time put
+// the same layer on 16 CUs (hidden layer 20.7 us, backward 49 us a launch; 4.0 and
+// 4.5 - 12 us now).
 template <int EPI>
-__global__ __launch_bounds__(GEMM_THREADS) void k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[TM][TK + KPAD];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[TN][TK + KPAD];
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  floatx4 acc[2][2];
+__global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
+  __shared__ float red[MLP_WG / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m0 = blockIdx.y * TILE, n0 = (blockIdx.x * (MLP_WG / 64) + wave) * TILE;
+  float e2 = 0.f;
+  if (n0 < g.N) {
+    const floatx4 acc = tile_product(g.A, g.K, g.B, g.K, m0, n0, g.K);
+    const int n = n0 + (lane & 15), mr = m0 + (lane >> 4) * 4;
+    uint16_t h[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  for (int k0 = 0; k0 < g.K; k0 += TK) {
-    load_tile(As, g.A, g.sam, g.sak, m0, k0, g.M, g.K);
-    load_tile(Bs, g.B, g.sbn, g.sbk, n0, k0, g.N, g.K);
-    __syncthreads();
-    // lane layout of v_mfma_f32_16x16x32_bf16: A row / B column = lane % 16,
-    // k = 8 (lane / 16) + 0..7
-    const int kq = (lane >> 4) * 8;
-    bf16x8 af[2], bfr[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const u16x8 va = *reinterpret_cast<const u16x8*>(&As[wm * 32 + i * 16 + (lane & 15)][kq]);
-      af[i] = __builtin_bit_cast(bf16x8, va);
-      const u16x8 vb = *reinterpret_cast<const u16x8*>(&Bs[wn * 32 + i * 16 + (lane & 15)][kq]);
-      bfr[i] = __builtin_bit_cast(bf16x8, vb);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
-  }
-  // C layout: column = lane % 16, rows 4 (lane / 16) + 0..3
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn * 32 + j * 16 + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm * 32 + i * 16 + (lane >> 4) * 4 + r;
-        if (m >= g.M || n >= g.N) continue;
-        const long long o = (long long)m * g.ldc + n;
-        float v = acc[i][j][r];
-        if (EPI == EPI_HIDDEN) {
-          v += g.bias[n];
-          g.Cf[o] = v;
-          g.Cb[o] = f2bf(gelu(v));
-        } else if (EPI == EPI_OUT) {
-          g.Cf[o] = v + g.bias[n];
-        } else if (EPI == EPI_DGELU) {
-          v *= dgelu(g.zaux[o]);
-          g.Cf[o] = v;
-          g.Cb[o] = f2bf(v);
-        } else {
-          g.Cf[o] = v;
-        }
+    for (int r = 0; r < 4; ++r) {
+      const int m = mr + r;
+      if (m >= g.M) continue;
+      const long long o = (long long)m * g.N + n;
+      float v = acc[r];
+      if (EPI == EPI_HIDDEN) {
+        v += g.bias[n];
+        g.z[o] = v;
+        h[r] = f2bf(gelu(v));
+        g.c[o] = h[r];
+      } else if (EPI == EPI_OUT) {
+        g.z[o] = v + g.bias[n];
+      } else if (EPI == EPI_LOSS) {
+        // loss gradient 2 (y - t) / (M N)
+        const float d = v + g.bias[n] - g.t[o];
+        const float gv = 2.0f * d * g.scale;
+        g.g[o] = gv;
+        h[r] = f2bf(gv);
+        g.c[o] = h[r];
+        e2 += d * d;
+      } else {
+        v *= dgelu(g.z[o]);
+        g.g[o] = v;
+        h[r] = f2bf(v);
+        g.c[o] = h[r];
       }
     }
+    // four consecutive rows of one column: one 8-byte value of the transpose
+    if (EPI != EPI_OUT && g.ct)
+      *reinterpret_cast<u16x4*>(g.ct + (long long)n * g.ldt + mr) = u16x4{h[0], h[1], h[2], h[3]};
   }
-}
-
-// x (FP32 [B][n_in]) -> BF16 [B][in_pad], zero padding
-__global__ void k_pack_input(const float* __restrict__ x, uint16_t* __restrict__ xb, int B, int n_in,
-                             int in_pad) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= B * in_pad) return;
-  const int b = i / in_pad, c = i - b * in_pad;
-  xb[i] = (c < n_in) ? f2bf(x[(long long)b * n_in + c]) : (uint16_t)0;
-}
-
-// loss gradient g = 2 (y - t)/(B n), FP32 and BF16; per-block squared-error sums
-__global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y, const float* __restrict__ t,
-                                              float* __restrict__ g32, uint16_t* __restrict__ gb,
-                                              float* __restrict__ partial, int count, float scale) {
-  __shared__ float red[4];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  float e2 = 0.f;
-  if (i < count) {
-    const float d = y[i] - t[i];
-    const float gv = 2.0f * d * scale;
-    g32[i] = gv;
-    gb[i] = f2bf(gv);
-    e2 = d * d;
-  }
+  if (EPI == EPI_LOSS) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) e2 += __shfl_down(e2, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e2;
-  __syncthreads();
-  if (threadIdx.x == 0) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    for (int off = 32; off > 0; off >>= 1) e2 += __shfl_down(e2, off, 64);
+    if (lane == 0) red[wave] = e2;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      g.partial[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+  }
 }
 
-// db[n] = sum_b g[b][n], fixed summation order
-__global__ __launch_bounds__(256) void k_bias_grad(const float* __restrict__ g, float* __restrict__ db,
-                                                   int B, int N) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
+// One layer of the network as the weight kernels see it
+struct Layer {
+  const uint16_t* at;   // a_{l-1} transposed [in][ldt]
+  const uint16_t* gt;   // g_l transposed [out][ldt]
+  const float* g;       // g_l, FP32 [B][out]
+  int in, out;
+  long long off_w, off_b;  // in the parameter vector
+  uint16_t* wt;         // W_l transposed [in][out], BF16 (null for the first layer)
+  int wg_first;         // first k_wgrad work-group: weight tiles, then 16-column bias blocks
+  int wg_bias;          // first of the bias blocks
+  int up_first;         // first k_update work-group: 32 x 32 weight tiles, then the bias
+};
+
+// layer of work-group wg (first(l) ascending)
+template <typename F>
+__device__ __forceinline__ int find_layer(int n, int wg, F first) {
+  int l = 0;
+  while (l + 1 < n && wg >= first(l + 1)) ++l;
+  return l;
+}
+
+// Weight and bias gradients of every layer in one launch:
+//   dW_l[o][i] = sum_b g_l[b][o] a_{l-1}[b][i], one 16 x 16 tile per wave (K = the
+//   batch rounded up to 32, zeros past it);
+//   db_l[n] = sum_b g_l[b][n] in FP32, one row after the other: 16 columns per
+//   work-group, 256 rows at a time through LDS (any other order would give
+//   other last bits, which Adam's normalisation and the BF16 shadows amplify
+//   over a training run).
+// Five products of 26-30 us and five one-lane-per-column sums of 46-55 us
+// before (a batch of 256): too few work-groups, and a serial chain of loads;
+// 8.2 us now.  A training step of the 6 -> 4 x 256 -> 1024 network at a batch of
+// 256, with its host copies: 840 -> 140 us, at 512 1309 -> 178 us.
+constexpr int BIAS_ROWS = 256;
+__global__ __launch_bounds__(MLP_WG) void k_wgrad(const Layer* __restrict__ layers, int n_layers, float* __restrict__ grad,
+                                                  long long ldt, int B) {
+  __shared__ float part[BIAS_ROWS][TILE + 1];
+  const int wg = blockIdx.x;
+  const Layer L = layers[find_layer(n_layers, wg, [&](int l) { return layers[l].wg_first; })];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (wg < L.wg_bias) {
+    const int tile = (wg - L.wg_first) * (MLP_WG / 64) + wave, nt = L.in / TILE;
+    const int m0 = tile / nt * TILE, n0 = (tile - tile / nt * nt) * TILE;
+    if (m0 >= L.out) return;
+    const floatx4 acc = tile_product(L.gt, ldt, L.at, ldt, m0, n0, (B + KSTEP - 1) / KSTEP * KSTEP);
+    float* o = grad + L.off_w + (long long)(m0 + (lane >> 4) * 4) * L.in + n0 + (lane & 15);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[(long long)r * L.in] = acc[r];
+    return;
+  }
+  const int n0 = (wg - L.wg_bias) * TILE, col = threadIdx.x & (TILE - 1), row = threadIdx.x / TILE;
   float s = 0.f;
-  for (int b = 0; b < B; ++b) s += g[(long long)b * N + n];
-  db[n] = s;
+  for (int b0 = 0; b0 < B; b0 += BIAS_ROWS) {
+    float v[TILE];
+#pragma unroll
+    for (int c = 0; c < TILE; ++c) v[c] = L.g[(long long)min(b0 + row + c * (MLP_WG / TILE), B - 1) * L.out + n0 + col];
+    __syncthreads();  // the previous rows have been added
+#pragma unroll
+    for (int c = 0; c < TILE; ++c) part[row + c * (MLP_WG / TILE)][col] = v[c];
+    __syncthreads();
+    if (row == 0)
+#pragma unroll 16
+      for (int k = 0; k < min(BIAS_ROWS, B - b0); ++k) s += part[k][col];
+  }
+  if (row == 0) grad[L.off_b + n0 + col] = s;
 }
 
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ pb, long long n, float lr, float b1,
-                       float b2, float eps, float wd, float c1, float c2) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i] + wd * p[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-  p[i] = pi;
-  pb[i] = f2bf(pi);
+struct AdamArgs {
+  float lr, b1, b2, eps, wd, c1, c2;
+};
+
+// Adam on the FP32 master parameters (UPDATE) and the BF16 shadows, as stored
+// and transposed; one 32 x 32 weight tile per work-group, then 1024 biases
+template <bool UPDATE>
+__global__ __launch_bounds__(MLP_WG) void k_update(const Layer* __restrict__ layers, int n_layers, float* __restrict__ p,
+                                                   const float* __restrict__ g, float* __restrict__ m,
+                                                   float* __restrict__ v, uint16_t* __restrict__ pb, AdamArgs a) {
+  __shared__ uint16_t tile[32][33];
+  const int wg = blockIdx.x;
+  const Layer L = layers[find_layer(n_layers, wg, [&](int l) { return layers[l].up_first; })];
+  auto update = [&](long long i) {
+    float pi = p[i];
+    if (UPDATE) {
+      // (the contractions are spelled out, so that they do not depend on what
+      // surrounds this)
+      const float gi = __builtin_fmaf(a.wd, pi, g[i]);
+      const float mi = __builtin_fmaf(a.b1, m[i], (1.f - a.b1) * gi);
+      const float vi = __builtin_fmaf(a.b2, v[i], (1.f - a.b2) * gi * gi);
+      m[i] = mi;
+      v[i] = vi;
+      pi = pi - a.lr * (mi * a.c1) / (sqrtf(vi * a.c2) + a.eps);
+      p[i] = pi;
+    }
+    const uint16_t h = f2bf(pi);
+    pb[i] = h;
+    return h;
+  };
+  const int nt = L.in / 32, t = wg - L.up_first, rt = t / nt;
+  if (rt >= L.out / 32) {
+    const int i0 = (t - nt * (L.out / 32)) * 1024;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int i = i0 + c * MLP_WG + (int)threadIdx.x;
+      if (i < L.out) update(L.off_b + i);
+    }
+    return;
+  }
+  const int r0 = rt * 32, c0 = (t - rt * nt) * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) tile[y + 8 * c][x] = update(L.off_w + (long long)(r0 + y + 8 * c) * L.in + c0 + x);
+  if (!L.wt) return;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 4; ++c) L.wt[(long long)(c0 + y + 8 * c) * L.out + r0 + x] = tile[x][y + 8 * c];
 }
 
-__global__ void k_to_bf16(const float* __restrict__ p, uint16_t* __restrict__ pb, long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) pb[i] = f2bf(p[i]);
+// x (FP32 [B][n_in]) -> BF16 [rows][in_pad] and its transpose, zeros past n_in
+// and past B
+__global__ void k_pack_input(const float* __restrict__ x, uint16_t* __restrict__ xb, uint16_t* __restrict__ xt,
+                             long long ldt, int rows, int B, int n_in, int in_pad) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= rows * in_pad) return;
+  const int b = i / in_pad, c = i - b * in_pad;
+  const uint16_t h = (c < n_in && b < B) ? f2bf(x[(long long)b * n_in + c]) : (uint16_t)0;
+  xb[i] = h;
+  xt[(long long)c * ldt + b] = h;
 }
 
 }  // namespace
@@ -209,20 +286,25 @@ __global__ void k_to_bf16(const float* __restrict__ p, uint16_t* __restrict__ pb
 struct ekpnp_mlp {
   ekpnp_mlp_config cfg{};
   int in_pad = 32, L = 0;
+  long long rows = 0;                      // max_batch rounded up to 32: rows of a and g, columns of their transposes
   std::vector<int> in_dim, out_dim;        // per layer 1..L+1 (index 0 unused)
   std::vector<long long> off_w, off_b;
   long long n_params = 0;
   float *p32 = nullptr, *m32 = nullptr, *v32 = nullptr, *g32 = nullptr;
   uint16_t* pbf = nullptr;
-  uint16_t* xb = nullptr;
   std::vector<float*> z;       // [L+2], z[l] FP32 [B][out_l]
-  std::vector<uint16_t*> a;    // [L+1], a[0] = xb, a[l] BF16 [B][out_l]
+  std::vector<uint16_t*> a;    // [L+1], a[0] the packed input, a[l] BF16 [rows][out_l]
+  std::vector<uint16_t*> at;   // [L+1], their transposes [out_l][rows]
+  std::vector<float*> g;       // [L+2], g[l] FP32 [B][out_l]
+  std::vector<uint16_t*> gb;   // [L+2], g[l] BF16 [rows][out_l]
+  std::vector<uint16_t*> gt;   // [L+2], its transpose [out_l][rows]
+  std::vector<uint16_t*> wt;   // [L+2], W_l transposed [in_l][out_l], l >= 2
   float* t = nullptr;          // targets
   float* xin = nullptr;        // FP32 input staging
-  float *gf = nullptr, *gf2 = nullptr;       // FP32 gradient rows
-  uint16_t *gb = nullptr, *gb2 = nullptr;    // BF16 gradient rows
-  float* partial = nullptr;
-  int max_partials = 0;
+  float* partial = nullptr;    // squared-error sums, written by the device into host memory
+  Layer* layers = nullptr;     // layer table of the weight kernels, layers 1..L+1
+  int n_wgrad = 0, n_update = 0;  // their work-groups
+  std::vector<void*> bufs;     // every device allocation
   hipStream_t stream = nullptr;
   float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f, wd = 0.f;
   long long adam_t = 0;
@@ -243,116 +325,100 @@ int mfail(ekpnp_mlp* m, int code, const std::string& msg) {
   } while (0)
 
 void release(ekpnp_mlp* m) {
-  void* ptrs[] = {m->p32, m->m32, m->v32, m->g32, m->pbf, m->xb, m->t, m->xin, m->gf, m->gf2, m->gb, m->gb2,
-                  m->partial};
-  for (void* p : ptrs)
+  for (void* p : m->bufs)
     if (p) (void)hipFree(p);
-  for (float* p : m->z)
-    if (p) (void)hipFree(p);
-  for (size_t i = 1; i < m->a.size(); ++i)
-    if (m->a[i]) (void)hipFree(m->a[i]);
+  if (m->partial) (void)hipHostFree(m->partial);
   if (m->stream) (void)hipStreamDestroy(m->stream);
 }
 
-hipError_t gemm(ekpnp_mlp* m, int epi, const GemmArgs& g) {
-  const dim3 grid((g.N + TN - 1) / TN, (g.M + TM - 1) / TM), block(GEMM_THREADS);
-  switch (epi) {
-    case EPI_HIDDEN: hipLaunchKernelGGL(k_gemm<EPI_HIDDEN>, grid, block, 0, m->stream, g); break;
-    case EPI_OUT: hipLaunchKernelGGL(k_gemm<EPI_OUT>, grid, block, 0, m->stream, g); break;
-    case EPI_DGELU: hipLaunchKernelGGL(k_gemm<EPI_DGELU>, grid, block, 0, m->stream, g); break;
-    default: hipLaunchKernelGGL(k_gemm<EPI_WGRAD>, grid, block, 0, m->stream, g); break;
-  }
-  return hipGetLastError();
-}
+int rows_of(int B) { return (B + KSTEP - 1) / KSTEP * KSTEP; }
+dim3 gemm_grid(int N, int rows) { return dim3((N / TILE + MLP_WG / 64 - 1) / (MLP_WG / 64), rows / TILE); }
 
-hipError_t forward(ekpnp_mlp* m, const float* x_host, int B) {
+// layers 1 .. last of the forward pass (hidden layers, or with L + 1 the
+// linear output too); train: the transposed activations are written as well
+hipError_t forward(ekpnp_mlp* m, const float* x_host, int B, int last, bool train) {
   hipError_t e = hipMemcpyAsync(m->xin, x_host, (size_t)B * m->cfg.n_in * sizeof(float),
                                 hipMemcpyHostToDevice, m->stream);
   if (e != hipSuccess) return e;
-  const int n = B * m->in_pad;
-  hipLaunchKernelGGL(k_pack_input, dim3((n + 255) / 256), dim3(256), 0, m->stream, m->xin, m->xb, B,
-                     m->cfg.n_in, m->in_pad);
-  for (int l = 1; l <= m->L + 1; ++l) {
+  const int rows = rows_of(B), n = rows * m->in_pad;
+  hipLaunchKernelGGL(k_pack_input, dim3((n + 255) / 256), dim3(256), 0, m->stream, m->xin, m->a[0], m->at[0], m->rows,
+                     rows, B, m->cfg.n_in, m->in_pad);
+  for (int l = 1; l <= last; ++l) {
     GemmArgs g{};
     g.A = m->a[l - 1];
-    g.sam = m->in_dim[l];
-    g.sak = 1;
     g.B = m->pbf + m->off_w[l];
-    g.sbn = m->in_dim[l];
-    g.sbk = 1;
     g.M = B;
     g.N = m->out_dim[l];
     g.K = m->in_dim[l];
     g.bias = m->p32 + m->off_b[l];
-    g.Cf = m->z[l];
-    g.Cb = (l <= m->L) ? m->a[l] : nullptr;
-    g.ldc = m->out_dim[l];
-    e = gemm(m, l <= m->L ? EPI_HIDDEN : EPI_OUT, g);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
-// backward after forward: fills g32 with the gradient of the loss; loss sum
-// into *loss (host)
-int backward(ekpnp_mlp* m, const float* t_host, int B, float* loss) {
-  const int L = m->L, no = m->cfg.n_out;
-  MHIP(m, hipMemcpyAsync(m->t, t_host, (size_t)B * no * sizeof(float), hipMemcpyHostToDevice, m->stream));
-  const int count = B * no, nblk = (count + 255) / 256;
-  hipLaunchKernelGGL(k_loss, dim3(nblk), dim3(256), 0, m->stream, m->z[L + 1], m->t, m->gf, m->gb, m->partial,
-                     count, 1.0f / (float)count);
-  MHIP(m, hipGetLastError());
-  float* gcur = m->gf;
-  uint16_t* gbcur = m->gb;
-  float* gnext = m->gf2;
-  uint16_t* gbnext = m->gb2;
-  for (int l = L + 1; l >= 1; --l) {
-    const int in = m->in_dim[l], out = m->out_dim[l];
-    // dW_l[o][i] = sum_b g[b][o] a_{l-1}[b][i]
-    GemmArgs gw{};
-    gw.A = gbcur;
-    gw.sam = 1;
-    gw.sak = out;
-    gw.B = m->a[l - 1];
-    gw.sbn = 1;
-    gw.sbk = in;
-    gw.M = out;
-    gw.N = in;
-    gw.K = B;
-    gw.Cf = m->g32 + m->off_w[l];
-    gw.ldc = in;
-    MHIP(m, gemm(m, EPI_WGRAD, gw));
-    hipLaunchKernelGGL(k_bias_grad, dim3((out + 255) / 256), dim3(256), 0, m->stream, gcur,
-                       m->g32 + m->off_b[l], B, out);
-    MHIP(m, hipGetLastError());
-    if (l > 1) {
-      // g_{l-1}[b][i] = sum_o g[b][o] W_l[o][i] * GELU'(z_{l-1}[b][i])
-      GemmArgs gd{};
-      gd.A = gbcur;
-      gd.sam = out;
-      gd.sak = 1;
-      gd.B = m->pbf + m->off_w[l];
-      gd.sbn = 1;
-      gd.sbk = in;
-      gd.M = B;
-      gd.N = in;
-      gd.K = out;
-      gd.Cf = gnext;
-      gd.Cb = gbnext;
-      gd.zaux = m->z[l - 1];
-      gd.ldc = in;
-      MHIP(m, gemm(m, EPI_DGELU, gd));
-      std::swap(gcur, gnext);
-      std::swap(gbcur, gbnext);
+    g.z = m->z[l];
+    const dim3 grid = gemm_grid(g.N, rows);
+    if (l <= m->L) {
+      g.c = m->a[l];
+      g.ct = train ? m->at[l] : nullptr;
+      g.ldt = m->rows;
+      hipLaunchKernelGGL(k_gemm<EPI_HIDDEN>, grid, dim3(MLP_WG), 0, m->stream, g);
+    } else {
+      hipLaunchKernelGGL(k_gemm<EPI_OUT>, grid, dim3(MLP_WG), 0, m->stream, g);
     }
   }
-  std::vector<float> part(nblk);
-  MHIP(m, hipMemcpyAsync(part.data(), m->partial, nblk * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-  MHIP(m, hipStreamSynchronize(m->stream));
-  double s = 0.0;
-  for (float v : part) s += v;
-  if (loss) *loss = (float)(s / (double)count);
+  return hipGetLastError();
+}
+
+// forward and backward pass: fills g32 with the gradient of the loss and
+// leaves the work-groups' squared-error sums in partial (host memory, valid
+// once the stream is synchronised; see loss_of)
+int loss_grad(ekpnp_mlp* m, const float* x_host, const float* t_host, int B) {
+  const int L = m->L, no = m->cfg.n_out, rows = rows_of(B);
+  MHIP(m, forward(m, x_host, B, L, true));
+  MHIP(m, hipMemcpyAsync(m->t, t_host, (size_t)B * no * sizeof(float), hipMemcpyHostToDevice, m->stream));
+  for (int l = L + 1; l >= 1; --l) {
+    GemmArgs g{};
+    if (l == L + 1) {
+      // output layer and the loss gradient g_{L+1}
+      g.A = m->a[L];
+      g.B = m->pbf + m->off_w[l];
+      g.K = m->in_dim[l];
+      g.bias = m->p32 + m->off_b[l];
+      g.t = m->t;
+      g.partial = m->partial;
+      g.scale = 1.0f / (float)(B * no);
+    } else {
+      // g_l[b][i] = sum_o g_{l+1}[b][o] W_{l+1}[o][i] * GELU'(z_l[b][i])
+      g.A = m->gb[l + 1];
+      g.B = m->wt[l + 1];
+      g.K = m->out_dim[l + 1];
+      g.z = m->z[l];
+    }
+    g.M = B;
+    g.N = m->out_dim[l];
+    g.g = m->g[l];
+    g.c = m->gb[l];
+    g.ct = m->gt[l];
+    g.ldt = m->rows;
+    const dim3 grid = gemm_grid(g.N, rows);
+    if (l == L + 1) hipLaunchKernelGGL(k_gemm<EPI_LOSS>, grid, dim3(MLP_WG), 0, m->stream, g);
+    else hipLaunchKernelGGL(k_gemm<EPI_DGELU>, grid, dim3(MLP_WG), 0, m->stream, g);
+  }
+  hipLaunchKernelGGL(k_wgrad, dim3(m->n_wgrad), dim3(MLP_WG), 0, m->stream, m->layers, L + 1, m->g32, m->rows, B);
+  MHIP(m, hipGetLastError());
   return 0;
+}
+
+float loss_of(const ekpnp_mlp* m, int B) {
+  const int no = m->cfg.n_out;
+  const dim3 grid = gemm_grid(no, rows_of(B));
+  double s = 0.0;
+  for (unsigned i = 0; i < grid.x * grid.y; ++i) s += m->partial[i];
+  return (float)(s / (double)(B * no));
+}
+
+// BF16 shadows of the master parameters, and the Adam step before them
+template <bool UPDATE>
+hipError_t update(ekpnp_mlp* m, const AdamArgs& a) {
+  hipLaunchKernelGGL(k_update<UPDATE>, dim3(m->n_update), dim3(MLP_WG), 0, m->stream, m->layers, m->L + 1, m->p32,
+                     m->g32, m->m32, m->v32, m->pbf, a);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -398,38 +464,68 @@ int ekpnp_mlp_create(const ekpnp_mlp_config* cfg, ekpnp_mlp** out) {
         p[m->off_w[l] + (long long)o * m->in_dim[l] + i] = (float)(sd * nrm);
       }
   }
-  const int maxw = std::max(H, cfg->n_out);
-  m->max_partials = (B * cfg->n_out + 255) / 256;
-  auto A = [&](void** ptr, size_t bytes) { return hipMalloc(ptr, std::max<size_t>(bytes, 16)); };
+  const long long R = m->rows = rows_of(B);
   hipError_t e = hipSuccess;
-  if (e == hipSuccess) e = A((void**)&m->p32, off * 4);
-  if (e == hipSuccess) e = A((void**)&m->m32, off * 4);
-  if (e == hipSuccess) e = A((void**)&m->v32, off * 4);
-  if (e == hipSuccess) e = A((void**)&m->g32, off * 4);
-  if (e == hipSuccess) e = A((void**)&m->pbf, off * 2);
-  if (e == hipSuccess) e = A((void**)&m->xb, (size_t)B * m->in_pad * 2);
-  if (e == hipSuccess) e = A((void**)&m->xin, (size_t)B * cfg->n_in * 4);
-  if (e == hipSuccess) e = A((void**)&m->t, (size_t)B * cfg->n_out * 4);
-  if (e == hipSuccess) e = A((void**)&m->gf, (size_t)B * maxw * 4);
-  if (e == hipSuccess) e = A((void**)&m->gf2, (size_t)B * maxw * 4);
-  if (e == hipSuccess) e = A((void**)&m->gb, (size_t)B * maxw * 2);
-  if (e == hipSuccess) e = A((void**)&m->gb2, (size_t)B * maxw * 2);
-  if (e == hipSuccess) e = A((void**)&m->partial, (size_t)m->max_partials * 4);
+  auto A = [&](auto** ptr, size_t count) {
+    if (e != hipSuccess) return;
+    void* p = nullptr;
+    e = hipMalloc(&p, std::max<size_t>(count * sizeof(**ptr), 16));
+    if (e != hipSuccess) return;
+    *ptr = static_cast<std::remove_reference_t<decltype(*ptr)>>(p);
+    m->bufs.push_back(p);
+  };
+  A(&m->p32, off);
+  A(&m->m32, off);
+  A(&m->v32, off);
+  A(&m->g32, off);
+  A(&m->pbf, off);
+  A(&m->xin, (size_t)B * cfg->n_in);
+  A(&m->t, (size_t)B * cfg->n_out);
+  A(&m->layers, L + 1);
   m->z.assign(L + 2, nullptr);
+  m->g.assign(L + 2, nullptr);
+  m->gb.assign(L + 2, nullptr);
+  m->gt.assign(L + 2, nullptr);
+  m->wt.assign(L + 2, nullptr);
   m->a.assign(L + 1, nullptr);
-  m->a[0] = m->xb;
-  for (int l = 1; l <= L + 1 && e == hipSuccess; ++l) {
-    e = A((void**)&m->z[l], (size_t)B * m->out_dim[l] * 4);
-    if (e == hipSuccess && l <= L) e = A((void**)&m->a[l], (size_t)B * m->out_dim[l] * 2);
+  m->at.assign(L + 1, nullptr);
+  A(&m->a[0], R * m->in_pad);
+  A(&m->at[0], R * m->in_pad);
+  for (int l = 1; l <= L + 1; ++l) {
+    const size_t n = (size_t)m->out_dim[l];
+    A(&m->z[l], (size_t)B * n);
+    A(&m->g[l], (size_t)B * n);
+    A(&m->gb[l], R * n);
+    A(&m->gt[l], R * n);
+    if (l <= L) A(&m->a[l], R * n);
+    if (l <= L) A(&m->at[l], R * n);
+    if (l >= 2) A(&m->wt[l], n * m->in_dim[l]);
+  }
+  const dim3 lg = gemm_grid(cfg->n_out, (int)R);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&m->partial, (size_t)lg.x * lg.y * sizeof(float), hipHostMallocDefault);
+  std::vector<Layer> tab(L + 1);
+  for (int l = 1; l <= L + 1; ++l) {
+    Layer& d = tab[l - 1];
+    d.at = m->at[l - 1];
+    d.gt = m->gt[l];
+    d.g = m->g[l];
+    d.in = m->in_dim[l];
+    d.out = m->out_dim[l];
+    d.off_w = m->off_w[l];
+    d.off_b = m->off_b[l];
+    d.wt = m->wt[l];
+    d.wg_first = m->n_wgrad;
+    d.wg_bias = d.wg_first + (d.in / TILE * (d.out / TILE) + MLP_WG / 64 - 1) / (MLP_WG / 64);
+    m->n_wgrad = d.wg_bias + d.out / TILE;
+    d.up_first = m->n_update;
+    m->n_update += d.in / 32 * (d.out / 32) + (d.out + 1023) / 1024;
   }
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipMemcpy(m->layers, tab.data(), tab.size() * sizeof(Layer), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(m->p32, p.data(), off * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(m->m32, 0, off * 4);
   if (e == hipSuccess) e = hipMemset(m->v32, 0, off * 4);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((off + 255) / 256)), dim3(256), 0, m->stream, m->p32, m->pbf, off);
-    e = hipGetLastError();
-  }
+  if (e == hipSuccess) e = update<false>(m, AdamArgs{});
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (e != hipSuccess) {
     release(m);
@@ -468,9 +564,7 @@ int ekpnp_mlp_set_params(ekpnp_mlp* m, const float* in) {
   MHIP(m, hipMemset(m->m32, 0, m->n_params * 4));
   MHIP(m, hipMemset(m->v32, 0, m->n_params * 4));
   m->adam_t = 0;
-  hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((m->n_params + 255) / 256)), dim3(256), 0, m->stream, m->p32,
-                     m->pbf, m->n_params);
-  MHIP(m, hipGetLastError());
+  MHIP(m, update<false>(m, AdamArgs{}));
   MHIP(m, hipStreamSynchronize(m->stream));
   return 0;
 }
@@ -479,7 +573,7 @@ int ekpnp_mlp_forward(ekpnp_mlp* m, const float* x, int batch, float* y) {
   if (!m || !x || !y) return -1;
   if (batch < 1 || batch > m->cfg.max_batch) return mfail(m, -1, "batch out of range");
   MHIP(m, hipSetDevice(m->cfg.device));
-  MHIP(m, forward(m, x, batch));
+  MHIP(m, forward(m, x, batch, m->L + 1, false));
   MHIP(m, hipMemcpyAsync(y, m->z[m->L + 1], (size_t)batch * m->cfg.n_out * 4, hipMemcpyDeviceToHost, m->stream));
   MHIP(m, hipStreamSynchronize(m->stream));
   return 0;
@@ -489,9 +583,10 @@ int ekpnp_mlp_loss_grad(ekpnp_mlp* m, const float* x, const float* t, int batch,
   if (!m || !x || !t) return -1;
   if (batch < 1 || batch > m->cfg.max_batch) return mfail(m, -1, "batch out of range");
   MHIP(m, hipSetDevice(m->cfg.device));
-  MHIP(m, forward(m, x, batch));
-  int rc = backward(m, t, batch, loss);
+  int rc = loss_grad(m, x, t, batch);
   if (rc) return rc;
+  MHIP(m, hipStreamSynchronize(m->stream));
+  if (loss) *loss = loss_of(m, batch);
   if (grad) MHIP(m, hipMemcpy(grad, m->g32, m->n_params * 4, hipMemcpyDeviceToHost));
   return 0;
 }
@@ -509,15 +604,14 @@ int ekpnp_mlp_train_step(ekpnp_mlp* m, const float* x, const float* t, int batch
   if (!m || !x || !t) return -1;
   if (batch < 1 || batch > m->cfg.max_batch) return mfail(m, -1, "batch out of range");
   MHIP(m, hipSetDevice(m->cfg.device));
-  MHIP(m, forward(m, x, batch));
-  int rc = backward(m, t, batch, loss);
+  int rc = loss_grad(m, x, t, batch);
   if (rc) return rc;
   m->adam_t++;
   const float c1 = 1.0f / (1.0f - std::pow(m->b1, (float)m->adam_t));
   const float c2 = 1.0f / (1.0f - std::pow(m->b2, (float)m->adam_t));
-  hipLaunchKernelGGL(k_adam, dim3((unsigned)((m->n_params + 255) / 256)), dim3(256), 0, m->stream, m->p32, m->g32,
-                     m->m32, m->v32, m->pbf, m->n_params, lr, m->b1, m->b2, m->eps, m->wd, c1, c2);
-  MHIP(m, hipGetLastError());
+  MHIP(m, update<true>(m, AdamArgs{lr, m->b1, m->b2, m->eps, m->wd, c1, c2}));
+  MHIP(m, hipStreamSynchronize(m->stream));
+  if (loss) *loss = loss_of(m, batch);
   return 0;
 }
 
