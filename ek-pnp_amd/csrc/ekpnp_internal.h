@@ -183,6 +183,8 @@ hipError_t launch_row_means(const StepBuffers& b, double* out, float* blocks_out
 // / new_blocks (state in cur, or in other for channels whose swap flag is set)
 hipError_t launch_rebase(int precision, const StepBuffers& b, void* cur, void* other, const double* new_refs,
                          const float* new_blocks, hipStream_t s);
+// rho_e = c+ - c- of channel chan (n nodes) from its macroscopic planes
+hipError_t launch_charge(const StepBuffers& b, int chan, long long n, hipStream_t s);
 hipError_t launch_pb_relax(const StepBuffers& b, double* psi_old, hipStream_t s);
 // one red-black SOR half-sweep of channel chan's 5-point Poisson system
 // (color 0: x + y even); partials[wg] = largest |change| per work-group,

@@ -2726,6 +2726,13 @@ __global__ __launch_bounds__(LBM_WG) void k_pb_fields(StepBuffers b) {
   b.rho_e[o] = cp - cn;
 }
 
+// charge density of fields set from the host: one pass over two planes in
+// place of a host loop, a host buffer and a third copy over the bus
+__global__ __launch_bounds__(256) void k_charge(StepBuffers b, int chan, long long n) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x, o = b.chans[chan].fld_off + i;
+  if (i < n) b.rho_e[o] = b.macro[M_CP * b.macro_stride + o] - b.macro[M_CN * b.macro_stride + o];
+}
+
 __global__ __launch_bounds__(LBM_WG) void k_pb_relax(StepBuffers b, double* __restrict__ psi_old) {
   const int2 tile = b.lbm_tiles[blockIdx.x];
   const ChanDesc* __restrict__ cd = b.chans + tile.x;
@@ -3028,6 +3035,11 @@ hipError_t launch_rebase(int precision, const StepBuffers& b, void* cur, void* o
 
 hipError_t launch_pb_fields(const StepBuffers& b, hipStream_t s) {
   hipLaunchKernelGGL(k_pb_fields, dim3(b.n_lbm_tiles), dim3(LBM_WG), 0, s, b);
+  return hipGetLastError();
+}
+
+hipError_t launch_charge(const StepBuffers& b, int chan, long long n, hipStream_t s) {
+  hipLaunchKernelGGL(k_charge, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, chan, n);
   return hipGetLastError();
 }
 
