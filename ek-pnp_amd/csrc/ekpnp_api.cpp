@@ -256,6 +256,49 @@ ChanDesc make_desc(const ekpnp_channel_params& p, int precision) {
   return d;
 }
 
+// How many of the 27 population planes go through the caches (an index into
+// LBM_CACHED).  A streamed plane is read from and written to HBM every step; a
+// cached one is found in the 256 MB Infinity Cache if both its lattices still
+// lie there a step later, and one that does not evicts psi and the spectrum for
+// nothing.  So as many planes as fit LBM_CACHE_BYTES: the largest count of
+// LBM_CACHED whose planes, both lattices of them (bytes: all 27), stay within
+// it.  k_lbm (the widths the row kernel does not take, FP64 storage) gains from
+// whole lattices a little longer, up to LBM_CACHE_BYTES_WHOLE, and with FP32
+// storage only from whole ones; the row kernel and FP64 storage stream what is
+// below LBM_CACHE_BYTES_MIN, which the L2 caches serve better so.  Step in us,
+// nothing cached -> the rule's count [another count]:
+//   32 channels fp32   33 MB  34.9 (0)                 [37.7 with 27]
+//   512x256     fp64   57 MB  30.6 (0)                 [31.8 with 27]
+//   64x128 x32  fp32   57 MB  33.9 (0)                 [34.7 with 27]
+//   128x128 x24 fp32   85 MB  43.0 -> 41.2 (27)
+//   512x500     fp64  111 MB  45.0 -> 39.9 (27)
+//   1024x514    fp32  114 MB  54.1 -> 49.7 (27)
+//   1024x1026   fp32  227 MB  82.2 -> 75.7 (18)        [80.6 with 27]
+//   1024x514    fp64  227 MB  76.9 -> 60.3 (27)        [66.4 with 18]
+//   odd 100 x64 fp64  290 MB  96.5 -> 86.6 (13)        [93.8 with 27]
+//   1024x800    fp64  354 MB  101.6 -> 89.6 (9)        [88.1 with 13]
+//   2048x1024   fp32  453 MB  139.6 -> 131.8 (9)       [136.8 with 13]
+//   4096x700    fp32  619 MB  181.5 -> 169.0 (6)       [170.9 with 9]
+//   2048x1024   fp64  906 MB  211.6 -> 198.3 (4)       [218.1 with 9]
+//   4096x1024   fp32  906 MB  230.3 -> 220.1 (4)       [235.1 with 6]
+//   4096x1400   fp32 1239 MB  335.6 -> 326.8 (2)       [342.4 with 4]
+//   4096x1024   fp64 1812 MB  394.4 -> 376.8 (2)       [385.5 with 4]
+//   8192x2048   fp32 3624 MB  955.1 (0)                [956.9 with 2]
+// and k_lbm with FP32 storage:
+//   n_x = 8 x200       62 MB  41.9 -> 35.3 (27)        [41.9 with 9]
+//   n_x = 8 x600      180 MB  91.2 -> 77.0 (27)        [90.1 with 13]
+//   1000x1001         216 MB  213.9 -> 209.3 (27)      [211.4 with 13]
+//   n_x = 8 x1000     294 MB  129.6 (0)                [138.6 with 27]
+constexpr double LBM_CACHE_BYTES = 160e6, LBM_CACHE_BYTES_WHOLE = 230e6, LBM_CACHE_BYTES_MIN = 80e6;
+
+int lbm_cached_planes(double bytes, bool fp64, bool rows) {
+  if (!rows && bytes <= LBM_CACHE_BYTES_WHOLE && (!fp64 || bytes >= LBM_CACHE_BYTES_MIN)) return LBM_CACHED_ALL;
+  if ((!rows && !fp64) || bytes < LBM_CACHE_BYTES_MIN) return 0;
+  int i = 0;
+  while (i < LBM_CACHED_ALL && LBM_CACHED[i + 1] / 27.0 * bytes <= LBM_CACHE_BYTES) ++i;
+  return i;
+}
+
 StepBuffers make_buffers(ekpnp_ctx* c) {
   StepBuffers b{};
   b.chans = c->d_desc;
@@ -290,6 +333,10 @@ StepBuffers make_buffers(ekpnp_ctx* c) {
   b.lbm_gen_tiles = c->d_lbm_split + c->n_lbm_row + c->n_lbm_wall;
   b.n_lbm_gen_tiles = (int)c->lbm_split.size() - c->n_lbm_row - c->n_lbm_wall;
   b.lbm_wrows = c->lbm_wrows;
+  const bool fp64 = c->opt.precision == EKPNP_POP_FP64;
+  const double pop_bytes = 2.0 * (double)c->total_pops * (fp64 ? 8 : 4);
+  b.lbm_cached = lbm_cached_planes(pop_bytes, fp64, false);
+  b.lbm_rows_cached = lbm_cached_planes(pop_bytes, fp64, true);
   return b;
 }
 

@@ -16,6 +16,10 @@ enum WallPlane { W_PSI_LO = 0, W_PSI_HI = 1, W_CP_LO = 2, W_CP_HI = 3, W_CN_LO =
 // Macroscopic output planes (FP64), each of total_nodes elements.
 enum MacroPlane { M_RHO = 0, M_UX = 1, M_UY = 2, M_CP = 3, M_CN = 4, M_COUNT = 5 };
 
+// population planes (in storage order, of 27) that the LBM kernels read and
+// write through the caches; the others are streamed past them
+constexpr int LBM_CACHED[] = {0, 2, 4, 6, 9, 13, 18, 27};
+constexpr int LBM_CACHED_ALL = 7;  // index of 27
 constexpr int LBM_WG = 256;       // nodes per LBM work-group (one node per lane)
 constexpr int FFT_WG = 256;       // lanes of a persistent x-FFT work-group
 constexpr int FFT_WG_ROWS = 512;  // lanes of a one-tile x-FFT work-group (radix-8 passes)
@@ -107,6 +111,7 @@ struct StepBuffers {
   int n_lbm_wall_tiles;
   const int2* lbm_gen_tiles;
   int n_lbm_gen_tiles;
+  int lbm_cached, lbm_rows_cached;  // cached planes of k_lbm and k_lbm_rows (indices into LBM_CACHED)
   int lbm_wrows;                // row-kernel interior tiles: 0 consecutive blocks, else rows per tile (2, 4)
   const int4* fft_tiles;        // (channel, first row, rows, matrix-core DFT: row tiles) per FFT work-group
   int n_fft_tiles;

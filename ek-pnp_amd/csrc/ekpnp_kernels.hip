@@ -42,24 +42,9 @@ namespace ekpnp {
 
 constexpr double W0 = 4.0 / 9.0, WS = 1.0 / 9.0, WD = 1.0 / 36.0;  // LBM.h:105-107
 
-// Build-time tuning of k_lbm (defaults chosen by measurement on MI355X, where
-// non-temporal loads and stores of the populations raised the kernel from
-// 5.0 to 5.7 TB/s at 4096 x 1024):
-//   EKPNP_NT_STORE  1: post-collision populations are written with
-//                      non-temporal stores (streamed past the caches)
-//   EKPNP_NT_LOAD   1: the gather reads are non-temporal as well
-//   EKPNP_LBM_WAVES N: ask for at least N waves per SIMD (register budget)
-#ifndef EKPNP_NT_STORE
-#define EKPNP_NT_STORE 1
-#endif
-#ifndef EKPNP_NT_LOAD
-#define EKPNP_NT_LOAD 1
-#endif
-// k_lbm asks for 3 waves per SIMD: its FP32-storage, FP64-arithmetic
-// variants otherwise take 169-171 VGPRs (2 waves); at 168 the compiler spills
-// 1-4 VGPRs and the kernel is 5-14 % faster (4096x1024: 214 -> 203 us;
-// 5000 channels of nx = 4: 214 -> 184 us); variants already within 168 are
-// unchanged
+// Build-time tuning of k_lbm:
+//   EKPNP_LBM_WAVES N: ask for at least N waves per SIMD (register budget);
+//                      3 holds every variant to 168 VGPRs, which none spills
 #ifndef EKPNP_LBM_WAVES
 #define EKPNP_LBM_WAVES 3
 #endif
@@ -69,23 +54,36 @@ constexpr double W0 = 4.0 / 9.0, WS = 1.0 / 9.0, WD = 1.0 / 36.0;  // LBM.h:105-
 #define LBM_WAVES_ATTR
 #endif
 
-template <typename S>
+// Population accesses: streamed past the caches (NT), which an HBM-bound sweep
+// over lattices larger than the caches wants (4096x1024: 5.0 -> 5.7 TB/s), or
+// ordinary for the first CACHED of the 27 planes, which then stay in the
+// Infinity Cache from one step to the next (lbm_cached_planes: how many, and
+// what each count measured).  A template parameter: with a run-time choice the
+// compiler merges both accesses into one ordinary one.
+template <bool NT, typename S>
 __device__ __forceinline__ S ld_pop(const S* p) {
-#if EKPNP_NT_LOAD
-  return __builtin_nontemporal_load(p);
-#else
-  return *p;
-#endif
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
 }
 
-template <typename S>
+template <bool NT, typename S>
 __device__ __forceinline__ void st_pop(S* p, S v) {
-#if EKPNP_NT_STORE
-  __builtin_nontemporal_store(v, p);
-#else
-  *p = v;
-#endif
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
 }
+
+// The (wave-uniform) plane stride as a value of its own.  Addresses formed from
+// it are computed where they are used: with the loads' stride the compiler keeps
+// all 27 plane offsets in registers from the gather to the stores (k_lbm with
+// FP32 storage: 168 VGPRs and 8 bytes of scratch per lane; this way 142, none).
+__device__ __forceinline__ long long own_stride(long long plane) {
+  unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)plane);
+  unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(plane >> 32));
+  long long p = (long long)(((unsigned long long)hi << 32) | lo);
+  asm("" : "+s"(p));
+  return p;
+}
+
 constexpr unsigned FLAG_G0_FLUID_U = 0x2u;
 
 // Work-groups are handed to the 8 XCDs round-robin; remap so that each XCD
@@ -199,12 +197,36 @@ __device__ __forceinline__ void add_src_refs(C* q, const double* dX, C j0, C jm,
   q[8] += C(WD) * (C(dX[8]) + jp);
 }
 
+// the gather of one species: stored values from the upstream neighbours of
+// node x (rows at offsets rm, r0, rp) plus the reference terms of their sources
+template <typename S, typename C, bool REF, int s, int CACHED>
+__device__ __forceinline__ void load_species(const S* P, long long plane, long long rm, long long r0,
+                                             long long rp, int x, int xm, int xp, const NodeRefs& rf, double tc,
+                                             C* q) {
+  constexpr int p = 9 * s;
+  const S* B = P + (long long)p * plane;
+  q[p + 0] = (C)ld_pop<(p + 0 >= CACHED)>(B + 0 * plane + r0 + x);
+  q[p + 1] = (C)ld_pop<(p + 1 >= CACHED)>(B + 1 * plane + r0 + xm);
+  q[p + 2] = (C)ld_pop<(p + 2 >= CACHED)>(B + 2 * plane + rm + x);
+  q[p + 3] = (C)ld_pop<(p + 3 >= CACHED)>(B + 3 * plane + r0 + xp);
+  q[p + 4] = (C)ld_pop<(p + 4 >= CACHED)>(B + 4 * plane + rp + x);
+  q[p + 5] = (C)ld_pop<(p + 5 >= CACHED)>(B + 5 * plane + rm + xm);
+  q[p + 6] = (C)ld_pop<(p + 6 >= CACHED)>(B + 6 * plane + rm + xp);
+  q[p + 7] = (C)ld_pop<(p + 7 >= CACHED)>(B + 7 * plane + rp + xp);
+  q[p + 8] = (C)ld_pop<(p + 8 >= CACHED)>(B + 8 * plane + rp + xm);
+  if (REF) {
+    double dX[9];
+    rf.diffs(s, dX);
+    add_src_refs(q + p, dX, C(rf.jo.J[s] * tc), C(rf.jm.J[s] * tc), C(rf.jp.J[s] * tc));
+  }
+}
+
 // rest deviation of node (x, y) from stored values at the node itself
 // (FROM_Q) or gathered from the upstream neighbours (pull streaming):
 //   q_i = stored_i(src) + w_i (X(src) - X(node)) + w_i c_ix tc J(src).
 // 27 values: f 0..8, h 9..17, g 18..26.  REF false (FP64 storage): no
 // reference terms.
-template <typename S, typename C, bool FROM_Q, bool REF>
+template <typename S, typename C, bool FROM_Q, bool REF, int CACHED = 0>
 __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plane, int nx, int ny,
                                          int x, int y, int xm, int xp, const NodeRefs& rf, double tc, C* q) {
   const long long r0 = (long long)y * nx;
@@ -214,7 +236,7 @@ __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plan
       const C j = REF ? C(rf.jo.J[s] * tc) : C(0);
 #pragma unroll
       for (int d = 0; d < 9; ++d) {
-        q[9 * s + d] = (C)ld_pop(P + (9 * s + d) * plane + r0 + x);
+        q[9 * s + d] = (C)ld_pop<true>(P + (9 * s + d) * plane + r0 + x);
         if (REF && CX[d] != 0) q[9 * s + d] += C(CX[d] * (d < 5 ? WS : WD)) * j;
       }
     }
@@ -223,30 +245,30 @@ __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plan
   const int ym = (y == 0) ? ny - 1 : y - 1;
   const int yp = (y == ny - 1) ? 0 : y + 1;
   const long long rm = (long long)ym * nx, rp = (long long)yp * nx;
-#pragma unroll
-  for (int s = 0; s < 3; ++s) {
-    const S* B = P + (long long)(9 * s) * plane;
-    q[9 * s + 0] = (C)ld_pop(B + 0 * plane + r0 + x);
-    q[9 * s + 1] = (C)ld_pop(B + 1 * plane + r0 + xm);
-    q[9 * s + 2] = (C)ld_pop(B + 2 * plane + rm + x);
-    q[9 * s + 3] = (C)ld_pop(B + 3 * plane + r0 + xp);
-    q[9 * s + 4] = (C)ld_pop(B + 4 * plane + rp + x);
-    q[9 * s + 5] = (C)ld_pop(B + 5 * plane + rm + xm);
-    q[9 * s + 6] = (C)ld_pop(B + 6 * plane + rm + xp);
-    q[9 * s + 7] = (C)ld_pop(B + 7 * plane + rp + xp);
-    q[9 * s + 8] = (C)ld_pop(B + 8 * plane + rp + xm);
-    if (REF) {
-      double dX[9];
-      rf.diffs(s, dX);
-      add_src_refs(q + 9 * s, dX, C(rf.jo.J[s] * tc), C(rf.jm.J[s] * tc), C(rf.jp.J[s] * tc));
-    }
-  }
+  load_species<S, C, REF, 0, CACHED>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
+  load_species<S, C, REF, 1, CACHED>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
+  load_species<S, C, REF, 2, CACHED>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
 }
 
 // stored value of rest deviation v in direction d of a row with flux term j = tc J
 template <typename C>
 __device__ __forceinline__ C to_stored(C v, int d, C j) {
   return CX[d] == 0 ? v : v - C(CX[d] * (d < 5 ? WS : WD)) * j;
+}
+
+// the 9 populations of species s of a node, its flux term j
+template <int s, int CACHED, typename S, typename C>
+__device__ __forceinline__ void store_species(S* Q, long long plane, long long node, const C* q, C j) {
+  constexpr int p = 9 * s;
+  st_pop<(p + 0 >= CACHED)>(Q + (p + 0) * plane + node, (S)to_stored(q[0], 0, j));
+  st_pop<(p + 1 >= CACHED)>(Q + (p + 1) * plane + node, (S)to_stored(q[1], 1, j));
+  st_pop<(p + 2 >= CACHED)>(Q + (p + 2) * plane + node, (S)to_stored(q[2], 2, j));
+  st_pop<(p + 3 >= CACHED)>(Q + (p + 3) * plane + node, (S)to_stored(q[3], 3, j));
+  st_pop<(p + 4 >= CACHED)>(Q + (p + 4) * plane + node, (S)to_stored(q[4], 4, j));
+  st_pop<(p + 5 >= CACHED)>(Q + (p + 5) * plane + node, (S)to_stored(q[5], 5, j));
+  st_pop<(p + 6 >= CACHED)>(Q + (p + 6) * plane + node, (S)to_stored(q[6], 6, j));
+  st_pop<(p + 7 >= CACHED)>(Q + (p + 7) * plane + node, (S)to_stored(q[7], 7, j));
+  st_pop<(p + 8 >= CACHED)>(Q + (p + 8) * plane + node, (S)to_stored(q[8], 8, j));
 }
 
 // Ion wall node: the next pre-collision state is the anti-bounce-back of the
@@ -366,7 +388,7 @@ __device__ __forceinline__ Moments<C> moments(const C* q, const ChanDesc* __rest
 // k_lbm: one coupled-step LBM update of every node of every channel.
 // ---------------------------------------------------------------------------
 // S: storage type of the populations; C: arithmetic type of the collision.
-template <typename S, typename C, bool FROM_Q, bool MACRO>
+template <typename S, typename C, bool FROM_Q, bool MACRO, int CACHED>
 __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, const int2* __restrict__ tiles,
                                                 const S* __restrict__ src, S* __restrict__ dst) {
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
@@ -409,7 +431,8 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
 #pragma unroll
       for (int s = 0; s < 3; ++s) X1[s] = r1.own(s);
     }
-    load_pre<S, C, FROM_Q, REF>(P, plane, nx, ny, x, 1, xm, xp, r1, tc, m1);
+    const long long p1 = own_stride(plane);
+    load_pre<S, C, FROM_Q, REF, CACHED>(P, p1, nx, ny, x, 1, xm, xp, r1, tc, m1);
     double Ex1, Ey1;
     efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1);
     const Moments<C> mm = moments(m1, cd, X1, Ex1, Ey1);
@@ -418,7 +441,7 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
   }
 
   C q[27];
-  load_pre<S, C, FROM_Q, REF>(P, plane, nx, ny, x, y, xm, xp, rf, tc, q);
+  load_pre<S, C, FROM_Q, REF, CACHED>(P, plane, nx, ny, x, y, xm, xp, rf, tc, q);
   if (!FROM_Q && (bottom || top)) {
     const double* __restrict__ Wl = b.walls + cd->wall_off + x;
     const long long ws = b.walls_stride;
@@ -489,11 +512,19 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
     collide_fluid(q, m.dr, m.rho, ux, uy, m.Fx, m.Fy, C(cd->om_pf), C(cd->om_mf), ics, icfl,
                   C(cd->src_p * cd->dt), C(cd->src_m * cd->dt));
   }
+  if constexpr (FROM_Q) {  // the flux term subtracted here is the one that load_pre added: as a loop,
+                           // the compiler contracts both alike
 #pragma unroll
-  for (int s = 0; s < 3; ++s) {
-    const C j = REF ? C(rf.jo.J[s] * tc) : C(0);
+    for (int s = 0; s < 3; ++s) {
+      const C j = REF ? C(rf.jo.J[s] * tc) : C(0);
 #pragma unroll
-    for (int d = 0; d < 9; ++d) st_pop(Q + (9 * s + d) * plane + node, (S)to_stored(q[9 * s + d], d, j));
+      for (int d = 0; d < 9; ++d) st_pop<true>(Q + (9 * s + d) * plane + node, (S)to_stored(q[9 * s + d], d, j));
+    }
+  } else {
+    const long long sp = own_stride(plane);
+    store_species<0, CACHED>(Q, sp, node, q, REF ? C(rf.jo.J[0] * tc) : C(0));
+    store_species<1, CACHED>(Q, sp, node, q + 9, REF ? C(rf.jo.J[1] * tc) : C(0));
+    store_species<2, CACHED>(Q, sp, node, q + 18, REF ? C(rf.jo.J[2] * tc) : C(0));
   }
 }
 
@@ -597,17 +628,18 @@ __device__ __forceinline__ void species_q(const float* v, const WaveRefs& rf, in
 // 9 FP32 values of species block B gathered for node x of row y (pull,
 // periodic in x and y; rm, r0, rp are the row offsets of y-1, y, y+1, which
 // fit 32 bits: a channel holds at most MAX_NX x (MAX_INTERIOR_ROWS + 2) nodes)
+template <int s, int CACHED>
 __device__ __forceinline__ void gather9(const float* __restrict__ B, long long plane, int rm, int r0, int rp, int x,
                                         int xm, int xp, float* v) {
-  v[0] = ld_pop(B + 0 * plane + (r0 + x));
-  v[1] = ld_pop(B + 1 * plane + (r0 + xm));
-  v[2] = ld_pop(B + 2 * plane + (rm + x));
-  v[3] = ld_pop(B + 3 * plane + (r0 + xp));
-  v[4] = ld_pop(B + 4 * plane + (rp + x));
-  v[5] = ld_pop(B + 5 * plane + (rm + xm));
-  v[6] = ld_pop(B + 6 * plane + (rm + xp));
-  v[7] = ld_pop(B + 7 * plane + (rp + xp));
-  v[8] = ld_pop(B + 8 * plane + (rp + xm));
+  v[0] = ld_pop<(9 * s + 0 >= CACHED)>(B + 0 * plane + (r0 + x));
+  v[1] = ld_pop<(9 * s + 1 >= CACHED)>(B + 1 * plane + (r0 + xm));
+  v[2] = ld_pop<(9 * s + 2 >= CACHED)>(B + 2 * plane + (rm + x));
+  v[3] = ld_pop<(9 * s + 3 >= CACHED)>(B + 3 * plane + (r0 + xp));
+  v[4] = ld_pop<(9 * s + 4 >= CACHED)>(B + 4 * plane + (rp + x));
+  v[5] = ld_pop<(9 * s + 5 >= CACHED)>(B + 5 * plane + (rm + xm));
+  v[6] = ld_pop<(9 * s + 6 >= CACHED)>(B + 6 * plane + (rm + xp));
+  v[7] = ld_pop<(9 * s + 7 >= CACHED)>(B + 7 * plane + (rp + xp));
+  v[8] = ld_pop<(9 * s + 8 >= CACHED)>(B + 8 * plane + (rp + xm));
 }
 
 // one node of a row tile (WALL: y = 0 or ny-1); a separate instantiation per
@@ -615,7 +647,8 @@ __device__ __forceinline__ void gather9(const float* __restrict__ B, long long p
 // step writes the macroscopic planes) is a run-time, wave-uniform flag: the
 // compiler allocates the interior kernel in 118 VGPRs (4 waves per SIMD) this
 // way, and in 136 (3 waves) when the flag is a template parameter and false.
-template <bool WALL>
+// Wall rows (2 of ny) are always streamed.
+template <bool WALL, int CACHED>
 __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int y, int x,
                                              const WaveRefs& rf, const float* __restrict__ P, float* __restrict__ Q,
                                              bool macro) {
@@ -629,19 +662,20 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
   const int xp = (x == nx - 1) ? 0 : x + 1;
   const bool bottom = WALL && (y == 0), top = WALL && (y == ny - 1);
   constexpr bool wall = WALL;
+  static_assert(!WALL || CACHED == 0, "the mirror's gather below takes every plane as streamed");
   // fluid: pull gather (LBM.cu:869-905, x and y wrap); ions: the same, or
   // on a wall row the node's own values (LBM.cu:915-1023)
   float v[27];
   {
     const int r0 = y * nx;
     const int rm = (bottom ? ny - 1 : y - 1) * nx, rp = (top ? 0 : y + 1) * nx;
-    gather9(P, plane, rm, r0, rp, x, xm, xp, v);
+    gather9<0, CACHED>(P, plane, rm, r0, rp, x, xm, xp, v);
     if (wall) {
 #pragma unroll
       for (int k = 9; k < 27; ++k) v[k] = P[(long long)k * plane + node];
     } else {
-#pragma unroll
-      for (int s = 1; s < 3; ++s) gather9(P + (long long)(9 * s) * plane, plane, rm, r0, rp, x, xm, xp, v + 9 * s);
+      gather9<1, CACHED>(P + 9 * plane, plane, rm, r0, rp, x, xm, xp, v + 9);
+      gather9<2, CACHED>(P + 18 * plane, plane, rm, r0, rp, x, xm, xp, v + 18);
     }
   }
   // the node's own references X(x, y)
@@ -664,7 +698,8 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
   if (bottom) {
     const int r0 = nx, rm = 0, rp = 2 * nx;
 #pragma unroll
-    for (int s = 0; s < 3; ++s) gather9(P + (long long)(9 * s) * plane, plane, rm, r0, rp, x, xm, xp, w + 9 * s);
+    for (int s = 0; s < 3; ++s)
+      gather9<0, 0>(P + (long long)(9 * s) * plane, plane, rm, r0, rp, x, xm, xp, w + 9 * s);
     efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1);
   }
   // every load is in flight before the first use: keep the scheduler from
@@ -750,8 +785,7 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
       species_q(v + 9, rf, 1, tc, wall, dcwp, q);
       collide_ion(q, m.dcp, cp, vpx, vpy, C(cd->om_pp), C(cd->om_mp), ics, ticf, om_p);
       const C j = C(rf.J(1, 1) * tc);
-#pragma unroll
-      for (int d = 0; d < 9; ++d) st_pop(Q + (9 + d) * plane + node, (float)to_stored(q[d], d, j));
+      store_species<1, CACHED>(Q, plane, node, q, j);
     }
     {
       const C cn = C(Xo[2]) + m.dcn;
@@ -761,8 +795,7 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
       collide_ion(q, m.dcn, cn, vnx, vny, C(cd->om_pn), C(cd->om_mn), ics, ticf,
                   (cd->flags & FLAG_G0_FLUID_U) ? om_f : om_n);
       const C j = C(rf.J(1, 2) * tc);
-#pragma unroll
-      for (int d = 0; d < 9; ++d) st_pop(Q + (18 + d) * plane + node, (float)to_stored(q[d], d, j));
+      store_species<2, CACHED>(Q, plane, node, q, j);
     }
   }
   {
@@ -787,8 +820,7 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
                     C(cd->src_p * cd->dt), C(cd->src_m * cd->dt));
     }
     const C j = C(rf.J(1, 0) * tc);
-#pragma unroll
-    for (int d = 0; d < 9; ++d) st_pop(Q + d * plane + node, (float)to_stored(q[d], d, j));
+    store_species<0, CACHED>(Q, plane, node, q, j);
   }
 }
 
@@ -802,7 +834,7 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
 // blocks from the tile's first node on (across row ends); wrows = 2 or 4,
 // the tile is wrows rows x (4 / wrows) blocks whose first node is the tile's
 // (waves past a row's end or past the last row return).
-template <bool WALL>
+template <bool WALL, int CACHED>
 __device__ __forceinline__ void lbm_rows_tile(const StepBuffers& b, int2 tile, const float* __restrict__ src,
                                               float* __restrict__ dst, bool macro, int wrows) {
   const ChanDesc* __restrict__ cd = b.chans + tile.x;
@@ -823,14 +855,14 @@ __device__ __forceinline__ void lbm_rows_tile(const StepBuffers& b, int2 tile, c
   const float* __restrict__ P = (cd->swap ? dst : src) + cd->pop_off;
   float* __restrict__ Q = (cd->swap ? const_cast<float*>(src) : dst) + cd->pop_off;
   const WaveRefs rf = wave_refs(b, cd, y, k, (int)threadIdx.x & 63);
-  lbm_row_node<WALL>(b, cd, y, x, rf, P, Q, macro);
+  lbm_row_node<WALL, CACHED>(b, cd, y, x, rf, P, Q, macro);
 }
 
-template <bool WALL>
+template <bool WALL, int CACHED>
 __global__ __launch_bounds__(LBM_WG) void k_lbm_rows(StepBuffers b, const int2* __restrict__ tiles,
                                                     const float* __restrict__ src, float* __restrict__ dst,
                                                     int macro) {
-  lbm_rows_tile<WALL>(b, tiles[xcd_remap(blockIdx.x, gridDim.x)], src, dst, macro != 0, WALL ? 0 : b.lbm_wrows);
+  lbm_rows_tile<WALL, CACHED>(b, tiles[xcd_remap(blockIdx.x, gridDim.x)], src, dst, macro != 0, WALL ? 0 : b.lbm_wrows);
 }
 
 
@@ -2515,7 +2547,7 @@ __global__ __launch_bounds__(TRI_WG) void k_tridiag_walls(StepBuffers b, const f
   if (i >= nw)
     tridiag_tile<LMAX>(b, b.tri_tiles[xcd_remap(i - nw, nt)], sA, sB);
   else if (i < b.n_lbm_wall_tiles)
-    lbm_rows_tile<true>(b, b.lbm_wall_tiles[i], src, dst, MACRO, 0);
+    lbm_rows_tile<true, 0>(b, b.lbm_wall_tiles[i], src, dst, MACRO, 0);
 }
 
 // table[j][k] = cprime_closed(j L, k kdy_scale) for chunks j = 1..C-1 (row
@@ -2849,6 +2881,29 @@ hipError_t launch_copy_nt(const void* src, void* dst, long long n_float4, int gr
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// f(CACHED) for an index into LBM_CACHED
+template <typename F>
+static void with_cached(int index, const F& f) {
+  switch (index) {
+    case 0: f(std::integral_constant<int, LBM_CACHED[0]>{}); break;
+    case 1: f(std::integral_constant<int, LBM_CACHED[1]>{}); break;
+    case 2: f(std::integral_constant<int, LBM_CACHED[2]>{}); break;
+    case 3: f(std::integral_constant<int, LBM_CACHED[3]>{}); break;
+    case 4: f(std::integral_constant<int, LBM_CACHED[4]>{}); break;
+    case 5: f(std::integral_constant<int, LBM_CACHED[5]>{}); break;
+    case 6: f(std::integral_constant<int, LBM_CACHED[6]>{}); break;
+    default: f(std::integral_constant<int, LBM_CACHED[7]>{}); break;
+  }
+}
+
+static void launch_rows(const StepBuffers& b, const void* src, void* dst, bool macro, hipStream_t s) {
+  if (b.n_lbm_row_tiles > 0)
+    with_cached(b.lbm_rows_cached, [&](auto cached) {
+      hipLaunchKernelGGL((k_lbm_rows<false, cached()>), dim3(b.n_lbm_row_tiles), dim3(LBM_WG), 0, s, b,
+                         b.lbm_row_tiles, static_cast<const float*>(src), static_cast<float*>(dst), macro ? 1 : 0);
+    });
+}
+
 template <typename S, typename C>
 static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBuffers& b, const void* src,
                                void* dst, hipStream_t s) {
@@ -2857,8 +2912,8 @@ static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBu
   const dim3 block(LBM_WG);
   if (from_q) {
     const dim3 grid(b.n_lbm_tiles);
-    if (macro) hipLaunchKernelGGL((k_lbm<S, C, true, true>), grid, block, 0, s, b, b.lbm_tiles, sp, dp);
-    else hipLaunchKernelGGL((k_lbm<S, C, true, false>), grid, block, 0, s, b, b.lbm_tiles, sp, dp);
+    if (macro) hipLaunchKernelGGL((k_lbm<S, C, true, true, 0>), grid, block, 0, s, b, b.lbm_tiles, sp, dp);
+    else hipLaunchKernelGGL((k_lbm<S, C, true, false, 0>), grid, block, 0, s, b, b.lbm_tiles, sp, dp);
     return hipGetLastError();
   }
   // the row kernel exists for FP32 storage with FP64 arithmetic
@@ -2867,19 +2922,20 @@ static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBu
   const int2* gen = rows ? b.lbm_gen_tiles : b.lbm_tiles;
   const int n_gen = rows ? b.n_lbm_gen_tiles : b.n_lbm_tiles;
   if (n_gen > 0) {
-    const dim3 grid(n_gen);
-    if (macro) hipLaunchKernelGGL((k_lbm<S, C, false, true>), grid, block, 0, s, b, gen, sp, dp);
-    else hipLaunchKernelGGL((k_lbm<S, C, false, false>), grid, block, 0, s, b, gen, sp, dp);
+    const auto launch = [&](auto cached) {
+      const dim3 grid(n_gen);
+      if (macro) hipLaunchKernelGGL((k_lbm<S, C, false, true, cached()>), grid, block, 0, s, b, gen, sp, dp);
+      else hipLaunchKernelGGL((k_lbm<S, C, false, false, cached()>), grid, block, 0, s, b, gen, sp, dp);
+    };
+    if constexpr (!std::is_same<S, float>::value) with_cached(b.lbm_cached, launch);
+    else if (b.lbm_cached == LBM_CACHED_ALL) launch(std::integral_constant<int, 27>{});
+    else launch(std::integral_constant<int, 0>{});
   }
   if (rows) {
-    const float* fs = reinterpret_cast<const float*>(src);
-    float* fd = reinterpret_cast<float*>(dst);
     if (walls && b.n_lbm_wall_tiles > 0)
-      hipLaunchKernelGGL((k_lbm_rows<true>), dim3(b.n_lbm_wall_tiles), block, 0, s, b, b.lbm_wall_tiles, fs, fd,
-                         macro ? 1 : 0);
-    if (b.n_lbm_row_tiles > 0)
-      hipLaunchKernelGGL((k_lbm_rows<false>), dim3(b.n_lbm_row_tiles), block, 0, s, b, b.lbm_row_tiles, fs, fd,
-                         macro ? 1 : 0);
+      hipLaunchKernelGGL((k_lbm_rows<true, 0>), dim3(b.n_lbm_wall_tiles), block, 0, s, b, b.lbm_wall_tiles,
+                         reinterpret_cast<const float*>(src), reinterpret_cast<float*>(dst), macro ? 1 : 0);
+    launch_rows(b, src, dst, macro, s);
   }
   return hipGetLastError();
 }
@@ -2887,9 +2943,7 @@ static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBu
 // the row kernel's interior launch alone (no macroscopic planes): the LBM
 // tile-shape autotuner's trial
 hipError_t launch_lbm_rows_interior(const StepBuffers& b, const void* src, void* dst, hipStream_t s) {
-  if (b.n_lbm_row_tiles > 0)
-    hipLaunchKernelGGL((k_lbm_rows<false>), dim3(b.n_lbm_row_tiles), dim3(LBM_WG), 0, s, b, b.lbm_row_tiles,
-                       static_cast<const float*>(src), static_cast<float*>(dst), 0);
+  launch_rows(b, src, dst, false, s);
   return hipGetLastError();
 }
 
