@@ -5,9 +5,11 @@
 // on the host except parameter bookkeeping, input generation (the seeded cold
 // start) and the D2H formatting of outputs.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
+#include <cerrno>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -731,6 +733,24 @@ std::vector<double> ref_offsets(ekpnp_ctx* c, int channel, int species, hipError
   return out;
 }
 
+// Have the whole pages of a destination that is about to be overwritten mapped
+// in one call: memory fresh from the allocator costs a fault per 4 KB page
+// otherwise (256 MB in 1 MB fields: 55 ms with the copy, 28 ms this way, 4 ms
+// once mapped).  Nothing is lost where the kernel does not know the request.
+void map_pages(char* p, size_t bytes) {
+#ifdef MADV_POPULATE_WRITE
+  const uintptr_t a = ((uintptr_t)p + 4095) & ~(uintptr_t)4095, e = ((uintptr_t)p + bytes) & ~(uintptr_t)4095;
+  if (e > a) {
+    const int err = errno;
+    (void)madvise(reinterpret_cast<void*>(a), e - a, MADV_POPULATE_WRITE);
+    errno = err;
+  }
+#else
+  (void)p;
+  (void)bytes;
+#endif
+}
+
 // dst = bytes of device memory at src, once the stream's earlier work is done.
 // The runtime's copy to pageable memory moves a field at 10 GB/s (13 ms for the
 // 134 MB of 8192 x 2048): it copies and first touches the caller's pages on one
@@ -767,6 +787,7 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
   }
   if (pieces == 1) {
     hipError_t e = hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream);
+    map_pages(static_cast<char*>(dst), bytes);
     const hipError_t e2 = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = e2;
     if (e == hipSuccess) std::memcpy(dst, c->stage, bytes);
@@ -784,18 +805,20 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
   std::atomic<int> left{0};
   std::atomic<bool> stop{false};
   const int threads = STAGE_THREADS;
-  auto share = [&](int t, size_t i) {
+  auto share = [&](int t, size_t i, bool map_only) {
     const size_t n = size_of(i), part = (n / threads + 4095) & ~(size_t)4095, a = std::min(n, part * t);
-    std::memcpy(out + i * chunk + a, c->stage + (i % slots) * chunk + a, std::min(part, n - a));
+    if (map_only) map_pages(out + i * chunk + a, std::min(part, n - a));
+    else std::memcpy(out + i * chunk + a, c->stage + (i % slots) * chunk + a, std::min(part, n - a));
   };
   std::vector<std::thread> helpers;
   try {
     for (int t = 1; t < STAGE_THREADS; ++t)
       helpers.emplace_back([&, t] {
-        for (size_t i = 0;; ++i) {
+        for (size_t i = 0; i < pieces; ++i) {
+          share(t, i, true);
           while (ready.load(std::memory_order_acquire) <= i)
             if (stop.load(std::memory_order_relaxed)) return;
-          share(t, i);
+          share(t, i, false);
           left.fetch_sub(1, std::memory_order_release);
         }
       });
@@ -806,12 +829,12 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
   hipError_t e = hipSuccess;
   for (size_t i = 0; i < slots && e == hipSuccess; ++i) e = issue(i);
   for (size_t i = 0; i < pieces && e == hipSuccess; ++i) {
+    share(0, i, true);
     e = hipEventSynchronize(c->stage_ev[i % slots]);
     if (e != hipSuccess) break;
     left.store(helping, std::memory_order_relaxed);
     ready.store(i + 1, std::memory_order_release);
-    share(0, i);
-    for (int t = helping + 1; t < threads; ++t) share(t, i);
+    for (int t = 0; t < threads; t = t == 0 ? helping + 1 : t + 1) share(t, i, false);
     while (left.load(std::memory_order_acquire) > 0) {
     }
     if (i + slots < pieces) e = issue(i + slots);
