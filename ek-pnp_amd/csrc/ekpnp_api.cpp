@@ -266,36 +266,39 @@ ChanDesc make_desc(const ekpnp_channel_params& p, int precision) {
 // LBM_CACHED whose planes, both lattices of them (bytes: all 27), stay within
 // it.  k_lbm (the widths the row kernel does not take, FP64 storage) gains from
 // whole lattices a little longer, up to LBM_CACHE_BYTES_WHOLE, and with FP32
-// storage only from whole ones; the row kernel and FP64 storage stream what is
-// below LBM_CACHE_BYTES_MIN, which the L2 caches serve better so.  Step in us,
-// nothing cached -> the rule's count [another count]:
+// storage and narrow channels only from whole ones; the row kernel and FP64
+// storage stream what is below LBM_CACHE_BYTES_MIN, which the L2 caches serve
+// better so.  Step in us, nothing cached -> the rule's count [another count]:
 //   32 channels fp32   33 MB  34.9 (0)                 [37.7 with 27]
 //   512x256     fp64   57 MB  30.6 (0)                 [31.8 with 27]
 //   64x128 x32  fp32   57 MB  33.9 (0)                 [34.7 with 27]
 //   128x128 x24 fp32   85 MB  43.0 -> 41.2 (27)
-//   512x500     fp64  111 MB  45.0 -> 39.9 (27)
+//   512x400     fp64   88 MB  41.1 -> 37.8 (27)
 //   1024x514    fp32  114 MB  54.1 -> 49.7 (27)
 //   1024x1026   fp32  227 MB  82.2 -> 75.7 (18)        [80.6 with 27]
-//   1024x514    fp64  227 MB  76.9 -> 60.3 (27)        [66.4 with 18]
-//   odd 100 x64 fp64  290 MB  96.5 -> 86.6 (13)        [93.8 with 27]
-//   1024x800    fp64  354 MB  101.6 -> 89.6 (9)        [88.1 with 13]
+//   1024x514    fp64  227 MB  80.1 -> 60.3 (27)        [63.8 with 18]
+//   1024x800    fp64  354 MB  100.7 -> 89.1 (9)        [86.7 with 13, 103 with 27]
 //   2048x1024   fp32  453 MB  139.6 -> 131.8 (9)       [136.8 with 13]
 //   4096x700    fp32  619 MB  181.5 -> 169.0 (6)       [170.9 with 9]
-//   2048x1024   fp64  906 MB  211.6 -> 198.3 (4)       [218.1 with 9]
+//   2048x1024   fp64  906 MB  210.3 -> 195.2 (4)       [214.7 with 9]
 //   4096x1024   fp32  906 MB  230.3 -> 220.1 (4)       [235.1 with 6]
 //   4096x1400   fp32 1239 MB  335.6 -> 326.8 (2)       [342.4 with 4]
-//   4096x1024   fp64 1812 MB  394.4 -> 376.8 (2)       [385.5 with 4]
+//   4096x1024   fp64 1812 MB  393.2 -> 369.7 (2)       [396.7 with 4]
 //   8192x2048   fp32 3624 MB  955.1 (0)                [956.9 with 2]
 // and k_lbm with FP32 storage:
-//   n_x = 8 x200       62 MB  41.9 -> 35.3 (27)        [41.9 with 9]
-//   n_x = 8 x600      180 MB  91.2 -> 77.0 (27)        [90.1 with 13]
-//   1000x1001         216 MB  213.9 -> 209.3 (27)      [211.4 with 13]
-//   n_x = 8 x1000     294 MB  129.6 (0)                [138.6 with 27]
+//   n_x = 8 x200       62 MB  42.1 -> 36.6 (27)        [40.9 with 13]
+//   n_x = 32 x300     213 MB  75.7 -> 68.0 (27)        [75.0 with 13]
+//   1000x1001         216 MB  214.1 -> 201.0 (27)      [207.1 with 13]
+//   1000x1251         270 MB  272.3 -> 264.1 (13)      [269.9 with 27]
+//   1500x1201         389 MB  528.0 -> 517.5 (9)       [523.0 with 18]
+//   n_x = 8 x1000     294 MB  120.6 (0)                [120.3 with 13, 125.8 with 27]
+//   n_x = 8 x4000    1178 MB  418.6 (0)                [433.1 with 2]
 constexpr double LBM_CACHE_BYTES = 160e6, LBM_CACHE_BYTES_WHOLE = 230e6, LBM_CACHE_BYTES_MIN = 80e6;
+constexpr int LBM_CACHE_PART_NX = 256;  // narrowest channel of FP32 storage k_lbm with a part of the planes cached
 
-int lbm_cached_planes(double bytes, bool fp64, bool rows) {
+int lbm_cached_planes(double bytes, bool fp64, bool rows, int min_nx) {
   if (!rows && bytes <= LBM_CACHE_BYTES_WHOLE && (!fp64 || bytes >= LBM_CACHE_BYTES_MIN)) return LBM_CACHED_ALL;
-  if ((!rows && !fp64) || bytes < LBM_CACHE_BYTES_MIN) return 0;
+  if ((!rows && !fp64 && min_nx < LBM_CACHE_PART_NX) || bytes < LBM_CACHE_BYTES_MIN) return 0;
   int i = 0;
   while (i < LBM_CACHED_ALL && LBM_CACHED[i + 1] / 27.0 * bytes <= LBM_CACHE_BYTES) ++i;
   return i;
@@ -337,8 +340,10 @@ StepBuffers make_buffers(ekpnp_ctx* c) {
   b.lbm_wrows = c->lbm_wrows;
   const bool fp64 = c->opt.precision == EKPNP_POP_FP64;
   const double pop_bytes = 2.0 * (double)c->total_pops * (fp64 ? 8 : 4);
-  b.lbm_cached = lbm_cached_planes(pop_bytes, fp64, false);
-  b.lbm_rows_cached = lbm_cached_planes(pop_bytes, fp64, true);
+  int min_nx = MAX_NX;
+  for (const auto& d : c->desc) min_nx = std::min(min_nx, d.nx);
+  b.lbm_cached = lbm_cached_planes(pop_bytes, fp64, false, min_nx);
+  b.lbm_rows_cached = lbm_cached_planes(pop_bytes, fp64, true, min_nx);
   return b;
 }
 

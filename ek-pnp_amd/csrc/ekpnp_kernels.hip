@@ -43,8 +43,7 @@ namespace ekpnp {
 constexpr double W0 = 4.0 / 9.0, WS = 1.0 / 9.0, WD = 1.0 / 36.0;  // LBM.h:105-107
 
 // Build-time tuning of k_lbm:
-//   EKPNP_LBM_WAVES N: ask for at least N waves per SIMD (register budget);
-//                      3 holds every variant to 168 VGPRs, which none spills
+//   EKPNP_LBM_WAVES N: ask for at least N waves per SIMD (register budget)
 #ifndef EKPNP_LBM_WAVES
 #define EKPNP_LBM_WAVES 3
 #endif
@@ -74,8 +73,7 @@ __device__ __forceinline__ void st_pop(S* p, S v) {
 
 // The (wave-uniform) plane stride as a value of its own.  Addresses formed from
 // it are computed where they are used: with the loads' stride the compiler keeps
-// all 27 plane offsets in registers from the gather to the stores (k_lbm with
-// FP32 storage: 168 VGPRs and 8 bytes of scratch per lane; this way 142, none).
+// all 27 plane offsets in registers from the gather to the stores.
 __device__ __forceinline__ long long own_stride(long long plane) {
   unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)plane);
   unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(plane >> 32));
@@ -178,6 +176,10 @@ __device__ __forceinline__ NodeRefs node_refs(const StepBuffers& b, const ChanDe
                   load_rowj(R, ym), load_rowj(R, y), load_rowj(R, yp)};
 }
 
+// a b + c in one rounding, whatever surrounds it
+__device__ __forceinline__ double pinned_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float pinned_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 // direction x-components c_ix of D2Q9 (0, E, N, W, S, NE, NW, SW, SE)
 __device__ constexpr int CX[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
 
@@ -237,7 +239,7 @@ __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plan
 #pragma unroll
       for (int d = 0; d < 9; ++d) {
         q[9 * s + d] = (C)ld_pop<true>(P + (9 * s + d) * plane + r0 + x);
-        if (REF && CX[d] != 0) q[9 * s + d] += C(CX[d] * (d < 5 ? WS : WD)) * j;
+        if (REF && CX[d] != 0) q[9 * s + d] = pinned_fma(C(CX[d] * (d < 5 ? WS : WD)), j, q[9 * s + d]);
       }
     }
     return;
@@ -254,6 +256,18 @@ __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plan
 template <typename C>
 __device__ __forceinline__ C to_stored(C v, int d, C j) {
   return CX[d] == 0 ? v : v - C(CX[d] * (d < 5 ? WS : WD)) * j;
+}
+
+// the same on the first step from the pre-collision form: the flux term was
+// added when the node was loaded, and its product with the weight, rounded
+// once, is taken off again; c_W's is fused.  (The compiler's own choice, kept
+// whatever surrounds the expression.)
+template <typename C>
+__device__ __forceinline__ C to_stored_from_q(C v, int d, C j) {
+#pragma clang fp contract(off)
+  if (CX[d] == 0) return v;
+  if (d == 3) return pinned_fma(C(WS), j, v);
+  return v - C(CX[d] * (d < 5 ? WS : WD)) * j;
 }
 
 // the 9 populations of species s of a node, its flux term j
@@ -308,17 +322,23 @@ __device__ __forceinline__ void trt_pair(C& a, C& b, C w, C dX, C X, C om, C t, 
   b = b - omp * np + omm * nm;
 }
 
+// x^2 + y^2, y^2 rounded on its own
+template <typename C>
+__device__ __forceinline__ C sum_sq(C x, C y) { return pinned_fma(x, x, y * y); }
+
 template <typename C>
 __device__ __forceinline__ void collide_ion(C* q, C dX, C X, C vx, C vy, C omp, C omm, C ics,
                                             C ticf, C rest_om) {
-  const C om = C(-0.5) * (vx * vx + vy * vy) * ics;
+  const C om = C(-0.5) * sum_sq(vx, vy) * ics;
   const C tx = vx * ticf, ty = vy * ticf;
   const C eq0 = C(W0) * (dX + X * rest_om);
   q[0] = q[0] - omp * (q[0] - eq0);
   trt_pair(q[1], q[3], C(WS), dX, X, om, tx, omp, omm);
   trt_pair(q[2], q[4], C(WS), dX, X, om, ty, omp, omm);
-  trt_pair(q[5], q[7], C(WD), dX, X, om, tx + ty, omp, omm);
-  trt_pair(q[6], q[8], C(WD), dX, X, om, ty - tx, omp, omm);
+  // tx + ty and ty - tx, ty = vy ticf unrounded in both: pinned, the compiler's
+  // own choice of what to fuse depends on the code around the call
+  trt_pair(q[5], q[7], C(WD), dX, X, om, pinned_fma(vy, ticf, tx), omp, omm);
+  trt_pair(q[6], q[8], C(WD), dX, X, om, pinned_fma(vy, ticf, -tx), omp, omm);
 }
 
 // Fluid pair with the Guo source split into its even part
@@ -339,9 +359,8 @@ __device__ __forceinline__ void trt_pair_src(C& a, C& b, C w, C dX, C X, C om, C
 
 template <typename C>
 __device__ __forceinline__ void collide_fluid(C* q, C dr, C rho, C ux, C uy, C Fx, C Fy, C omp,
-                                              C omm, C ics, C icfl, C sp_dt, C sm_dt) {
+                                              C omm, C ics, C icfl, C om, C sp_dt, C sm_dt) {
   const C ticf = ics * icfl;
-  const C om = C(-0.5) * (ux * ux + uy * uy) * ics;
   const C tx = ux * ticf, ty = uy * ticf;
   const C uF = ux * Fx + uy * Fy;
   const C cFx = Fx * icfl, cFy = Fy * icfl;
@@ -349,8 +368,11 @@ __device__ __forceinline__ void collide_fluid(C* q, C dr, C rho, C ux, C uy, C F
   q[0] = q[0] - omp * (q[0] - eq0) + sp_dt * (C(W0) * ics * (-uF));
   trt_pair_src(q[1], q[3], C(WS), dr, rho, om, tx, omp, omm, uF, cFx, ics, sp_dt, sm_dt);
   trt_pair_src(q[2], q[4], C(WS), dr, rho, om, ty, omp, omm, uF, cFy, ics, sp_dt, sm_dt);
-  trt_pair_src(q[5], q[7], C(WD), dr, rho, om, tx + ty, omp, omm, uF, cFx + cFy, ics, sp_dt, sm_dt);
-  trt_pair_src(q[6], q[8], C(WD), dr, rho, om, ty - tx, omp, omm, uF, cFy - cFx, ics, sp_dt, sm_dt);
+  // the diagonals' t and c.F, pinned as in collide_ion
+  trt_pair_src(q[5], q[7], C(WD), dr, rho, om, pinned_fma(uy, ticf, tx), omp, omm, uF, pinned_fma(Fy, icfl, cFx), ics,
+               sp_dt, sm_dt);
+  trt_pair_src(q[6], q[8], C(WD), dr, rho, om, pinned_fma(uy, ticf, -tx), omp, omm, uF, pinned_fma(Fy, icfl, -cFx), ics,
+               sp_dt, sm_dt);
 }
 
 template <typename S>
@@ -388,16 +410,17 @@ __device__ __forceinline__ Moments<C> moments(const C* q, const ChanDesc* __rest
 // k_lbm: one coupled-step LBM update of every node of every channel.
 // ---------------------------------------------------------------------------
 // S: storage type of the populations; C: arithmetic type of the collision.
+// One node.  A function of restrict pointers, not the kernel's own body: the
+// descriptor's fields then stay scalar loads past the stores instead of being
+// read again into vector registers.  127 VGPRs with FP32 storage and 106 with
+// FP64 storage, four waves per SIMD (168 and 157 in one body, three): 300
+// channels of n_x = 32 82 -> 68 us a step, 2000 of n_x = 8 239 -> 218,
+// 1000x1001 209 -> 201.  Bound: HBM, or at a few work-groups per CU the loads'
+// latency and the FP64 issue rate of a lone wave (8 clocks an instruction).
 template <typename S, typename C, bool FROM_Q, bool MACRO, int CACHED>
-__global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, const int2* __restrict__ tiles,
-                                                const S* __restrict__ src, S* __restrict__ dst) {
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
-  const int2 tile = tiles[wg];
-  const ChanDesc* __restrict__ cd = b.chans + tile.x;
-  if (!cd->active) return;  // converged channel, frozen by the residual driver
+__device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int node,
+                                           const S* __restrict__ src, S* __restrict__ dst) {
   const int nx = cd->nx, ny = cd->ny;
-  const int node = tile.y + (int)threadIdx.x;
-  if (node >= nx * ny) return;
   const int y = node / nx;
   const int x = node - y * nx;
   const long long plane = cd->plane;
@@ -461,6 +484,7 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
   }
 
   // charge density for the Poisson solve, summed in FP64
+  double rho_e;
   {
     double sp = 0.0, sn = 0.0;
 #pragma unroll
@@ -468,7 +492,8 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
       sp += (double)q[9 + k];
       sn += (double)q[18 + k];
     }
-    b.rho_e[cd->fld_off + node] = (sp - sn) + (Xo[1] - Xo[2]);
+    rho_e = (sp - sn) + (Xo[1] - Xo[2]);
+    b.rho_e[cd->fld_off + node] = rho_e;
   }
   if (MACRO) {
     const long long o = cd->fld_off + node, st = b.macro_stride;
@@ -480,6 +505,10 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
   }
 
   const C ics = C(cd->inv_cs2), icfl = C(cd->inv_cfl), ticf = ics * icfl;
+  // which square is rounded on its own is pinned; FP32 storage with FP64
+  // arithmetic does it the other way round
+  const C u2 = REF && std::is_same<C, double>::value && !FROM_Q ? sum_sq(ux, uy) : sum_sq(uy, ux);
+  const C om_f = C(-0.5) * u2 * ics;
   // ions: drift velocity u + K E (LBM.cu:479-488)
   {
     const C Eix = C(Ex + cd->drift_app), Eiy = C(Ey);
@@ -487,9 +516,8 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
     const C kp = C(cd->kp), kn = C(cd->kn);
     const C vpx = ux + kp * Eix, vpy = uy + kp * Eiy;
     const C vnx = ux + kn * Eix, vny = uy + kn * Eiy;
-    const C om_p = C(-0.5) * (vpx * vpx + vpy * vpy) * ics;
-    const C om_n = C(-0.5) * (vnx * vnx + vny * vny) * ics;
-    const C om_f = C(-0.5) * (ux * ux + uy * uy) * ics;
+    const C om_p = C(-0.5) * sum_sq(vpx, vpy) * ics;
+    const C om_n = C(-0.5) * sum_sq(vnx, vny) * ics;
     collide_ion(q + 9, m.dcp, cp, vpx, vpy, C(cd->om_pp), C(cd->om_mp), ics, ticf, om_p);
     collide_ion(q + 18, m.dcn, cn, vnx, vny, C(cd->om_pn), C(cd->om_mn), ics, ticf,
                 (cd->flags & FLAG_G0_FLUID_U) ? om_f : om_n);
@@ -509,16 +537,16 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
     q[5] = f7 + md;
     q[6] = f8 - md;
   } else {
-    collide_fluid(q, m.dr, m.rho, ux, uy, m.Fx, m.Fy, C(cd->om_pf), C(cd->om_mf), ics, icfl,
+    collide_fluid(q, m.dr, m.rho, ux, uy, m.Fx, m.Fy, C(cd->om_pf), C(cd->om_mf), ics, icfl, om_f,
                   C(cd->src_p * cd->dt), C(cd->src_m * cd->dt));
   }
-  if constexpr (FROM_Q) {  // the flux term subtracted here is the one that load_pre added: as a loop,
-                           // the compiler contracts both alike
+  if constexpr (FROM_Q) {
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
       const C j = REF ? C(rf.jo.J[s] * tc) : C(0);
 #pragma unroll
-      for (int d = 0; d < 9; ++d) st_pop<true>(Q + (9 * s + d) * plane + node, (S)to_stored(q[9 * s + d], d, j));
+      for (int d = 0; d < 9; ++d)
+        st_pop<true>(Q + (9 * s + d) * plane + node, (S)(REF ? to_stored_from_q(q[9 * s + d], d, j) : q[9 * s + d]));
     }
   } else {
     const long long sp = own_stride(plane);
@@ -526,6 +554,18 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
     store_species<1, CACHED>(Q, sp, node, q + 9, REF ? C(rf.jo.J[1] * tc) : C(0));
     store_species<2, CACHED>(Q, sp, node, q + 18, REF ? C(rf.jo.J[2] * tc) : C(0));
   }
+  return rho_e;
+}
+
+template <typename S, typename C, bool FROM_Q, bool MACRO, int CACHED>
+__global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, const int2* __restrict__ tiles,
+                                                const S* __restrict__ src, S* __restrict__ dst) {
+  const int2 tile = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+  const ChanDesc* __restrict__ cd = b.chans + tile.x;
+  if (!cd->active) return;  // converged channel, frozen by the residual driver
+  const int node = tile.y + (int)threadIdx.x;
+  if (node >= cd->nx * cd->ny) return;
+  lbm_node<S, C, FROM_Q, MACRO, CACHED>(b, cd, node, src, dst);
 }
 
 // ---------------------------------------------------------------------------
@@ -649,7 +689,7 @@ __device__ __forceinline__ void gather9(const float* __restrict__ B, long long p
 // way, and in 136 (3 waves) when the flag is a template parameter and false.
 // Wall rows (2 of ny) are always streamed.
 template <bool WALL, int CACHED>
-__device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int y, int x,
+__device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int y, int x,
                                              const WaveRefs& rf, const float* __restrict__ P, float* __restrict__ Q,
                                              bool macro) {
   using C = double;
@@ -761,7 +801,8 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
     m.uy = (jy * icfl + m.Fy * hdt) * irho;
   }
   const C ux = bottom ? mux : m.ux, uy = bottom ? muy : m.uy;
-  b.rho_e[cd->fld_off + node] = (sp - sn) + (Xo[1] - Xo[2]);
+  const double rho_e = (sp - sn) + (Xo[1] - Xo[2]);
+  b.rho_e[cd->fld_off + node] = rho_e;
   if (macro) {
     const long long o = cd->fld_off + node, st = b.macro_stride;
     b.macro[M_RHO * st + o] = (double)m.rho;
@@ -772,16 +813,16 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
   }
 
   const C ics = C(cd->inv_cs2), icfl = C(cd->inv_cfl), ticf = ics * icfl;
+  const C om_f = C(-0.5) * sum_sq(uy, ux) * ics;
   // ions: drift velocity u + K E (LBM.cu:479-488), collide, store
   {
     const C Eix = C(Ex + cd->drift_app), Eiy = C(Ey);
     const C kp = C(cd->kp), kn = C(cd->kn);
-    const C om_f = C(-0.5) * (ux * ux + uy * uy) * ics;
     C q[9];
     {
       const C cp = C(Xo[1]) + m.dcp;
       const C vpx = ux + kp * Eix, vpy = uy + kp * Eiy;
-      const C om_p = C(-0.5) * (vpx * vpx + vpy * vpy) * ics;
+      const C om_p = C(-0.5) * sum_sq(vpx, vpy) * ics;
       species_q(v + 9, rf, 1, tc, wall, dcwp, q);
       collide_ion(q, m.dcp, cp, vpx, vpy, C(cd->om_pp), C(cd->om_mp), ics, ticf, om_p);
       const C j = C(rf.J(1, 1) * tc);
@@ -790,7 +831,7 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
     {
       const C cn = C(Xo[2]) + m.dcn;
       const C vnx = ux + kn * Eix, vny = uy + kn * Eiy;
-      const C om_n = C(-0.5) * (vnx * vnx + vny * vny) * ics;
+      const C om_n = C(-0.5) * sum_sq(vnx, vny) * ics;
       species_q(v + 18, rf, 2, tc, wall, dcwn, q);
       collide_ion(q, m.dcn, cn, vnx, vny, C(cd->om_pn), C(cd->om_mn), ics, ticf,
                   (cd->flags & FLAG_G0_FLUID_U) ? om_f : om_n);
@@ -816,12 +857,13 @@ __device__ __forceinline__ void lbm_row_node(const StepBuffers& b, const ChanDes
       q[5] = f7 + md;
       q[6] = f8 - md;
     } else {
-      collide_fluid(q, m.dr, m.rho, ux, uy, m.Fx, m.Fy, C(cd->om_pf), C(cd->om_mf), ics, icfl,
+      collide_fluid(q, m.dr, m.rho, ux, uy, m.Fx, m.Fy, C(cd->om_pf), C(cd->om_mf), ics, icfl, om_f,
                     C(cd->src_p * cd->dt), C(cd->src_m * cd->dt));
     }
     const C j = C(rf.J(1, 0) * tc);
     store_species<0, CACHED>(Q, plane, node, q, j);
   }
+  return rho_e;
 }
 
 // Channels with nx a multiple of 64: the 64 nodes of a wave lie in one row
@@ -2927,9 +2969,7 @@ static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBu
       if (macro) hipLaunchKernelGGL((k_lbm<S, C, false, true, cached()>), grid, block, 0, s, b, gen, sp, dp);
       else hipLaunchKernelGGL((k_lbm<S, C, false, false, cached()>), grid, block, 0, s, b, gen, sp, dp);
     };
-    if constexpr (!std::is_same<S, float>::value) with_cached(b.lbm_cached, launch);
-    else if (b.lbm_cached == LBM_CACHED_ALL) launch(std::integral_constant<int, 27>{});
-    else launch(std::integral_constant<int, 0>{});
+    with_cached(b.lbm_cached, launch);
   }
   if (rows) {
     if (walls && b.n_lbm_wall_tiles > 0)

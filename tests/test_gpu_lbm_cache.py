@@ -33,11 +33,13 @@ def advance(nx, ny, precision, copies, compute):
 
 # both lattices of one copy: 13.8-14.2 MB (FP32 storage), 28.3 MB (FP64);
 # row kernel: none below 80 MB, then 27, 18, 13, 9, 6, 4, 2 and no planes;
-# k_lbm with FP32 storage: 27 up to 230 MB, then none; with FP64 storage: none,
+# k_lbm with FP32 storage: 27 up to 230 MB, then 13, 6, 2, or with
+# narrow channels none; with FP64 storage: none,
 # 27, 13, 9, 4
 @pytest.mark.parametrize("nx,ny,precision,compute,batches", [
     (1024, 64, "fp32", True, (5, 6, 11, 12, 16, 20, 30, 45, 70, 100, 160)),
-    (1000, 64, "fp32", True, (16, 17)),
+    (1000, 64, "fp32", True, (16, 17, 24, 45, 90)),
+    (32, 256, "fp32", True, (130, 131)),
     (1000, 64, "fp32", False, (16, 17)),
     (1024, 64, "fp64", True, (2, 3, 8, 9, 12, 35)),
 ])
