@@ -99,6 +99,10 @@ struct ekpnp_ctx {
   int2* d_lbm_split = nullptr;   // lbm_split on the device
   std::vector<int2> lbm_split;   // LBM tiles for the step: row-kernel interior, row-kernel wall, others
   int n_lbm_row = 0, n_lbm_wall = 0;
+  std::vector<int2> lbm_fwd;     // k_lbm_fwd tiles; empty: the context is too wide or too large for it
+  int2* d_lbm_fwd = nullptr;
+  int lbm_fwd_kind = FWD_GENERAL;
+  bool lbm_fuse = false;         // the step takes k_lbm_fwd (the Poisson plan's x-transform is the one it holds)
   int lbm_wrows = 0;             // interior tile shape of the row kernel (0: consecutive blocks)
   size_t lbm_split_cap = 0;      // capacity of d_lbm_split (the largest shape)
   // the coupled step updates the row kernel's wall tiles inside the
@@ -338,6 +342,9 @@ StepBuffers make_buffers(ekpnp_ctx* c) {
   b.lbm_gen_tiles = c->d_lbm_split + c->n_lbm_row + c->n_lbm_wall;
   b.n_lbm_gen_tiles = (int)c->lbm_split.size() - c->n_lbm_row - c->n_lbm_wall;
   b.lbm_wrows = c->lbm_wrows;
+  b.lbm_fwd_tiles = c->d_lbm_fwd;
+  b.n_lbm_fwd_tiles = (int)c->lbm_fwd.size();
+  b.lbm_fwd_kind = c->lbm_fwd_kind;
   const bool fp64 = c->opt.precision == EKPNP_POP_FP64;
   const double pop_bytes = 2.0 * (double)c->total_pops * (fp64 ? 8 : 4);
   int min_nx = MAX_NX;
@@ -363,7 +370,7 @@ void release(ekpnp_ctx* c) {
                   c->d_tri_tiles, c->d_first_tile, c->d_rho_e, c->d_psi, c->d_macro,
                   c->d_walls, c->d_tw, c->d_spec, c->d_ux_prev, c->d_partials, c->d_red,
                   c->d_refs, c->d_refs_new, c->d_row_tiles, c->d_cprime, c->d_lbm_split,
-                  c->d_blocks, c->d_blocks_new, c->d_diag};
+                  c->d_blocks, c->d_blocks_new, c->d_diag, c->d_lbm_fwd};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->stage) (void)hipHostFree(c->stage);
@@ -416,6 +423,48 @@ void build_lbm_split(ekpnp_ctx* c, int wrows) {
   c->lbm_wrows = wrows;
 }
 
+// x-transform of a channel, in the order of the FFT tile table: 0 power-of-two
+// FFT, 1 matrix-core direct DFT, 2 direct DFT of narrow rows
+int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2; }
+
+// Tiles of k_lbm_fwd: contexts of FP64 arithmetic whose every channel has rows
+// of at most LBM_WG nodes, of a power of two or of the narrow rows' direct DFT,
+// as long as the chip is not full: the transform holds every work-group for
+// some us longer, which is less than the launch it saves only while there are
+// few work-groups a CU (n_cu = 256).  Step in us, launches apart -> one launch:
+//   10x101 fp64               4 tiles  18.4 -> 15.6
+//   64x128 fp64              32        21.7 -> 18.7
+//   256x256 fp32            256        26.0 -> 23.4
+//   32 channels (32, 64)    576        35.2 -> 31.9
+//   64x128 x25 fp32         800        33.0 -> 31.4
+//   512 channels n_x = 4   1280        47.0 -> 45.0
+//   64x128 x50 fp32        1600        43.7 -> 42.9   n_x = 32 x150  1950  44.1 -> 45.3
+//   64x128 x64 fp64        2048        57.8 -> 54.9   64x128 x200 fp64  6400  150.4 -> 154.9
+//   n_x = 4 x1000          2500        74.6 -> 69.6   n_x = 4 x2000     5000  141.9 -> 151.2
+//   64x128 x100 fp32       3200        60.8 -> 67.4
+constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_LONG = 10;  // the latter: FP64 storage, narrow rows only
+void build_lbm_fwd(ekpnp_ctx* c) {
+  c->lbm_fwd.clear();
+  for (auto& d : c->desc) d.lbm_span = d.nx <= LBM_WG ? LBM_WG / d.nx * d.nx : LBM_WG;
+  if (c->opt.precision == EKPNP_POP_FP32 && !c->opt.compute_fp64) return;
+  for (const auto& d : c->desc)
+    if (d.nx > LBM_WG || x_family(d) == 1) return;
+  const char* env = std::getenv("EKPNP_LBM_ROWS");
+  const bool use_rows = c->opt.precision == EKPNP_POP_FP32 && !(env && env[0] == '0');
+  int n_rows = 0;
+  for (int i = 0; i < c->nchan; ++i) {
+    const ChanDesc& d = c->desc[i];
+    n_rows += use_rows && d.nx % 64 == 0;
+    for (int n = 0; n < d.nx * d.ny; n += d.lbm_span) c->lbm_fwd.push_back(make_int2(i, n));
+  }
+  c->lbm_fwd_kind = n_rows == 0 ? FWD_GENERAL : n_rows == c->nchan ? FWD_ROWS : FWD_MIXED;
+  bool pow2 = false;
+  for (const auto& d : c->desc) pow2 = pow2 || d.pow2;
+  const bool longer = !pow2 || c->opt.precision == EKPNP_POP_FP64;
+  if (c->lbm_fwd.size() > (size_t)(longer ? LBM_FWD_TILES_PER_CU_LONG : LBM_FWD_TILES_PER_CU) * c->n_cu)
+    c->lbm_fwd.clear();
+}
+
 // a new interior tile shape for the row kernel: table, buffers, graphs
 hipError_t apply_lbm_tiles(ekpnp_ctx* c, int wrows) {
   hipError_t e = hipStreamSynchronize(c->stream);  // no launch still reads the table
@@ -435,10 +484,6 @@ hipError_t apply_lbm_tiles(ekpnp_ctx* c, int wrows) {
   drop_graphs(c);
   return hipSuccess;
 }
-
-// x-transform of a channel, in the order of the FFT tile table: 0 power-of-two
-// FFT, 1 matrix-core direct DFT, 2 direct DFT of narrow rows
-int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2; }
 
 // Poisson work decomposition.  x-FFT: a work-group transforms whole rows,
 // up to fft_elems complex values (power-of-two channels and narrow others; the
@@ -608,6 +653,8 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
     const long long nt = (long long)c->tri_tiles.size(), nw = (c->n_lbm_wall + 7) & ~7;
     c->walls_in_tri = !(env && env[0] == '0') && nw > 0 && (nt + nw + slots - 1) / slots == (nt + slots - 1) / slots;
   }
+  c->lbm_fuse = !c->lbm_fwd.empty() && (n_fft_pow2 == 0 || c->sb.fft_persist == 1);
+  if (c->lbm_fuse) c->walls_in_tri = false;
   c->fft_elems = fft_elems;
   c->tri_rows = tri_rows;
   c->fft_persist = c->sb.fft_pair_s > 0 ? 2 : c->sb.fft_persist;
@@ -651,14 +698,21 @@ bool defer_walls(const ekpnp_ctx* c) {
 }
 
 // one coupled step: collide-stream, then the Poisson stages; ev (optional)
-// receives an event after each of the four launches
+// receives an event after each of the four stages
 hipError_t enqueue_step(ekpnp_ctx* c, bool macro, hipEvent_t* ev = nullptr) {
-  const bool defer = defer_walls(c);
+  const bool fuse = c->lbm_fuse && !c->state_q;
+  const bool defer = !fuse && defer_walls(c);
   const void* src = c->lat[c->cur];
   void* dst = c->lat[c->cur ^ 1];
-  hipError_t e = enqueue_lbm(c, macro, !defer);
+  hipError_t e;
+  if (fuse) {
+    e = launch_lbm_fwd(c->opt.precision, macro, c->sb, src, dst, c->stream);
+    c->cur ^= 1;
+  } else {
+    e = enqueue_lbm(c, macro, !defer);
+  }
   if (e == hipSuccess && ev) e = hipEventRecord(ev[0], c->stream);
-  if (e == hipSuccess) e = launch_poisson_fwd(c->sb, c->stream);
+  if (e == hipSuccess && !fuse) e = launch_poisson_fwd(c->sb, c->stream);
   if (e == hipSuccess && ev) e = hipEventRecord(ev[1], c->stream);
   if (e == hipSuccess)
     e = defer ? launch_poisson_tri_walls(macro, c->sb, src, dst, c->stream) : launch_poisson_tri(c->sb, c->stream);
@@ -1062,6 +1116,7 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
     wall += (int)pad64(d.nx);
     c->desc[i] = d;
   }
+  build_lbm_fwd(c);
   c->total_pops = pop;
   c->total_nodes = fld;
   c->total_spec = spec;
@@ -1123,6 +1178,7 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
     if ((e = dalloc(c, &c->d_desc, n_channels)) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_lbm_tiles, c->lbm_tiles.size())) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_lbm_split, c->lbm_split_cap)) != hipSuccess) return e;
+    if ((e = dalloc(c, &c->d_lbm_fwd, c->lbm_fwd.size())) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_fft_tiles, c->fft_tiles_cap)) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_tri_tiles, c->tri_tiles_cap)) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_first_tile, c->first_tile.size())) != hipSuccess) return e;
@@ -1157,6 +1213,9 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
     if ((e = hipMemcpy(c->d_desc, c->desc.data(), n_channels * sizeof(ChanDesc), hipMemcpyHostToDevice)) != hipSuccess) return e;
     if ((e = hipMemcpy(c->d_lbm_tiles, c->lbm_tiles.data(), c->lbm_tiles.size() * sizeof(int2), hipMemcpyHostToDevice)) != hipSuccess) return e;
     if ((e = hipMemcpy(c->d_lbm_split, c->lbm_split.data(), c->lbm_split.size() * sizeof(int2), hipMemcpyHostToDevice)) != hipSuccess) return e;
+    if (!c->lbm_fwd.empty() &&
+        (e = hipMemcpy(c->d_lbm_fwd, c->lbm_fwd.data(), c->lbm_fwd.size() * sizeof(int2), hipMemcpyHostToDevice)) != hipSuccess)
+      return e;
     if ((e = hipMemcpy(c->d_first_tile, c->first_tile.data(), c->first_tile.size() * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess) return e;
     if ((e = hipMemcpy(c->d_walls, c->walls.data(), c->walls.size() * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess) return e;
     if ((e = hipMemcpy(c->d_tw, tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice)) != hipSuccess) return e;

@@ -16,6 +16,8 @@ enum WallPlane { W_PSI_LO = 0, W_PSI_HI = 1, W_CP_LO = 2, W_CP_HI = 3, W_CN_LO =
 // Macroscopic output planes (FP64), each of total_nodes elements.
 enum MacroPlane { M_RHO = 0, M_UX = 1, M_UY = 2, M_CP = 3, M_CN = 4, M_COUNT = 5 };
 
+// node updates a k_lbm_fwd launch holds: k_lbm's, the row kernel's, or both
+constexpr int FWD_GENERAL = 1, FWD_ROWS = 2, FWD_MIXED = 3;
 // population planes (in storage order, of 27) that the LBM kernels read and
 // write through the caches; the others are streamed past them
 constexpr int LBM_CACHED[] = {0, 2, 4, 6, 9, 13, 18, 27};
@@ -80,6 +82,7 @@ struct ChanDesc {
   int tw_off;                   // offset of this channel's twiddles e^{-2 pi i j/nx}
   int pow2;                     // nx is a power of two (Stockham path)
   int fft_rows;                 // rows per FFT work-group
+  int lbm_span;                 // nodes per k_lbm_fwd tile: whole rows
   int tri_C, tri_G, tri_L, tile0;  // tridiagonal chunks, modes per WG, rows per chunk
   // collision constants (double; the FP32 kernel rounds them once)
   double inv_cfl, inv_cs2;
@@ -111,6 +114,9 @@ struct StepBuffers {
   int n_lbm_wall_tiles;
   const int2* lbm_gen_tiles;
   int n_lbm_gen_tiles;
+  const int2* lbm_fwd_tiles;    // (channel, first node) per k_lbm_fwd work-group
+  int n_lbm_fwd_tiles;
+  int lbm_fwd_kind;             // FWD_GENERAL, FWD_ROWS or FWD_MIXED
   int lbm_cached, lbm_rows_cached;  // cached planes of k_lbm and k_lbm_rows (indices into LBM_CACHED)
   int lbm_wrows;                // row-kernel interior tiles: 0 consecutive blocks, else rows per tile (2, 4)
   const int4* fft_tiles;        // (channel, first row, rows, matrix-core DFT: row tiles) per FFT work-group
@@ -158,6 +164,7 @@ struct StepBuffers {
 hipError_t launch_lbm_rows_interior(const StepBuffers& b, const void* src, void* dst, hipStream_t s);
 hipError_t launch_lbm(int precision, bool compute64, bool from_q, bool macro, const StepBuffers& b,
                       const void* src, void* dst, hipStream_t s, bool walls = true);
+hipError_t launch_lbm_fwd(int precision, bool macro, const StepBuffers& b, const void* src, void* dst, hipStream_t s);
 hipError_t launch_poisson_fwd(const StepBuffers& b, hipStream_t s);
 hipError_t launch_poisson_tri(const StepBuffers& b, hipStream_t s);
 // the tridiagonal plus the row kernel's wall tiles of the collide-stream that

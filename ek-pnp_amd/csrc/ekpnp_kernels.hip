@@ -185,23 +185,46 @@ __device__ constexpr int CX[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
 
 // The gathered species' stored values v (FP32 storage) plus the reference
 // terms of their sources: q_i = v_i + w_i (X(src) - X(node)) + w_i c_ix tc J(src row)
-// with dX = X(src) - X(node) and the row fluxes (times tc) j0 (row y), jm
-// (y-1), jp (y+1).
-template <typename C>
-__device__ __forceinline__ void add_src_refs(C* q, const double* dX, C j0, C jm, C jp) {
-  q[1] += C(WS) * (C(dX[1]) + j0);
-  q[3] += C(WS) * (C(dX[3]) - j0);
-  q[2] += C(WS) * C(dX[2]);
-  q[4] += C(WS) * C(dX[4]);
-  q[5] += C(WD) * (C(dX[5]) + jm);
-  q[6] += C(WD) * (C(dX[6]) - jm);
-  q[7] += C(WD) * (C(dX[7]) - jp);
-  q[8] += C(WD) * (C(dX[8]) + jp);
+// with dX = X(src) - X(node) and the row fluxes J0 (row y), Jm (y-1), Jp (y+1).
+// Pinned: the products of the row fluxes with tc go into the sums unrounded for
+// row y if FUSE0, for rows y-1 and y+1 if FUSE1 (as the compiler once chose:
+// k_lbm rounds the ions' of row y, which its wall rule and stores take too; the
+// row kernel rounds none for the moments and all of them for the collision).
+__device__ __forceinline__ double plus_rounded(double a, double b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+template <bool FUSE>
+__device__ __forceinline__ double plus_flux(double dX, double J, double tc) {
+  return FUSE ? pinned_fma(J, tc, dX) : plus_rounded(dX, J * tc);
+}
+template <bool FUSE0, bool FUSE1>
+__device__ __forceinline__ void add_src_refs(double* q, const double* dX, double J0, double Jm, double Jp, double tc) {
+  q[1] += WS * plus_flux<FUSE0>(dX[1], J0, tc);
+  q[3] += WS * plus_flux<FUSE0>(dX[3], -J0, tc);
+  q[2] += WS * dX[2];
+  q[4] += WS * dX[4];
+  q[5] += WD * plus_flux<FUSE1>(dX[5], Jm, tc);
+  q[6] += WD * plus_flux<FUSE1>(dX[6], -Jm, tc);
+  q[7] += WD * plus_flux<FUSE1>(dX[7], -Jp, tc);
+  q[8] += WD * plus_flux<FUSE1>(dX[8], Jp, tc);
+}
+template <bool FUSE0, bool FUSE1>
+__device__ __forceinline__ void add_src_refs(float* q, const double* dX, double J0, double Jm, double Jp, double tc) {
+  const float j0 = (float)(J0 * tc), jm = (float)(Jm * tc), jp = (float)(Jp * tc);
+  q[1] += float(WS) * ((float)dX[1] + j0);
+  q[3] += float(WS) * ((float)dX[3] - j0);
+  q[2] += float(WS) * (float)dX[2];
+  q[4] += float(WS) * (float)dX[4];
+  q[5] += float(WD) * ((float)dX[5] + jm);
+  q[6] += float(WD) * ((float)dX[6] - jm);
+  q[7] += float(WD) * ((float)dX[7] - jp);
+  q[8] += float(WD) * ((float)dX[8] + jp);
 }
 
 // the gather of one species: stored values from the upstream neighbours of
 // node x (rows at offsets rm, r0, rp) plus the reference terms of their sources
-template <typename S, typename C, bool REF, int s, int CACHED>
+template <typename S, typename C, bool REF, int s, int CACHED, bool FUSE0>
 __device__ __forceinline__ void load_species(const S* P, long long plane, long long rm, long long r0,
                                              long long rp, int x, int xm, int xp, const NodeRefs& rf, double tc,
                                              C* q) {
@@ -219,7 +242,7 @@ __device__ __forceinline__ void load_species(const S* P, long long plane, long l
   if (REF) {
     double dX[9];
     rf.diffs(s, dX);
-    add_src_refs(q + p, dX, C(rf.jo.J[s] * tc), C(rf.jm.J[s] * tc), C(rf.jp.J[s] * tc));
+    add_src_refs<FUSE0 || s == 0, true>(q + p, dX, rf.jo.J[s], rf.jm.J[s], rf.jp.J[s], tc);
   }
 }
 
@@ -228,7 +251,7 @@ __device__ __forceinline__ void load_species(const S* P, long long plane, long l
 //   q_i = stored_i(src) + w_i (X(src) - X(node)) + w_i c_ix tc J(src).
 // 27 values: f 0..8, h 9..17, g 18..26.  REF false (FP64 storage): no
 // reference terms.
-template <typename S, typename C, bool FROM_Q, bool REF, int CACHED = 0>
+template <typename S, typename C, bool FROM_Q, bool REF, int CACHED, bool FUSE0>
 __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plane, int nx, int ny,
                                          int x, int y, int xm, int xp, const NodeRefs& rf, double tc, C* q) {
   const long long r0 = (long long)y * nx;
@@ -247,9 +270,9 @@ __device__ __forceinline__ void load_pre(const S* __restrict__ P, long long plan
   const int ym = (y == 0) ? ny - 1 : y - 1;
   const int yp = (y == ny - 1) ? 0 : y + 1;
   const long long rm = (long long)ym * nx, rp = (long long)yp * nx;
-  load_species<S, C, REF, 0, CACHED>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
-  load_species<S, C, REF, 1, CACHED>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
-  load_species<S, C, REF, 2, CACHED>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
+  load_species<S, C, REF, 0, CACHED, FUSE0>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
+  load_species<S, C, REF, 1, CACHED, FUSE0>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
+  load_species<S, C, REF, 2, CACHED, FUSE0>(P, plane, rm, r0, rp, x, xm, xp, rf, tc, q);
 }
 
 // stored value of rest deviation v in direction d of a row with flux term j = tc J
@@ -417,9 +440,9 @@ __device__ __forceinline__ Moments<C> moments(const C* q, const ChanDesc* __rest
 // channels of n_x = 32 82 -> 68 us a step, 2000 of n_x = 8 239 -> 218,
 // 1000x1001 209 -> 201.  Bound: HBM, or at a few work-groups per CU the loads'
 // latency and the FP64 issue rate of a lone wave (8 clocks an instruction).
-template <typename S, typename C, bool FROM_Q, bool MACRO, int CACHED>
+template <typename S, typename C, bool FROM_Q, int CACHED>
 __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int node,
-                                           const S* __restrict__ src, S* __restrict__ dst) {
+                                           const S* __restrict__ src, S* __restrict__ dst, bool macro) {
   const int nx = cd->nx, ny = cd->ny;
   const int y = node / nx;
   const int x = node - y * nx;
@@ -455,7 +478,7 @@ __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc*
       for (int s = 0; s < 3; ++s) X1[s] = r1.own(s);
     }
     const long long p1 = own_stride(plane);
-    load_pre<S, C, FROM_Q, REF, CACHED>(P, p1, nx, ny, x, 1, xm, xp, r1, tc, m1);
+    load_pre<S, C, FROM_Q, REF, CACHED, true>(P, p1, nx, ny, x, 1, xm, xp, r1, tc, m1);
     double Ex1, Ey1;
     efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1);
     const Moments<C> mm = moments(m1, cd, X1, Ex1, Ey1);
@@ -464,7 +487,7 @@ __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc*
   }
 
   C q[27];
-  load_pre<S, C, FROM_Q, REF, CACHED>(P, plane, nx, ny, x, y, xm, xp, rf, tc, q);
+  load_pre<S, C, FROM_Q, REF, CACHED, false>(P, plane, nx, ny, x, y, xm, xp, rf, tc, q);
   if (!FROM_Q && (bottom || top)) {
     const double* __restrict__ Wl = b.walls + cd->wall_off + x;
     const long long ws = b.walls_stride;
@@ -495,7 +518,7 @@ __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc*
     rho_e = (sp - sn) + (Xo[1] - Xo[2]);
     b.rho_e[cd->fld_off + node] = rho_e;
   }
-  if (MACRO) {
+  if (macro) {
     const long long o = cd->fld_off + node, st = b.macro_stride;
     b.macro[M_RHO * st + o] = (double)m.rho;
     b.macro[M_UX * st + o] = (double)ux;
@@ -565,7 +588,7 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
   if (!cd->active) return;  // converged channel, frozen by the residual driver
   const int node = tile.y + (int)threadIdx.x;
   if (node >= cd->nx * cd->ny) return;
-  lbm_node<S, C, FROM_Q, MACRO, CACHED>(b, cd, node, src, dst);
+  lbm_node<S, C, FROM_Q, CACHED>(b, cd, node, src, dst, MACRO);
 }
 
 // ---------------------------------------------------------------------------
@@ -632,13 +655,15 @@ __device__ __forceinline__ WaveRefs wave_refs(const StepBuffers& b, const ChanDe
                   k == 0 ? nb - 1 : k - 1, k, k + 1 == nb ? 0 : k + 1, lane};
 }
 
-// FP64 rest deviations of species sp from its gathered FP32 values (load_pre)
+// FP64 rest deviations of species sp from its gathered FP32 values (load_pre);
+// FUSE: for the moments, else for the collision
+template <bool FUSE>
 __device__ __forceinline__ void widen_species(const float* v, const WaveRefs& rf, int sp, double tc, double* q) {
 #pragma unroll
   for (int d = 0; d < 9; ++d) q[d] = (double)v[d];
   double dX[9];
   rf.diffs(sp, dX);
-  add_src_refs(q, dX, rf.J(1, sp) * tc, rf.J(0, sp) * tc, rf.J(2, sp) * tc);
+  add_src_refs<FUSE, FUSE>(q, dX, rf.J(1, sp), rf.J(0, sp), rf.J(2, sp), tc);
 }
 
 // wall node, one ion species: anti-bounce-back of its own stored
@@ -659,10 +684,11 @@ __device__ __forceinline__ void abb_species(const float* p, double dcw, double j
 
 // the 9 values of species s at row y (s = 0: gathered; ions: gathered, or on
 // a wall row anti-bounced from the node's own values, dcw = c_w - X_s)
+template <bool FUSE>
 __device__ __forceinline__ void species_q(const float* v, const WaveRefs& rf, int s, double tc, bool wall,
                                           double dcw, double* q) {
   if (s > 0 && wall) abb_species(v, dcw, rf.J(1, s) * tc, q);
-  else widen_species(v, rf, s, tc, q);
+  else widen_species<FUSE>(v, rf, s, tc, q);
 }
 
 // 9 FP32 values of species block B gathered for node x of row y (pull,
@@ -752,13 +778,13 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
   if (bottom) {
     const WaveRefs r1 = wave_refs(b, cd, 1, rf.k, rf.lane);
     C q[9], dr, jx, jy, dcp, dcn;
-    widen_species(w, r1, 0, tc, q);
+    widen_species<true>(w, r1, 0, tc, q);
     dr = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7])) + q[8];
     jx = (q[1] + q[5] + q[8]) - (q[3] + q[6] + q[7]);
     jy = (q[2] + q[5] + q[6]) - (q[4] + q[7] + q[8]);
-    widen_species(w + 9, r1, 1, tc, q);
+    widen_species<true>(w + 9, r1, 1, tc, q);
     dcp = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7])) + q[8];
-    widen_species(w + 18, r1, 2, tc, q);
+    widen_species<true>(w + 18, r1, 2, tc, q);
     dcn = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7])) + q[8];
     const double x0 = r1.own(0), x1 = r1.own(1), x2 = r1.own(2);
     const C rho = C(x0) + dr;
@@ -777,15 +803,15 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
   C jx, jy, sp = 0.0, sn = 0.0;
   {
     C q[9];
-    widen_species(v, rf, 0, tc, q);
+    widen_species<true>(v, rf, 0, tc, q);
     m.dr = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7])) + q[8];
     jx = (q[1] + q[5] + q[8]) - (q[3] + q[6] + q[7]);
     jy = (q[2] + q[5] + q[6]) - (q[4] + q[7] + q[8]);
-    species_q(v + 9, rf, 1, tc, wall, dcwp, q);
+    species_q<true>(v + 9, rf, 1, tc, wall, dcwp, q);
     m.dcp = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7])) + q[8];
 #pragma unroll
     for (int k = 0; k < 9; ++k) sp += q[k];
-    species_q(v + 18, rf, 2, tc, wall, dcwn, q);
+    species_q<true>(v + 18, rf, 2, tc, wall, dcwn, q);
     m.dcn = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7])) + q[8];
 #pragma unroll
     for (int k = 0; k < 9; ++k) sn += q[k];
@@ -823,7 +849,7 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
       const C cp = C(Xo[1]) + m.dcp;
       const C vpx = ux + kp * Eix, vpy = uy + kp * Eiy;
       const C om_p = C(-0.5) * sum_sq(vpx, vpy) * ics;
-      species_q(v + 9, rf, 1, tc, wall, dcwp, q);
+      species_q<false>(v + 9, rf, 1, tc, wall, dcwp, q);
       collide_ion(q, m.dcp, cp, vpx, vpy, C(cd->om_pp), C(cd->om_mp), ics, ticf, om_p);
       const C j = C(rf.J(1, 1) * tc);
       store_species<1, CACHED>(Q, plane, node, q, j);
@@ -832,7 +858,7 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
       const C cn = C(Xo[2]) + m.dcn;
       const C vnx = ux + kn * Eix, vny = uy + kn * Eiy;
       const C om_n = C(-0.5) * sum_sq(vnx, vny) * ics;
-      species_q(v + 18, rf, 2, tc, wall, dcwn, q);
+      species_q<false>(v + 18, rf, 2, tc, wall, dcwn, q);
       collide_ion(q, m.dcn, cn, vnx, vny, C(cd->om_pn), C(cd->om_mn), ics, ticf,
                   (cd->flags & FLAG_G0_FLUID_U) ? om_f : om_n);
       const C j = C(rf.J(1, 2) * tc);
@@ -841,7 +867,7 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
   }
   {
     C q[9];
-    widen_species(v, rf, 0, tc, q);
+    widen_species<false>(v, rf, 0, tc, q);
     if (wall) {
       // full-way bounce-back of the pre-collision state, f0 unchanged
       // (LBM.cu:816-846); moving-wall terms on the top wall only
@@ -977,7 +1003,7 @@ __global__ __launch_bounds__(LBM_WG) void k_to_q(StepBuffers b, const S* __restr
   if (REF) rf = node_refs(b, cd, x, y, xm, xp);
   const double tc = cd->inv_cs2 * cd->inv_cfl;
   C q[27];
-  load_pre<S, C, false, REF>(P, plane, nx, ny, x, y, xm, xp, rf, tc, q);
+  load_pre<S, C, false, REF, 0, true>(P, plane, nx, ny, x, y, xm, xp, rf, tc, q);
   if (y == 0 || y == ny - 1) {
     const double* __restrict__ Wl = b.walls + cd->wall_off + x;
     const long long ws = b.walls_stride;
@@ -1181,12 +1207,12 @@ __device__ __forceinline__ int sw(int i) { return i ^ ((i >> 4) & 15); }
 // one pass of 2^(lgN mod 4) when lgN is not a multiple of 4, then radix 16.
 // Each lane holds 16 values per pass.  twq is the quadrant table of e^{-2 pi i j/nx}.
 // ---------------------------------------------------------------------------
-template <int SIGN, int R, int WGT, bool TW2>
+template <int SIGN, int R, int WGT, bool TW2, int MAXE>
 __device__ __forceinline__ void stockham_pass(double2* x, int rows, int lgN, int lgn, int lgs,
                                               const double2* __restrict__ twq, int lgnx) {
   constexpr int LGR = R == 16 ? 4 : (R == 8 ? 3 : (R == 4 ? 2 : 1));
-  // butterflies per lane: rows N / R <= FFT_MAX_ELEMS / R of them over WGT lanes
-  constexpr int BPT = (FFT_MAX_ELEMS / R + WGT - 1) / WGT;
+  // butterflies per lane: rows N / R <= MAXE / R of them over WGT lanes
+  constexpr int BPT = (MAXE / R + WGT - 1) / WGT;
   const int lgm = lgn - LGR, s = 1 << lgs;
   const int lgper = lgN - LGR;
   const int nb = rows << lgper;
@@ -1250,27 +1276,27 @@ __device__ __forceinline__ void stockham_pass(double2* x, int rows, int lgN, int
 }
 
 // WGT lanes; MAXR = 16 (16 values per lane per pass) or 8 (one more pass,
-// half the registers: the 512-lane one-tile kernels)
-template <int SIGN, int WGT, int MAXR, bool TW2 = false>
+// half the registers: the 512-lane one-tile kernels); rows N <= MAXE
+template <int SIGN, int WGT, int MAXR, bool TW2 = false, int MAXE = FFT_MAX_ELEMS>
 __device__ __forceinline__ void stockham(double2* x, int rows, int N, int lgN, const double2* __restrict__ twq, int lgnx) {
   constexpr int LGM = MAXR == 16 ? 4 : 3;
   int lgn = lgN, lgs = 0;
   const int r = lgN % LGM;
   if (r == 1) {
-    stockham_pass<SIGN, 2, WGT, TW2>(x, rows, lgN, lgn, lgs, twq, lgnx);
+    stockham_pass<SIGN, 2, WGT, TW2, MAXE>(x, rows, lgN, lgn, lgs, twq, lgnx);
     lgn -= 1;
     lgs += 1;
   } else if (r == 2) {
-    stockham_pass<SIGN, 4, WGT, TW2>(x, rows, lgN, lgn, lgs, twq, lgnx);
+    stockham_pass<SIGN, 4, WGT, TW2, MAXE>(x, rows, lgN, lgn, lgs, twq, lgnx);
     lgn -= 2;
     lgs += 2;
   } else if (r == 3) {
-    stockham_pass<SIGN, 8, WGT, TW2>(x, rows, lgN, lgn, lgs, twq, lgnx);
+    stockham_pass<SIGN, 8, WGT, TW2, MAXE>(x, rows, lgN, lgn, lgs, twq, lgnx);
     lgn -= 3;
     lgs += 3;
   }
   while (lgn >= LGM) {
-    stockham_pass<SIGN, MAXR, WGT, TW2>(x, rows, lgN, lgn, lgs, twq, lgnx);
+    stockham_pass<SIGN, MAXR, WGT, TW2, MAXE>(x, rows, lgN, lgn, lgs, twq, lgnx);
     lgn -= LGM;
     lgs += LGM;
   }
@@ -1447,6 +1473,111 @@ __global__ __launch_bounds__(FFT_WG_ROWS) void k_fft_fwd(StepBuffers b, const in
       spec[spec_idx(cd->ny, y0 + r, k)] = acc;
     }
   }
+}
+
+// a - b, never contracted with the product that made a (the right-hand side
+// rounds -pc rho_e before the wall lift is taken off, as rhs_at's branches do)
+__device__ __forceinline__ double sub_pinned(double a, double b) {
+#pragma clang fp contract(off)
+  return a - b;
+}
+
+// ---------------------------------------------------------------------------
+// k_lbm_fwd: the collide-stream and the forward x-transforms of a small context
+// in one launch.  Tiles are whole rows (cd->lbm_span consecutive nodes), each
+// node on the row kernel's update (interior and wall rows) or k_lbm's; the
+// charge density goes on through LDS to the transform of those rows.  One
+// launch and one read of the charge density less, where a step is a chain of
+// launches of a few us each: an empty one takes 1.6 us in a graph, and each
+// begins by fetching descriptors, tables and rows that the one before has just
+// written.  64x128 with FP64 storage: 21.7 -> 18.7 us a step.  Bound: latency,
+// of the gather, of a lone wave's FP64 instructions, of the transform's passes.
+// The transforms are k_fft_fwd_p's and the narrow rows' of k_fft_fwd, operation
+// for operation.
+// ---------------------------------------------------------------------------
+constexpr int FUSE_ROWS = LBM_WG / 2 + 64;  // double2 of LDS rows (narrow: row stride nx | 1)
+constexpr int FUSE_TW = LBM_WG / 4;         // twiddles: a quadrant of at most LBM_WG nodes, or a narrow row's
+
+__device__ __forceinline__ void fused_fwd(const StepBuffers& b, const ChanDesc* __restrict__ cd, int node0, double rho_e,
+                                          double2* lds, const double2* twl) {
+  const int nx = cd->nx, ny = cd->ny, rows = cd->lbm_span / nx, tid = threadIdx.x;
+  const int y0 = node0 / nx;
+  const int r = tid / nx, n = tid - r * nx, y = y0 + r;
+  double2* __restrict__ spec = b.spec + cd->spec_off;
+  // right-hand side of the node (rhs_at); rows past the channel's end hold 0,
+  // wall rows are transformed and not stored
+  double rhs = -cd->pc_dy2 * rho_e;
+  const double* __restrict__ Wl = b.walls + cd->wall_off;
+  const long long ws = b.walls_stride;
+  if (y == 1) rhs = sub_pinned(rhs, Wl[W_PSI_LO * ws + n]);
+  if (y == ny - 2) rhs = sub_pinned(rhs, Wl[W_PSI_HI * ws + n]);
+  double* v = reinterpret_cast<double*>(lds);
+  if (cd->pow2) {
+    const int N = nx >> 1, lgN = ilog2(N), lgnx = lgN + 1, quarter = nx >> 2;
+    if (r < rows) v[2 * sw((r << lgN) + (n >> 1)) + (n & 1)] = rhs;
+    __syncthreads();
+    stockham<-1, LBM_WG, 16, false, LBM_WG / 2>(lds, rows, N, lgN, twl, lgnx);
+    const int lgr = ilog2(rows), k = tid >> lgr, ro = tid & (rows - 1), yo = y0 + ro;
+    if (k <= N && yo >= 1 && yo <= ny - 2) {
+      const double2 zk = lds[sw((ro << lgN) + (k & (N - 1)))];
+      const double2 zc = cconj(lds[sw((ro << lgN) + ((N - k) & (N - 1)))]);
+      const double2 E = make_double2(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));
+      const double2 dd = csub(zk, zc);
+      const double2 O = make_double2(0.5 * dd.y, -0.5 * dd.x);  // (zk - zc)/(2i)
+      spec[spec_idx(ny, yo, k)] = cadd(E, cmul(tw_half(twl, k, quarter), O));
+    }
+  } else {
+    const int ldv = nx | 1, nk = cd->nk;
+    if (r < rows) v[r * ldv + n] = rhs;
+    __syncthreads();
+    const int ro = tid / nk, k = tid - ro * nk, yo = y0 + ro;
+    if (ro < rows && yo >= 1 && yo <= ny - 2) {
+      const double* vr = v + ro * ldv;
+      double2 acc = make_double2(0.0, 0.0);
+      int idx = 0;
+      for (int m = 0; m < nx; ++m) {
+        const double2 w = twl[idx];
+        acc.x += vr[m] * w.x;
+        acc.y += vr[m] * w.y;
+        idx += k;
+        if (idx >= nx) idx -= nx;
+      }
+      spec[spec_idx(ny, yo, k)] = acc;
+    }
+  }
+}
+
+template <typename S, int KIND, int CACHED>
+__global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm_fwd(StepBuffers b, const int2* __restrict__ tiles,
+                                                                   const S* __restrict__ src, S* __restrict__ dst,
+                                                                   int macro) {
+  __shared__ double2 lds[FUSE_ROWS];
+  __shared__ double2 twl[FUSE_TW];
+  const int2 tile = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+  const ChanDesc* __restrict__ cd = b.chans + tile.x;
+  if (!cd->active) return;  // converged channel, frozen by the residual driver
+  const int nx = cd->nx, ny = cd->ny, tid = threadIdx.x;
+  if (tid < (cd->pow2 ? nx >> 2 : nx)) twl[tid] = b.tw[cd->tw_off + tid];
+  double rho_e = 0.0;
+  const bool general = KIND == FWD_GENERAL || (KIND == FWD_MIXED && (nx & 63) != 0);
+  if constexpr (KIND != FWD_GENERAL) {
+    const int node0 = tile.y + (tid & ~63);  // the wave's first node
+    if (!general && node0 < nx * ny) {
+      const int y = __builtin_amdgcn_readfirstlane(node0 / nx);
+      const int x0 = __builtin_amdgcn_readfirstlane(node0) - y * nx, x = x0 + (tid & 63);
+      const float* __restrict__ P = (cd->swap ? dst : src) + cd->pop_off;
+      float* __restrict__ Q = (cd->swap ? const_cast<float*>(src) : dst) + cd->pop_off;
+      const WaveRefs rf = wave_refs(b, cd, y, x0 >> 6, tid & 63);
+      if (y == 0 || y == ny - 1) rho_e = lbm_row_node<true, 0>(b, cd, y, x, rf, P, Q, macro != 0);
+      else rho_e = lbm_row_node<false, 0>(b, cd, y, x, rf, P, Q, macro != 0);
+    }
+  }
+  if constexpr (KIND != FWD_ROWS) {
+    const int node = tile.y + tid;
+    if (general && tid < cd->lbm_span && node < nx * ny)
+      rho_e = lbm_node<S, double, false, CACHED>(b, cd, node, src, dst, macro != 0);
+  }
+  fused_fwd(b, cd, tile.y, rho_e, lds, twl);
 }
 
 // ---------------------------------------------------------------------------
@@ -1764,13 +1895,6 @@ __global__ __launch_bounds__(FFT_WG_ROWS) void k_fft_inv(StepBuffers b, const in
 typedef double d4 __attribute__((ext_vector_type(4)));
 constexpr int DFT_LD_PAD = 2;               // row padding of a forward chunk (bank spread)
 constexpr int DFT_MODES = DFT_CHUNK / 32;   // modes of an inverse chunk, over wr
-
-// a - b, never contracted with the product that made a (the right-hand side
-// rounds -pc rho_e before the wall lift is taken off, as rhs_at's branches do)
-__device__ __forceinline__ double sub_pinned(double a, double b) {
-#pragma clang fp contract(off)
-  return a - b;
-}
 
 // (i + d) mod n for i, d < n: one of the two candidates wraps below zero
 __device__ __forceinline__ unsigned wrap_add(unsigned i, unsigned d, unsigned n) { return min(i + d, i + d - n); }
@@ -2976,6 +3100,31 @@ static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBu
       hipLaunchKernelGGL((k_lbm_rows<true, 0>), dim3(b.n_lbm_wall_tiles), block, 0, s, b, b.lbm_wall_tiles,
                          reinterpret_cast<const float*>(src), reinterpret_cast<float*>(dst), macro ? 1 : 0);
     launch_rows(b, src, dst, macro, s);
+  }
+  return hipGetLastError();
+}
+
+// the coupled step's collide-stream and forward x-transforms in one launch
+// (FP64 arithmetic, populations not in pre-collision form)
+hipError_t launch_lbm_fwd(int precision, bool macro, const StepBuffers& b, const void* src, void* dst, hipStream_t s) {
+  const dim3 grid(b.n_lbm_fwd_tiles), block(LBM_WG);
+  const int m = macro ? 1 : 0;
+  if (precision == 0) {
+    const float* sp = static_cast<const float*>(src);
+    float* dp = static_cast<float*>(dst);
+    if (b.lbm_fwd_kind == FWD_ROWS)
+      hipLaunchKernelGGL((k_lbm_fwd<float, FWD_ROWS, 0>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
+    else if (b.lbm_fwd_kind == FWD_MIXED)
+      hipLaunchKernelGGL((k_lbm_fwd<float, FWD_MIXED, 27>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
+    else
+      hipLaunchKernelGGL((k_lbm_fwd<float, FWD_GENERAL, 27>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
+  } else {
+    const double* sp = static_cast<const double*>(src);
+    double* dp = static_cast<double*>(dst);
+    if (b.lbm_cached == LBM_CACHED_ALL)
+      hipLaunchKernelGGL((k_lbm_fwd<double, FWD_GENERAL, 27>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
+    else
+      hipLaunchKernelGGL((k_lbm_fwd<double, FWD_GENERAL, 0>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
   }
   return hipGetLastError();
 }
