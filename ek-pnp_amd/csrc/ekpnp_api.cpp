@@ -102,6 +102,7 @@ struct ekpnp_ctx {
   std::vector<int2> lbm_fwd;     // k_lbm_fwd tiles; empty: the context is too wide or too large for it
   int2* d_lbm_fwd = nullptr;
   int lbm_fwd_kind = FWD_GENERAL;
+  bool lbm_inv = false;          // k_lbm_fwd does the step before's inverse x-transforms too
   bool lbm_fuse = false;         // the step takes k_lbm_fwd (the Poisson plan's x-transform is the one it holds)
   int lbm_wrows = 0;             // interior tile shape of the row kernel (0: consecutive blocks)
   size_t lbm_split_cap = 0;      // capacity of d_lbm_split (the largest shape)
@@ -117,6 +118,7 @@ struct ekpnp_ctx {
   double* d_walls = nullptr;
   double2* d_tw = nullptr;
   double2* d_spec = nullptr;
+  double2* d_spec2 = nullptr;    // every other step's spectrum (lbm_inv)
   double* d_ux_prev = nullptr;
   double* d_refs = nullptr;      // storage references in use, [ny][8] per channel
   double* d_refs_new = nullptr;  // staging for a change of reference
@@ -325,6 +327,7 @@ StepBuffers make_buffers(ekpnp_ctx* c) {
   b.walls_stride = c->total_nx;
   b.tw = c->d_tw;
   b.spec = c->d_spec;
+  b.spec_prev = c->d_spec;
   b.ux_prev = c->d_ux_prev;
   b.partials = c->d_partials;
   b.red_out = c->d_red;
@@ -368,7 +371,7 @@ void release(ekpnp_ctx* c) {
   drop_graphs(c);
   void* ptrs[] = {c->lat[0], c->lat[1], c->d_desc, c->d_lbm_tiles, c->d_fft_tiles,
                   c->d_tri_tiles, c->d_first_tile, c->d_rho_e, c->d_psi, c->d_macro,
-                  c->d_walls, c->d_tw, c->d_spec, c->d_ux_prev, c->d_partials, c->d_red,
+                  c->d_walls, c->d_tw, c->d_spec, c->d_spec2, c->d_ux_prev, c->d_partials, c->d_red,
                   c->d_refs, c->d_refs_new, c->d_row_tiles, c->d_cprime, c->d_lbm_split,
                   c->d_blocks, c->d_blocks_new, c->d_diag, c->d_lbm_fwd};
   for (void* p : ptrs)
@@ -443,6 +446,16 @@ int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2
 //   n_x = 4 x1000          2500        74.6 -> 69.6   n_x = 4 x2000     5000  141.9 -> 151.2
 //   64x128 x100 fp32       3200        60.8 -> 67.4
 constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_LONG = 10;  // the latter: FP64 storage, narrow rows only
+// and as long as it is emptier still, the inverse x-transforms of the step
+// before in the same launch (each work-group transforms a row to either side
+// as well: half as much again at 4 rows a tile, three times at one).  Step in
+// us, inverse apart -> in it:
+//   10x101 fp64     4 tiles  15.5 -> 13.5    32 channels (32, 64)  576  29.6 -> 23.4
+//   64x128 fp64    32        18.7 -> 16.3    512 channels n_x = 4 1280  38.5 -> 35.2
+//   256x256 fp32  256        21.8 -> 18.6    64x128 x48 fp32      1536  41.0 -> 38.7
+//   256x512 fp64  512        29.1 -> 25.4    256 wide x15 fp32    1440  42.4 -> 42.9
+//   256x1000 fp64 1000       37.6 -> 38.4    64x128 x32 fp64      1024  35.4 -> 36.4
+constexpr int LBM_FWD_INV_TILES_PER_CU = 5, LBM_FWD_INV_TILES_PER_CU_FP64 = 3;
 void build_lbm_fwd(ekpnp_ctx* c) {
   c->lbm_fwd.clear();
   for (auto& d : c->desc) d.lbm_span = d.nx <= LBM_WG ? LBM_WG / d.nx * d.nx : LBM_WG;
@@ -463,6 +476,8 @@ void build_lbm_fwd(ekpnp_ctx* c) {
   const bool longer = !pow2 || c->opt.precision == EKPNP_POP_FP64;
   if (c->lbm_fwd.size() > (size_t)(longer ? LBM_FWD_TILES_PER_CU_LONG : LBM_FWD_TILES_PER_CU) * c->n_cu)
     c->lbm_fwd.clear();
+  const int inv = c->opt.precision == EKPNP_POP_FP64 ? LBM_FWD_INV_TILES_PER_CU_FP64 : LBM_FWD_INV_TILES_PER_CU;
+  c->lbm_inv = !c->lbm_fwd.empty() && c->lbm_fwd.size() <= (size_t)inv * c->n_cu;
 }
 
 // a new interior tile shape for the row kernel: table, buffers, graphs
@@ -706,7 +721,7 @@ hipError_t enqueue_step(ekpnp_ctx* c, bool macro, hipEvent_t* ev = nullptr) {
   void* dst = c->lat[c->cur ^ 1];
   hipError_t e;
   if (fuse) {
-    e = launch_lbm_fwd(c->opt.precision, macro, c->sb, src, dst, c->stream);
+    e = launch_lbm_fwd(c->opt.precision, macro, false, c->sb, src, dst, c->stream);
     c->cur ^= 1;
   } else {
     e = enqueue_lbm(c, macro, !defer);
@@ -722,7 +737,25 @@ hipError_t enqueue_step(ekpnp_ctx* c, bool macro, hipEvent_t* ev = nullptr) {
   return e;
 }
 
+// n steps.  With lbm_inv a step's inverse x-transforms are the next one's
+// first work (psi goes to memory after the last step only): the
+// spectrum alternates between two buffers, because a work-group transforms the
+// rows beside its own too, whose owners may already be writing the new ones.
 hipError_t enqueue_steps(ekpnp_ctx* c, int n, bool macro_last) {
+  if (c->lbm_fuse && c->lbm_inv && !c->state_q && n > 1) {
+    StepBuffers b = c->sb;
+    for (int i = 0; i < n; ++i) {
+      hipError_t e = launch_lbm_fwd(c->opt.precision, macro_last && i == n - 1, i > 0, b, c->lat[c->cur],
+                                    c->lat[c->cur ^ 1], c->stream);
+      c->cur ^= 1;
+      if (e == hipSuccess) e = launch_poisson_tri(b, c->stream);
+      if (e == hipSuccess && i == n - 1) e = launch_poisson_inv(b, c->stream);
+      if (e != hipSuccess) return e;
+      b.spec_prev = b.spec;
+      b.spec = b.spec == c->d_spec ? c->d_spec2 : c->d_spec;
+    }
+    return hipSuccess;
+  }
   for (int i = 0; i < n; ++i) {
     hipError_t e = enqueue_step(c, macro_last && i == n - 1);
     if (e != hipSuccess) return e;
@@ -1188,6 +1221,7 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
     if ((e = dalloc(c, &c->d_walls, c->walls.size())) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_tw, tw.size())) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_spec, c->total_spec)) != hipSuccess) return e;
+    if (c->lbm_inv && (e = dalloc(c, &c->d_spec2, c->total_spec)) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_ux_prev, c->total_nodes)) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_refs, c->total_refs)) != hipSuccess) return e;
     if ((e = dalloc(c, &c->d_refs_new, c->total_refs)) != hipSuccess) return e;
@@ -1232,6 +1266,7 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
     if ((e = hipMemset(c->d_macro, 0, M_COUNT * c->total_nodes * sizeof(double))) != hipSuccess) return e;
     if ((e = hipMemset(c->d_ux_prev, 0, c->total_nodes * sizeof(double))) != hipSuccess) return e;
     if ((e = hipMemset(c->d_spec, 0, c->total_spec * sizeof(double2))) != hipSuccess) return e;
+    if (c->d_spec2 && (e = hipMemset(c->d_spec2, 0, c->total_spec * sizeof(double2))) != hipSuccess) return e;
     return hipDeviceSynchronize();
   };
   he = upload();

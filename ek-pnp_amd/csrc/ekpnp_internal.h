@@ -144,6 +144,7 @@ struct StepBuffers {
   int walls_stride;             // = total nx
   const double2* tw;            // twiddles
   double2* spec;                // spectrum [nk_stride/8][ny][8] per channel
+  const double2* spec_prev;     // the step before's spectrum (k_lbm_fwd)
   double* ux_prev;              // residual snapshot
   double* partials;             // reduction partials [n_lbm_tiles][8]
   double* red_out;              // reductions [n_channels][8]
@@ -164,7 +165,8 @@ struct StepBuffers {
 hipError_t launch_lbm_rows_interior(const StepBuffers& b, const void* src, void* dst, hipStream_t s);
 hipError_t launch_lbm(int precision, bool compute64, bool from_q, bool macro, const StepBuffers& b,
                       const void* src, void* dst, hipStream_t s, bool walls = true);
-hipError_t launch_lbm_fwd(int precision, bool macro, const StepBuffers& b, const void* src, void* dst, hipStream_t s);
+hipError_t launch_lbm_fwd(int precision, bool macro, bool inv, const StepBuffers& b, const void* src, void* dst,
+                          hipStream_t s);
 hipError_t launch_poisson_fwd(const StepBuffers& b, hipStream_t s);
 hipError_t launch_poisson_tri(const StepBuffers& b, hipStream_t s);
 // the tridiagonal plus the row kernel's wall tiles of the collide-stream that

@@ -94,17 +94,17 @@ __device__ __forceinline__ int xcd_remap(int wg, int nwg) {
 
 // ---------------------------------------------------------------------------
 // E = -grad(psi) by central differences at node (x, y); wall rows copy Ey of
-// the neighbouring row (poisson.cu:145-174).
+// the neighbouring row (poisson.cu:145-174).  ps holds psi from row row0 on.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void efield_at(const double* __restrict__ ps, int nx, int ny, int x,
                                           int xm, int xp, int y, double inv2dx, double inv2dy,
-                                          double& Ex, double& Ey) {
-  const double* row = ps + (long long)y * nx;
+                                          double& Ex, double& Ey, int row0 = 0) {
+  const double* row = ps + (long long)(y - row0) * nx;
   Ex = (row[xm] - row[xp]) * inv2dx;
   int ya = y - 1, yb = y + 1;
   if (y == 0) { ya = 0; yb = 2; }
   if (y == ny - 1) { ya = ny - 3; yb = ny - 1; }
-  Ey = (ps[(long long)ya * nx + x] - ps[(long long)yb * nx + x]) * inv2dy;
+  Ey = (ps[(long long)(ya - row0) * nx + x] - ps[(long long)(yb - row0) * nx + x]) * inv2dy;
 }
 
 // Storage references (FP32 storage; FP64 storage keeps absolute populations
@@ -442,7 +442,8 @@ __device__ __forceinline__ Moments<C> moments(const C* q, const ChanDesc* __rest
 // latency and the FP64 issue rate of a lone wave (8 clocks an instruction).
 template <typename S, typename C, bool FROM_Q, int CACHED>
 __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int node,
-                                           const S* __restrict__ src, S* __restrict__ dst, bool macro) {
+                                           const S* __restrict__ src, S* __restrict__ dst, bool macro,
+                                           const double* __restrict__ ps, int row0) {
   const int nx = cd->nx, ny = cd->ny;
   const int y = node / nx;
   const int x = node - y * nx;
@@ -450,7 +451,6 @@ __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc*
   // a channel frozen for an odd number of steps holds its state in the other lattice
   const S* __restrict__ P = (cd->swap ? dst : src) + cd->pop_off;
   S* __restrict__ Q = (cd->swap ? const_cast<S*>(src) : dst) + cd->pop_off;
-  const double* __restrict__ ps = b.psi + cd->fld_off;
   const int xm = (x == 0) ? nx - 1 : x - 1;
   const int xp = (x == nx - 1) ? 0 : x + 1;
   const bool bottom = (y == 0), top = (y == ny - 1);
@@ -480,7 +480,7 @@ __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc*
     const long long p1 = own_stride(plane);
     load_pre<S, C, FROM_Q, REF, CACHED, true>(P, p1, nx, ny, x, 1, xm, xp, r1, tc, m1);
     double Ex1, Ey1;
-    efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1);
+    efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1, row0);
     const Moments<C> mm = moments(m1, cd, X1, Ex1, Ey1);
     mux = -mm.ux;
     muy = -mm.uy;
@@ -498,7 +498,7 @@ __device__ __forceinline__ double lbm_node(const StepBuffers& b, const ChanDesc*
   }
 
   double Ex, Ey;
-  efield_at(ps, nx, ny, x, xm, xp, y, cd->inv2dx, cd->inv2dy, Ex, Ey);
+  efield_at(ps, nx, ny, x, xm, xp, y, cd->inv2dx, cd->inv2dy, Ex, Ey, row0);
   const Moments<C> m = moments(q, cd, Xo, Ex, Ey);
   C ux = m.ux, uy = m.uy;
   if (bottom) {
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm(StepBuffers b, co
   if (!cd->active) return;  // converged channel, frozen by the residual driver
   const int node = tile.y + (int)threadIdx.x;
   if (node >= cd->nx * cd->ny) return;
-  lbm_node<S, C, FROM_Q, CACHED>(b, cd, node, src, dst, MACRO);
+  lbm_node<S, C, FROM_Q, CACHED>(b, cd, node, src, dst, MACRO, b.psi + cd->fld_off, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -717,12 +717,11 @@ __device__ __forceinline__ void gather9(const float* __restrict__ B, long long p
 template <bool WALL, int CACHED>
 __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanDesc* __restrict__ cd, int y, int x,
                                              const WaveRefs& rf, const float* __restrict__ P, float* __restrict__ Q,
-                                             bool macro) {
+                                             bool macro, const double* __restrict__ ps, int row0) {
   using C = double;
   const int nx = cd->nx, ny = cd->ny;
   const long long node = (long long)y * nx + x;
   const long long plane = cd->plane;
-  const double* __restrict__ ps = b.psi + cd->fld_off;
   const double tc = cd->inv_cs2 * cd->inv_cfl;
   const int xm = (x == 0) ? nx - 1 : x - 1;
   const int xp = (x == nx - 1) ? 0 : x + 1;
@@ -756,7 +755,7 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
     dcwn = (bottom ? Wl[W_CN_LO * ws] : Wl[W_CN_HI * ws]) - Xo[2];
   }
   double Ex, Ey;
-  efield_at(ps, nx, ny, x, xm, xp, y, cd->inv2dx, cd->inv2dy, Ex, Ey);
+  efield_at(ps, nx, ny, x, xm, xp, y, cd->inv2dx, cd->inv2dy, Ex, Ey, row0);
   // y = 0: the mirror's inputs, node (x,1)'s pre-collision values and field,
   // loaded together with the node's own
   float w[27];
@@ -766,7 +765,7 @@ __device__ __forceinline__ double lbm_row_node(const StepBuffers& b, const ChanD
 #pragma unroll
     for (int s = 0; s < 3; ++s)
       gather9<0, 0>(P + (long long)(9 * s) * plane, plane, rm, r0, rp, x, xm, xp, w + 9 * s);
-    efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1);
+    efield_at(ps, nx, ny, x, xm, xp, 1, cd->inv2dx, cd->inv2dy, Ex1, Ey1, row0);
   }
   // every load is in flight before the first use: keep the scheduler from
   // interleaving the species' loads with the arithmetic
@@ -923,7 +922,7 @@ __device__ __forceinline__ void lbm_rows_tile(const StepBuffers& b, int2 tile, c
   const float* __restrict__ P = (cd->swap ? dst : src) + cd->pop_off;
   float* __restrict__ Q = (cd->swap ? const_cast<float*>(src) : dst) + cd->pop_off;
   const WaveRefs rf = wave_refs(b, cd, y, k, (int)threadIdx.x & 63);
-  lbm_row_node<WALL, CACHED>(b, cd, y, x, rf, P, Q, macro);
+  lbm_row_node<WALL, CACHED>(b, cd, y, x, rf, P, Q, macro, b.psi + cd->fld_off, 0);
 }
 
 template <bool WALL, int CACHED>
@@ -1490,13 +1489,15 @@ __device__ __forceinline__ double sub_pinned(double a, double b) {
 // launch and one read of the charge density less, where a step is a chain of
 // launches of a few us each: an empty one takes 1.6 us in a graph, and each
 // begins by fetching descriptors, tables and rows that the one before has just
-// written.  64x128 with FP64 storage: 21.7 -> 18.7 us a step.  Bound: latency,
-// of the gather, of a lone wave's FP64 instructions, of the transform's passes.
-// The transforms are k_fft_fwd_p's and the narrow rows' of k_fft_fwd, operation
+// written.  64x128 with FP64 storage: 21.7 -> 18.7 us a step, with INV (below)
+// 16.3.  Bound: latency, of the gather, of a lone wave's FP64 instructions, of
+// the transforms' passes.  The transforms are k_fft_fwd_p's and the narrow rows' of k_fft_fwd, operation
 // for operation.
 // ---------------------------------------------------------------------------
 constexpr int FUSE_ROWS = LBM_WG / 2 + 64;  // double2 of LDS rows (narrow: row stride nx | 1)
 constexpr int FUSE_TW = LBM_WG / 4;         // twiddles: a quadrant of at most LBM_WG nodes, or a narrow row's
+// with one row to either side: at most three of LBM_WG / 2 values (n_x = LBM_WG)
+constexpr int FUSE_INV = 3 * LBM_WG / 2;
 
 __device__ __forceinline__ void fused_fwd(const StepBuffers& b, const ChanDesc* __restrict__ cd, int node0, double rho_e,
                                           double2* lds, const double2* twl) {
@@ -1547,17 +1548,97 @@ __device__ __forceinline__ void fused_fwd(const StepBuffers& b, const ChanDesc* 
   }
 }
 
-template <typename S, int KIND, int CACHED>
+// psi of the rows a tile's node updates read, rows row0 .. row0 + rows - 1, from
+// the spectrum of the step before: the tile's own rows and one more to either
+// side (k_fft_inv_p's and the narrow rows' k_fft_inv, operation for operation)
+__device__ __forceinline__ void fused_inv(const StepBuffers& b, const ChanDesc* __restrict__ cd, int row0, int rows,
+                                          double2* lds, const double2* twl, double* psl) {
+  const int nx = cd->nx, nk = cd->nk, ny = cd->ny, tid = threadIdx.x;
+  const double2* __restrict__ spec = b.spec_prev + cd->spec_off;
+  if (cd->pow2) {
+    const int N = nx >> 1, lgN = ilog2(N), lgnx = lgN + 1, quarter = nx >> 2, half = N >> 1;
+    const int p = tid / rows, r = tid - p * rows;
+    if (p <= half) {
+      const int y = min(max(row0 + r, 1), ny - 2);  // wall rows are replaced below
+      const double2 xa = spec[spec_idx(ny, y, p)], xb = spec[spec_idx(ny, y, N - p)];
+      const int rb = r << lgN;
+      {
+        const double2 xk = xa, xc = cconj(xb);
+        const double2 E = make_double2(0.5 * (xk.x + xc.x), 0.5 * (xk.y + xc.y));
+        const double2 O = cmul(make_double2(0.5 * (xk.x - xc.x), 0.5 * (xk.y - xc.y)),
+                               cconj(tw_half(twl, p, quarter)));
+        lds[sw(rb + p)] = make_double2(E.x - O.y, E.y + O.x);
+      }
+      if (p > 0 && p < half) {
+        const double2 xk = xb, xc = cconj(xa);
+        const double2 E = make_double2(0.5 * (xk.x + xc.x), 0.5 * (xk.y + xc.y));
+        const double2 O = cmul(make_double2(0.5 * (xk.x - xc.x), 0.5 * (xk.y - xc.y)),
+                               cconj(tw_half(twl, N - p, quarter)));
+        lds[sw(rb + N - p)] = make_double2(E.x - O.y, E.y + O.x);
+      }
+    }
+    __syncthreads();
+    stockham<+1, LBM_WG, 16, false, FUSE_INV>(lds, rows, N, lgN, twl, lgnx);
+    const double invN = 1.0 / (double)N;
+    for (int e = tid; e < rows * N; e += LBM_WG) {
+      const double2 z = lds[sw(e)];
+      psl[2 * e] = z.x * invN;
+      psl[2 * e + 1] = z.y * invN;
+    }
+  } else {
+    for (int e = tid; e < rows * nk; e += LBM_WG) {
+      const int r = e / nk, k = e - r * nk;
+      lds[e] = spec[spec_idx(ny, min(max(row0 + r, 1), ny - 2), k)];
+    }
+    __syncthreads();
+    const int kmax = (nx - 1) / 2;  // modes counted twice
+    const bool nyq = (nx & 1) == 0;
+    for (int e = tid; e < rows * nx; e += LBM_WG) {
+      const int r = e / nx, n = e - r * nx;
+      const double2* z = lds + r * nk;
+      double acc = z[0].x;
+      int idx = 0;
+      for (int k = 1; k <= kmax; ++k) {
+        idx += n;
+        if (idx >= nx) idx -= nx;
+        const double2 w = twl[idx];
+        acc += 2.0 * (z[k].x * w.x + z[k].y * w.y);
+      }
+      if (nyq) acc += (n & 1) ? -z[nx / 2].x : z[nx / 2].x;
+      psl[e] = acc / (double)nx;
+    }
+  }
+  __syncthreads();
+  const double* __restrict__ Wl = b.walls + cd->wall_off;
+  const long long ws = b.walls_stride;
+  if (row0 == 0 && tid < nx) psl[tid] = Wl[W_PSI_LO * ws + tid];
+  if (row0 + rows == ny && tid < nx) psl[(rows - 1) * nx + tid] = Wl[W_PSI_HI * ws + tid];
+  __syncthreads();
+}
+
+// INV: psi comes from the step before's spectrum (spec_prev, which the forward
+// transforms of other work-groups do not write) instead of from memory
+template <typename S, int KIND, int CACHED, bool INV>
 __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm_fwd(StepBuffers b, const int2* __restrict__ tiles,
                                                                    const S* __restrict__ src, S* __restrict__ dst,
                                                                    int macro) {
-  __shared__ double2 lds[FUSE_ROWS];
+  __shared__ double2 lds[INV ? FUSE_INV : FUSE_ROWS];
   __shared__ double2 twl[FUSE_TW];
+  __shared__ double psl[INV ? 2 * FUSE_INV : 1];
   const int2 tile = tiles[xcd_remap(blockIdx.x, gridDim.x)];
   const ChanDesc* __restrict__ cd = b.chans + tile.x;
   if (!cd->active) return;  // converged channel, frozen by the residual driver
   const int nx = cd->nx, ny = cd->ny, tid = threadIdx.x;
   if (tid < (cd->pow2 ? nx >> 2 : nx)) twl[tid] = b.tw[cd->tw_off + tid];
+  const double* ps = b.psi + cd->fld_off;
+  int row0 = 0;
+  if (INV) {
+    const int rows = min(cd->lbm_span / nx + 2, ny);
+    row0 = max(0, min(tile.y / nx - 1, ny - rows));
+    __syncthreads();  // the twiddles
+    fused_inv(b, cd, row0, rows, lds, twl, psl);
+    ps = psl;
+  }
   double rho_e = 0.0;
   const bool general = KIND == FWD_GENERAL || (KIND == FWD_MIXED && (nx & 63) != 0);
   if constexpr (KIND != FWD_GENERAL) {
@@ -1568,14 +1649,14 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm_fwd(StepBuffers b
       const float* __restrict__ P = (cd->swap ? dst : src) + cd->pop_off;
       float* __restrict__ Q = (cd->swap ? const_cast<float*>(src) : dst) + cd->pop_off;
       const WaveRefs rf = wave_refs(b, cd, y, x0 >> 6, tid & 63);
-      if (y == 0 || y == ny - 1) rho_e = lbm_row_node<true, 0>(b, cd, y, x, rf, P, Q, macro != 0);
-      else rho_e = lbm_row_node<false, 0>(b, cd, y, x, rf, P, Q, macro != 0);
+      if (y == 0 || y == ny - 1) rho_e = lbm_row_node<true, 0>(b, cd, y, x, rf, P, Q, macro != 0, ps, row0);
+      else rho_e = lbm_row_node<false, 0>(b, cd, y, x, rf, P, Q, macro != 0, ps, row0);
     }
   }
   if constexpr (KIND != FWD_ROWS) {
     const int node = tile.y + tid;
     if (general && tid < cd->lbm_span && node < nx * ny)
-      rho_e = lbm_node<S, double, false, CACHED>(b, cd, node, src, dst, macro != 0);
+      rho_e = lbm_node<S, double, false, CACHED>(b, cd, node, src, dst, macro != 0, ps, row0);
   }
   fused_fwd(b, cd, tile.y, rho_e, lds, twl);
 }
@@ -3105,26 +3186,34 @@ static hipError_t lbm_dispatch(bool from_q, bool macro, bool walls, const StepBu
 }
 
 // the coupled step's collide-stream and forward x-transforms in one launch
-// (FP64 arithmetic, populations not in pre-collision form)
-hipError_t launch_lbm_fwd(int precision, bool macro, const StepBuffers& b, const void* src, void* dst, hipStream_t s) {
+// (FP64 arithmetic, populations not in pre-collision form); inv: psi by the
+// inverse transforms of spec_prev, in the same launch
+hipError_t launch_lbm_fwd(int precision, bool macro, bool inv, const StepBuffers& b, const void* src, void* dst,
+                          hipStream_t s) {
   const dim3 grid(b.n_lbm_fwd_tiles), block(LBM_WG);
-  const int m = macro ? 1 : 0;
+  const auto launch = [&](auto* sp, auto* dp, auto kind, auto cached) {
+    using S = std::remove_pointer_t<decltype(dp)>;
+    if (inv)
+      hipLaunchKernelGGL((k_lbm_fwd<S, kind(), cached(), true>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, macro ? 1 : 0);
+    else
+      hipLaunchKernelGGL((k_lbm_fwd<S, kind(), cached(), false>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, macro ? 1 : 0);
+  };
+  const std::integral_constant<int, FWD_GENERAL> general{};
+  const std::integral_constant<int, FWD_ROWS> rows{};
+  const std::integral_constant<int, FWD_MIXED> mixed{};
+  const std::integral_constant<int, 0> none{};
+  const std::integral_constant<int, 27> all{};
   if (precision == 0) {
     const float* sp = static_cast<const float*>(src);
     float* dp = static_cast<float*>(dst);
-    if (b.lbm_fwd_kind == FWD_ROWS)
-      hipLaunchKernelGGL((k_lbm_fwd<float, FWD_ROWS, 0>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
-    else if (b.lbm_fwd_kind == FWD_MIXED)
-      hipLaunchKernelGGL((k_lbm_fwd<float, FWD_MIXED, 27>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
-    else
-      hipLaunchKernelGGL((k_lbm_fwd<float, FWD_GENERAL, 27>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
+    if (b.lbm_fwd_kind == FWD_ROWS) launch(sp, dp, rows, none);
+    else if (b.lbm_fwd_kind == FWD_MIXED) launch(sp, dp, mixed, all);
+    else launch(sp, dp, general, all);
   } else {
     const double* sp = static_cast<const double*>(src);
     double* dp = static_cast<double*>(dst);
-    if (b.lbm_cached == LBM_CACHED_ALL)
-      hipLaunchKernelGGL((k_lbm_fwd<double, FWD_GENERAL, 27>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
-    else
-      hipLaunchKernelGGL((k_lbm_fwd<double, FWD_GENERAL, 0>), grid, block, 0, s, b, b.lbm_fwd_tiles, sp, dp, m);
+    if (b.lbm_cached == LBM_CACHED_ALL) launch(sp, dp, general, all);
+    else launch(sp, dp, general, none);
   }
   return hipGetLastError();
 }

@@ -1,5 +1,5 @@
-"""Collide-stream and forward x-transform in one launch (small contexts of
-narrow rows): the coupled step against the same step in a context that one
+"""Collide-stream and forward x-transform, and the inverse one of the step
+before, in one launch (small contexts of narrow rows): the coupled step against the same step in a context that one
 wide channel more keeps on the separate launches, and on both sides of the
 size limit.  The same bits."""
 import numpy as np
@@ -12,9 +12,9 @@ pytestmark = pytest.mark.gpu
 FIELDS = ("rho", "ux", "uy", "cpos", "cneg", "psi")
 
 
-def start(sizes, precision):
+def start(sizes, precision, **kw):
     s = ekpnp.Solver([ekpnp.lattice_params(nx, ny, kappa_h=min(4.0, 0.15 * ny)) for nx, ny in sizes],
-                     precision=precision)
+                     precision=precision, **kw)
     for ch, (nx, ny) in enumerate(sizes):
         rng = np.random.default_rng(100 * nx + ny)
         zw = -1 + 0.3 * rng.standard_normal(nx)
@@ -56,9 +56,21 @@ def test_step_equals_the_separate_launches(sizes, precision):
     assert np.array_equal(a.reductions(), b.reductions()[:-1])
 
 
-# one tile per row: at and just past the limit of a card with 256 CUs
+def test_replayed_and_enqueued_steps_are_the_same():
+    sizes = [(64, 40), (10, 33), (32, 20)]
+    a, b = start(sizes, "fp32"), start(sizes, "fp32", use_graph=False)
+    for n in (7, 1, 2, 70):  # the spectrum's two buffers in every order
+        a.step(n)
+        b.step(n)
+    for ch in range(len(sizes)):
+        same(state(a, ch), state(b, ch), sizes[ch])
+
+
+# one tile per row: at and just past the limits of a card with 256 CUs, of the
+# forward transforms in the launch and of the inverse ones
 @pytest.mark.parametrize("nx,ny,precision,copies", [(256, 6, "fp32", (256, 257)), (256, 10, "fp64", (256, 257)),
-                                                    (4, 64, "fp32", (2560, 2561))])
+                                                    (4, 64, "fp32", (2560, 2561)), (256, 5, "fp32", (256, 257)),
+                                                    (256, 6, "fp64", (128, 129)), (4, 64, "fp32", (1280, 1281))])
 def test_both_sides_of_the_limit(nx, ny, precision, copies):
     got = []
     for n in copies:
