@@ -446,16 +446,17 @@ int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2
 //   n_x = 4 x1000          2500        74.6 -> 69.6   n_x = 4 x2000     5000  141.9 -> 151.2
 //   64x128 x100 fp32       3200        60.8 -> 67.4
 constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_LONG = 10;  // the latter: FP64 storage, narrow rows only
-// and as long as it is emptier still, the inverse x-transforms of the step
-// before in the same launch (each work-group transforms a row to either side
-// as well: half as much again at 4 rows a tile, three times at one).  Step in
-// us, inverse apart -> in it:
+// The inverse x-transforms of the step before are in that launch too, with FP64
+// storage while it is emptier still (each work-group transforms a row to either
+// side as well: half as much again at 4 rows a tile, three times at one).  Step
+// in us, inverse apart -> in it:
 //   10x101 fp64     4 tiles  15.5 -> 13.5    32 channels (32, 64)  576  29.6 -> 23.4
-//   64x128 fp64    32        18.7 -> 16.3    512 channels n_x = 4 1280  38.5 -> 35.2
+//   64x128 fp64    32        18.7 -> 16.3    n_x = 4 x512 fp32    1280  38.7 -> 35.2
 //   256x256 fp32  256        21.8 -> 18.6    64x128 x48 fp32      1536  41.0 -> 38.7
 //   256x512 fp64  512        29.1 -> 25.4    256 wide x15 fp32    1440  42.4 -> 42.9
-//   256x1000 fp64 1000       37.6 -> 38.4    64x128 x32 fp64      1024  35.4 -> 36.4
-constexpr int LBM_FWD_INV_TILES_PER_CU = 5, LBM_FWD_INV_TILES_PER_CU_FP64 = 3;
+//   256x1000 fp64 1000       37.6 -> 38.4    n_x = 4 x900 fp32    2250  56.2 -> 54.6
+//   64x128 x32 fp64 1024     35.4 -> 36.4
+constexpr int LBM_FWD_INV_TILES_PER_CU_FP64 = 3;
 void build_lbm_fwd(ekpnp_ctx* c) {
   c->lbm_fwd.clear();
   for (auto& d : c->desc) d.lbm_span = d.nx <= LBM_WG ? LBM_WG / d.nx * d.nx : LBM_WG;
@@ -476,8 +477,8 @@ void build_lbm_fwd(ekpnp_ctx* c) {
   const bool longer = !pow2 || c->opt.precision == EKPNP_POP_FP64;
   if (c->lbm_fwd.size() > (size_t)(longer ? LBM_FWD_TILES_PER_CU_LONG : LBM_FWD_TILES_PER_CU) * c->n_cu)
     c->lbm_fwd.clear();
-  const int inv = c->opt.precision == EKPNP_POP_FP64 ? LBM_FWD_INV_TILES_PER_CU_FP64 : LBM_FWD_INV_TILES_PER_CU;
-  c->lbm_inv = !c->lbm_fwd.empty() && c->lbm_fwd.size() <= (size_t)inv * c->n_cu;
+  c->lbm_inv = !c->lbm_fwd.empty() && (c->opt.precision == EKPNP_POP_FP32 ||
+                                       c->lbm_fwd.size() <= (size_t)LBM_FWD_INV_TILES_PER_CU_FP64 * c->n_cu);
 }
 
 // a new interior tile shape for the row kernel: table, buffers, graphs
