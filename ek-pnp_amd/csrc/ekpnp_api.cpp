@@ -433,19 +433,20 @@ int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2
 // Tiles of k_lbm_fwd: contexts of FP64 arithmetic whose every channel has rows
 // of at most LBM_WG nodes, of a power of two or of the narrow rows' direct DFT,
 // as long as the chip is not full: the transform holds every work-group for
-// some us longer, which is less than the launch it saves only while there are
-// few work-groups a CU (n_cu = 256).  Step in us, launches apart -> one launch:
-//   10x101 fp64               4 tiles  18.4 -> 15.6
-//   64x128 fp64              32        21.7 -> 18.7
-//   256x256 fp32            256        26.0 -> 23.4
-//   32 channels (32, 64)    576        35.2 -> 31.9
-//   64x128 x25 fp32         800        33.0 -> 31.4
-//   512 channels n_x = 4   1280        47.0 -> 45.0
-//   64x128 x50 fp32        1600        43.7 -> 42.9   n_x = 32 x150  1950  44.1 -> 45.3
-//   64x128 x64 fp64        2048        57.8 -> 54.9   64x128 x200 fp64  6400  150.4 -> 154.9
-//   n_x = 4 x1000          2500        74.6 -> 69.6   n_x = 4 x2000     5000  141.9 -> 151.2
-//   64x128 x100 fp32       3200        60.8 -> 67.4
-constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_LONG = 10;  // the latter: FP64 storage, narrow rows only
+// some us longer, which is less than the launches it saves only while there are
+// few work-groups a CU (n_cu = 256).  Step in us, launches apart -> this one,
+// with the inverse transforms where the rule below puts them in:
+//   10x101 fp64              4 tiles  18.4 -> 13.5
+//   64x128 fp64             32        21.7 -> 16.3
+//   256x256 fp32           256        26.0 -> 18.6
+//   32 channels (32, 64)   576        35.2 -> 23.4
+//   64x128 x48 fp32       1536        41.5 -> 38.7    64x128 x56 fp32  1792  44.0 -> 44.7
+//   64x128 x40 fp64       1280        42.7 -> 40.4    64x128 x64 fp64  2048  56.4 -> 58.7
+//   32 wide x90           1010        34.3 -> 32.9    32 wide x120     1440  38.6 -> 39.6
+// and with rows below 24 nodes, FP32 storage:
+//   n_x = 4 x1100         2750        70.4 -> 63.1    n_x = 4 x1300    3250  89.3 -> 89.4
+//   n_x = 8 x450          2800        51.4 -> 50.6    12, 20 x400      4000  99.5 -> 100.6
+constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_NARROW = 12;
 // The inverse x-transforms of the step before are in that launch too, with FP64
 // storage while it is emptier still (each work-group transforms a row to either
 // side as well: half as much again at 4 rows a tile, three times at one).  Step
@@ -472,10 +473,9 @@ void build_lbm_fwd(ekpnp_ctx* c) {
     for (int n = 0; n < d.nx * d.ny; n += d.lbm_span) c->lbm_fwd.push_back(make_int2(i, n));
   }
   c->lbm_fwd_kind = n_rows == 0 ? FWD_GENERAL : n_rows == c->nchan ? FWD_ROWS : FWD_MIXED;
-  bool pow2 = false;
-  for (const auto& d : c->desc) pow2 = pow2 || d.pow2;
-  const bool longer = !pow2 || c->opt.precision == EKPNP_POP_FP64;
-  if (c->lbm_fwd.size() > (size_t)(longer ? LBM_FWD_TILES_PER_CU_LONG : LBM_FWD_TILES_PER_CU) * c->n_cu)
+  bool narrow = c->opt.precision == EKPNP_POP_FP32;
+  for (const auto& d : c->desc) narrow = narrow && d.nx < DFT_MIN_NX;
+  if (c->lbm_fwd.size() > (size_t)(narrow ? LBM_FWD_TILES_PER_CU_NARROW : LBM_FWD_TILES_PER_CU) * c->n_cu)
     c->lbm_fwd.clear();
   c->lbm_inv = !c->lbm_fwd.empty() && (c->opt.precision == EKPNP_POP_FP32 ||
                                        c->lbm_fwd.size() <= (size_t)LBM_FWD_INV_TILES_PER_CU_FP64 * c->n_cu);

@@ -68,8 +68,8 @@ def test_replayed_and_enqueued_steps_are_the_same():
 
 # one tile per row: at and just past the limits of a card with 256 CUs, of the
 # forward transforms in the launch and of the inverse ones
-@pytest.mark.parametrize("nx,ny,precision,copies", [(256, 6, "fp32", (256, 257)), (256, 10, "fp64", (256, 257)),
-                                                    (4, 64, "fp32", (2560, 2561)), (256, 6, "fp64", (128, 129))])
+@pytest.mark.parametrize("nx,ny,precision,copies", [(256, 6, "fp32", (256, 257)), (256, 6, "fp64", (256, 257)),
+                                                    (4, 64, "fp32", (3072, 3073)), (256, 6, "fp64", (128, 129))])
 def test_both_sides_of_the_limit(nx, ny, precision, copies):
     got = []
     for n in copies:
