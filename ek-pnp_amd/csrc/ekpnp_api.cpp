@@ -620,7 +620,7 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
   c->sb.tri_lmax = tri_lmax;
   // the persistent kernels take tiles of <= FFT_PERSIST_ELEMS values and keep
   // twiddles in LDS
-  bool persist_ok = fft_persist == 1 && fft_elems <= FFT_PERSIST_ELEMS && FFT_LDS_PERSIST <= (unsigned)c->max_lds;
+  bool persist_ok = fft_persist == 1 && fft_elems <= FFT_PERSIST_ELEMS && fft_lds_persist(FFT_PF) <= (unsigned)c->max_lds;
   for (const auto& d : c->desc) {
     if (!d.pow2) continue;
     const int N = d.nx / 2;
@@ -629,7 +629,11 @@ hipError_t build_poisson_plan(ekpnp_ctx* c, int fft_elems, int tri_rows, int fft
     if (N * d.fft_rows > FFT_PERSIST_ELEMS || d.fft_rows > FFT_MAX_ROWS) persist_ok = false;
   }
   c->sb.fft_persist = persist_ok ? 1 : 0;
-  c->sb.fft_grid = std::max(1, std::min(n_fft_pow2, 2 * c->n_cu));
+  int max_tile = 0;
+  for (const auto& d : c->desc)
+    if (d.pow2) max_tile = std::max(max_tile, d.nx / 2 * d.fft_rows);
+  c->sb.fft_pf = max_tile <= 4 * FFT_WG ? 4 : FFT_PF;
+  c->sb.fft_grid = std::max(1, std::min(n_fft_pow2, (c->sb.fft_pf == 4 ? 3 : 2) * c->n_cu));
   // row-pair kernels: every power-of-two channel of one width nx = 2 N with
   // N = S * FFT_WG_ROWS, S in {2, 4}, two rows per tile (fft_elems = 2 N),
   // rows and twiddles in LDS

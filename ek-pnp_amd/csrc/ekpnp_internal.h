@@ -36,10 +36,10 @@ constexpr int FFT_MAX_ROWS = 256;  // rows per power-of-two FFT tile
 // spectrum pairs (X[p], X[N-p]) per lane: rows (N/2 + 1) <= FFT_MAX_ELEMS/2 + FFT_MAX_ROWS
 constexpr int FFT_PAIR_SLOTS = (FFT_MAX_ELEMS / 2 + FFT_MAX_ROWS + FFT_WG_ROWS - 1) / FFT_WG_ROWS;
 // persistent pipelined x-FFT: tiles of <= FFT_PERSIST_ELEMS complex values,
-// 8 prefetched per lane; LDS = rows + quadrant twiddles (nx <= 2 FFT_PERSIST_ELEMS)
+// up to 8 prefetched per lane; LDS = rows + quadrant twiddles (N / 2 <= elements / 2)
 constexpr int FFT_PF = 8;
 constexpr int FFT_PERSIST_ELEMS = FFT_PF * FFT_WG;  // 2048
-constexpr unsigned FFT_LDS_PERSIST = (FFT_PERSIST_ELEMS + FFT_PERSIST_ELEMS / 2) * 16;
+constexpr unsigned fft_lds_persist(int pf) { return (unsigned)(pf * FFT_WG + pf * FFT_WG / 2) * 16; }
 constexpr int TRI_WG = 256;       // lanes of a tridiagonal work-group (modes x chunks)
 constexpr int MAX_NX = 8192;      // LDS-resident x-rows (64 KiB of complex FP64)
 constexpr int MAX_NX_DFT = 2048;  // non-power-of-two rows use a direct DFT
@@ -126,7 +126,7 @@ struct StepBuffers {
   int fft_pair_s;               // > 0: by the row-pair kernels, N = fft_pair_s * FFT_WG_ROWS for every one
                                 //   (2, 4: two row buffers and the quadrant table; FFT_PAIR_WIDE_S: one row
                                 //   buffer, the second row in registers, the two-level table)
-  int fft_grid;                 // work-groups of the persistent kernels
+  int fft_grid, fft_pf;         // persistent kernels: work-groups, values prefetched per lane (4, FFT_PF)
   unsigned fft_lds_pow2;        // dynamic LDS bytes of the Stockham kernels
   int n_fft_dft;                // then come the tiles of the matrix-core direct DFT, then the narrow rows'
   unsigned dft_lds;             // dynamic LDS bytes of the matrix-core direct-DFT kernels

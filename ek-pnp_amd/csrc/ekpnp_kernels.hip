@@ -1670,25 +1670,30 @@ __global__ __launch_bounds__(LBM_WG) LBM_WAVES_ATTR void k_lbm_fwd(StepBuffers b
 // LDS only).  Tiles hold rows * N <= FFT_PERSIST_ELEMS complex values.  The
 // quadrant twiddle table is (re)loaded into LDS when the channel changes.
 // ---------------------------------------------------------------------------
+// PF: values prefetched per lane, tiles of up to PF FFT_WG values: 4 where every
+// tile fits, so that three work-groups share a CU (8: two).  The 256-channel
+// sweep's transforms, bound by the loads in flight: 92 + 108 -> 73 + 84 us.
 static_assert(FFT_PF * FFT_WG == FFT_PERSIST_ELEMS, "persistent FFT tile size");
-constexpr int FFT_PF_PAIRS = (FFT_PERSIST_ELEMS / 2 + FFT_MAX_ROWS) / FFT_WG;  // spectrum pairs per lane
+constexpr int fft_pf_pairs(int pf) { return (pf * FFT_WG / 2 + FFT_MAX_ROWS) / FFT_WG; }  // spectrum pairs per lane
 
+template <int PF>
 __device__ __forceinline__ void fwd_prefetch(const StepBuffers& b, const int4* __restrict__ tiles,
-                                             const ChanDesc* __restrict__ chans, int t, double2 (&pf)[FFT_PF]) {
+                                             const ChanDesc* __restrict__ chans, int t, double2 (&pf)[PF]) {
   const int4 tt = tiles[t];
   const ChanDesc* __restrict__ cd = chans + tt.x;
   const int nx = cd->nx, total = tt.z * (nx >> 1);
   const double2* __restrict__ src = reinterpret_cast<const double2*>(b.rho_e + cd->fld_off + (long long)tt.y * nx);
 #pragma unroll
-  for (int c = 0; c < FFT_PF; ++c) pf[c] = src[min((int)threadIdx.x + c * FFT_WG, total - 1)];
+  for (int c = 0; c < PF; ++c) pf[c] = src[min((int)threadIdx.x + c * FFT_WG, total - 1)];
 }
 
-__global__ __launch_bounds__(FFT_WG, 2) void k_fft_fwd_p(StepBuffers b, const int4* __restrict__ tiles,
+template <int PF>
+__global__ __launch_bounds__(FFT_WG, PF == 4 ? 3 : 2) void k_fft_fwd_p(StepBuffers b, const int4* __restrict__ tiles,
                                                       const ChanDesc* __restrict__ chans, int n_tiles) {
   extern __shared__ double2 lds[];
-  double2* twl = lds + FFT_PERSIST_ELEMS;  // quadrant twiddle table after the rows
+  double2* twl = lds + PF * FFT_WG;  // quadrant twiddle table after the rows
   int tw_chan = -1;
-  double2 pf[FFT_PF];
+  double2 pf[PF];
   if ((int)blockIdx.x < n_tiles) fwd_prefetch(b, tiles, chans, blockIdx.x, pf);
   for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
     const int4 tt = tiles[t];
@@ -1711,7 +1716,7 @@ __global__ __launch_bounds__(FFT_WG, 2) void k_fft_fwd_p(StepBuffers b, const in
       const double* __restrict__ Wl = b.walls + cd->wall_off;
       const long long ws = b.walls_stride;
 #pragma unroll
-      for (int c = 0; c < FFT_PF; ++c) {
+      for (int c = 0; c < PF; ++c) {
         const int e = threadIdx.x + c * FFT_WG;
         if (e < total) {
           double v0 = -pc * pf[c].x, v1 = -pc * pf[c].y;
@@ -1732,7 +1737,7 @@ __global__ __launch_bounds__(FFT_WG, 2) void k_fft_fwd_p(StepBuffers b, const in
     if (t + (int)gridDim.x < n_tiles) fwd_prefetch(b, tiles, chans, t + gridDim.x, pf);
     if (active) {
       __syncthreads();
-      stockham<-1, FFT_WG, 16>(lds, rows, N, lgN, twl, lgnx);
+      stockham<-1, FFT_WG, 16, false, PF * FFT_WG>(lds, rows, N, lgN, twl, lgnx);
       double2* __restrict__ spec = b.spec + cd->spec_off;
       const float inv_rows = 1.0f / (float)rows;
       for (int e = threadIdx.x; e < rows * (N + 1); e += FFT_WG) {
@@ -1750,9 +1755,10 @@ __global__ __launch_bounds__(FFT_WG, 2) void k_fft_fwd_p(StepBuffers b, const in
 }
 
 // spectrum pairs (X[p], X[N-p]) of tile t, p = e / rows, r = e - p rows
+template <int PAIRS>
 __device__ __forceinline__ void inv_prefetch(const StepBuffers& b, const int4* __restrict__ tiles,
                                              const ChanDesc* __restrict__ chans, int t,
-                                             double2 (&xa)[FFT_PF_PAIRS], double2 (&xb)[FFT_PF_PAIRS]) {
+                                             double2 (&xa)[PAIRS], double2 (&xb)[PAIRS]) {
   const int4 tt = tiles[t];
   const ChanDesc* __restrict__ cd = chans + tt.x;
   const int N = cd->nx >> 1, rows = tt.z, ny = cd->ny;
@@ -1760,7 +1766,7 @@ __device__ __forceinline__ void inv_prefetch(const StepBuffers& b, const int4* _
   const float inv_rows = 1.0f / (float)rows;
   const double2* __restrict__ spec = b.spec + cd->spec_off;
 #pragma unroll
-  for (int c = 0; c < FFT_PF_PAIRS; ++c) {
+  for (int c = 0; c < PAIRS; ++c) {
     const int e = min((int)threadIdx.x + c * FFT_WG, npair - 1);
     const int p = div_rows(e, inv_rows), r = e - p * rows;
     xa[c] = spec[spec_idx(ny, tt.y + r, p)];
@@ -1768,12 +1774,14 @@ __device__ __forceinline__ void inv_prefetch(const StepBuffers& b, const int4* _
   }
 }
 
-__global__ __launch_bounds__(FFT_WG, 2) void k_fft_inv_p(StepBuffers b, const int4* __restrict__ tiles,
+template <int PF>
+__global__ __launch_bounds__(FFT_WG, PF == 4 ? 3 : 2) void k_fft_inv_p(StepBuffers b, const int4* __restrict__ tiles,
                                                       const ChanDesc* __restrict__ chans, int n_tiles) {
   extern __shared__ double2 lds[];
-  double2* twl = lds + FFT_PERSIST_ELEMS;  // quadrant twiddle table after the rows
+  double2* twl = lds + PF * FFT_WG;  // quadrant twiddle table after the rows
   int tw_chan = -1;
-  double2 xa[FFT_PF_PAIRS], xb[FFT_PF_PAIRS];
+  constexpr int PAIRS = fft_pf_pairs(PF);
+  double2 xa[PAIRS], xb[PAIRS];
   if ((int)blockIdx.x < n_tiles) inv_prefetch(b, tiles, chans, blockIdx.x, xa, xb);
   for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
     const int4 tt = tiles[t];
@@ -1794,7 +1802,7 @@ __global__ __launch_bounds__(FFT_WG, 2) void k_fft_inv_p(StepBuffers b, const in
       // O = (X[k] - conj X[N-k]) / 2 * conj W^k, for k = p and k = N - p
       const float inv_rows = 1.0f / (float)rows;
 #pragma unroll
-      for (int c = 0; c < FFT_PF_PAIRS; ++c) {
+      for (int c = 0; c < PAIRS; ++c) {
         const int e = threadIdx.x + c * FFT_WG;
         if (e < npair) {
           const int p = div_rows(e, inv_rows), r = e - p * rows;
@@ -1819,7 +1827,7 @@ __global__ __launch_bounds__(FFT_WG, 2) void k_fft_inv_p(StepBuffers b, const in
     if (t + (int)gridDim.x < n_tiles) inv_prefetch(b, tiles, chans, t + gridDim.x, xa, xb);
     if (active) {
       __syncthreads();
-      stockham<+1, FFT_WG, 16>(lds, rows, N, lgN, twl, lgnx);
+      stockham<+1, FFT_WG, 16, false, PF * FFT_WG>(lds, rows, N, lgN, twl, lgnx);
       double* __restrict__ ps = b.psi + cd->fld_off;
       const double invN = 1.0 / (double)N;
       double2* __restrict__ dst = reinterpret_cast<double2*>(ps + (long long)y0 * nx);
@@ -3245,8 +3253,12 @@ hipError_t launch_poisson_fwd(const StepBuffers& b, hipStream_t s) {
       hipLaunchKernelGGL(k_fft_fwd2w<FFT_PAIR_WIDE_S>, grid, block, b.fft_lds_pow2, s, b, b.fft_tiles, b.chans);
     else return hipErrorInvalidValue;
   } else if (b.n_fft_pow2 > 0 && b.fft_persist) {
-    hipLaunchKernelGGL(k_fft_fwd_p, dim3(b.fft_grid), dim3(FFT_WG), FFT_LDS_PERSIST, s, b, b.fft_tiles, b.chans,
-                       b.n_fft_pow2);
+    if (b.fft_pf == 4)
+      hipLaunchKernelGGL(k_fft_fwd_p<4>, dim3(b.fft_grid), dim3(FFT_WG), fft_lds_persist(4), s, b, b.fft_tiles, b.chans,
+                         b.n_fft_pow2);
+    else
+      hipLaunchKernelGGL(k_fft_fwd_p<FFT_PF>, dim3(b.fft_grid), dim3(FFT_WG), fft_lds_persist(FFT_PF), s, b, b.fft_tiles,
+                         b.chans, b.n_fft_pow2);
   } else if (b.n_fft_pow2 > 0) {
     if (b.fft_tw_lds)
       hipLaunchKernelGGL((k_fft_fwd<true, true>), dim3(b.n_fft_pow2), dim3(FFT_WG_ROWS), b.fft_lds_pow2, s, b, b.fft_tiles, b.chans, 0);
@@ -3286,8 +3298,12 @@ hipError_t launch_poisson_inv(const StepBuffers& b, hipStream_t s) {
       hipLaunchKernelGGL(k_fft_inv2w<FFT_PAIR_WIDE_S>, grid, block, b.fft_lds_pow2, s, b, b.fft_tiles, b.chans);
     else return hipErrorInvalidValue;
   } else if (b.n_fft_pow2 > 0 && b.fft_persist) {
-    hipLaunchKernelGGL(k_fft_inv_p, dim3(b.fft_grid), dim3(FFT_WG), FFT_LDS_PERSIST, s, b, b.fft_tiles, b.chans,
-                       b.n_fft_pow2);
+    if (b.fft_pf == 4)
+      hipLaunchKernelGGL(k_fft_inv_p<4>, dim3(b.fft_grid), dim3(FFT_WG), fft_lds_persist(4), s, b, b.fft_tiles, b.chans,
+                         b.n_fft_pow2);
+    else
+      hipLaunchKernelGGL(k_fft_inv_p<FFT_PF>, dim3(b.fft_grid), dim3(FFT_WG), fft_lds_persist(FFT_PF), s, b, b.fft_tiles,
+                         b.chans, b.n_fft_pow2);
   } else if (b.n_fft_pow2 > 0) {
     if (b.fft_tw_lds)
       hipLaunchKernelGGL((k_fft_inv<true, true>), dim3(b.n_fft_pow2), dim3(FFT_WG_ROWS), b.fft_lds_pow2, s, b, b.fft_tiles, b.chans, 0);
