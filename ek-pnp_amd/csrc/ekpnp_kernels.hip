@@ -1,20 +1,24 @@
 // ekpnp_kernels.hip -- gfx950 kernels of the EK-PNP coupled time step.
 //
-// One step is an LBM stage and three Poisson launches, each launch covering
-// every channel of the context:
+// One step is an LBM stage and three Poisson launches (two launches in all for a
+// small context), each launch covering every channel of the context:
 //   k_lbm       fused pull collide-stream of f (fluid), h (c+), g (c-) with the
 //               wall rules folded in; writes the post-collision state of every
 //               node in place of the next lattice and the FP64 charge density
 //               (replaces gpu_collide_save, gpu_boundary, gpu_stream,
 //               gpu_bc_charge: LBM.cu:331-1024)
-//   k_lbm_rows  the same, same bits, with fewer registers for FP32 storage with
-//               FP64 arithmetic on channels with nx a multiple of 64 (one
-//               launch for their wall rows, one for their interior rows; k_lbm
-//               keeps the other channels and the first step after
-//               initialisation)
+//   k_lbm_rows  the same, with fewer registers for FP32 storage with FP64
+//               arithmetic on channels with nx a multiple of 64 (one launch for
+//               their wall rows, one for their interior rows; k_lbm keeps the
+//               other channels and the first step after initialisation)
+//   k_lbm_fwd   small contexts of narrow rows: the step before's inverse
+//               x-transforms, the node updates of both and this step's forward
+//               x-transforms in one launch
 //   k_fft_fwd   per x-row: right-hand side with the wall lifts, real-to-complex
 //               FFT in LDS (replaces odd_extension + forward cuFFT,
-//               poisson.cu:211-263, 190)
+//               poisson.cu:211-263, 190); k_dft_fwd / k_dft_inv for widths of at
+//               least 24 that are no power of two, direct sums on the FP64 matrix
+//               cores
 //   k_tridiag   per wavenumber: the wall-normal tridiagonal solve as a chunked
 //               Thomas sweep joined by affine scans in LDS (replaces
 //               gpu_derivative and the y half of the 2-D cuFFT,
@@ -1491,8 +1495,8 @@ __device__ __forceinline__ double sub_pinned(double a, double b) {
 // begins by fetching descriptors, tables and rows that the one before has just
 // written.  64x128 with FP64 storage: 21.7 -> 18.7 us a step, with INV (below)
 // 16.3.  Bound: latency, of the gather, of a lone wave's FP64 instructions, of
-// the transforms' passes.  The transforms are k_fft_fwd_p's and the narrow rows' of k_fft_fwd, operation
-// for operation.
+// the transforms' passes.  The transforms are k_fft_fwd_p's and the narrow
+// rows' of k_fft_fwd, operation for operation.
 // ---------------------------------------------------------------------------
 constexpr int FUSE_ROWS = LBM_WG / 2 + 64;  // double2 of LDS rows (narrow: row stride nx | 1)
 constexpr int FUSE_TW = LBM_WG / 4;         // twiddles: a quadrant of at most LBM_WG nodes, or a narrow row's

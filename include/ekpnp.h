@@ -386,8 +386,9 @@ int ekpnp_autotune_lbm(ekpnp_ctx* ctx, int reps, double* out);
  * a launch of their own.  That
  * placement is chosen with the plan, when the wall work-groups fit beside
  * the tridiagonal's without another round; EKPNP_WALLS_IN_TRI=0 in the
- * environment at plan time turns it off.  Results do not depend on it.  No
- * counterpart in the reference. */
+ * environment at plan time turns it off, and small contexts of narrow rows
+ * update them in their one collide-stream launch.  Results do not depend on
+ * it.  No counterpart in the reference. */
 int ekpnp_get_poisson_plan(const ekpnp_ctx* ctx, int* out);
 
 /* ---- introspection / timing -------------------------------------------------- */
