@@ -72,6 +72,7 @@ constexpr int STAGE_SLOTS = 3, STAGE_THREADS = 4;
 struct ChannelTiles {
   int fft_first, fft_count;  // range in the FFT tile table
   int tri_first, tri_count;  // range in the tridiagonal tile table
+  int row_first;             // first of its ny entries in the row table
 };
 
 }  // namespace
@@ -91,6 +92,7 @@ struct ekpnp_ctx {
   std::vector<int2> tri_tiles;
   std::vector<int> first_tile;
   std::vector<int2> row_tiles;
+  int n_row_narrow = 0;          // its first rows, of channels of at most ROW_WAVE_NX nodes a row
   std::vector<double> walls;  // 6 planes x total_nx
   // device
   void* lat[2] = {nullptr, nullptr};
@@ -337,6 +339,7 @@ StepBuffers make_buffers(ekpnp_ctx* c) {
   b.blocks = c->d_blocks;
   b.row_tiles = c->d_row_tiles;
   b.n_row_tiles = (int)c->row_tiles.size();
+  b.n_row_narrow = c->n_row_narrow;
   b.cprime = c->d_cprime;
   b.lbm_row_tiles = c->d_lbm_split;
   b.n_lbm_row_tiles = c->n_lbm_row;
@@ -1162,8 +1165,15 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
   c->total_blocks = blocks;
   c->total_cprime = cprime;
   c->total_nx = wall;
-  for (int i = 0; i < n_channels; ++i)
-    for (int y = 0; y < c->desc[i].ny; ++y) c->row_tiles.push_back(make_int2(i, y));
+  // rows of narrow channels first (k_row_means_narrow)
+  for (const bool narrow : {true, false}) {
+    for (int i = 0; i < n_channels; ++i) {
+      if ((c->desc[i].nx <= ROW_WAVE_NX) != narrow) continue;
+      c->ctiles[i].row_first = (int)c->row_tiles.size();
+      for (int y = 0; y < c->desc[i].ny; ++y) c->row_tiles.push_back(make_int2(i, y));
+    }
+    if (narrow) c->n_row_narrow = (int)c->row_tiles.size();
+  }
 
   // LBM tiles, channel-major
   c->first_tile.resize(n_channels + 1);
@@ -1487,10 +1497,9 @@ int ekpnp_restart_channel(ekpnp_ctx* ctx, int channel, int mode, uint64_t seed) 
   const int t1 = channel + 1 < ctx->nchan ? ctx->first_tile[channel + 1] : (int)ctx->lbm_tiles.size();
   b.lbm_tiles = ctx->d_lbm_tiles + t0;
   b.n_lbm_tiles = t1 - t0;
-  int r0 = 0;
-  for (int ch = 0; ch < channel; ++ch) r0 += ctx->desc[ch].ny;
-  b.row_tiles = ctx->d_row_tiles + r0;
+  b.row_tiles = ctx->d_row_tiles + ctx->ctiles[channel].row_first;
   b.n_row_tiles = d.ny;
+  b.n_row_narrow = d.nx <= ROW_WAVE_NX ? d.ny : 0;
   if (ctx->opt.precision == EKPNP_POP_FP32)
     HIP_OR_FAIL(ctx, launch_row_means(b, ctx->d_refs, ctx->d_blocks, ctx->stream));
   HIP_OR_FAIL(ctx, launch_init_equilibrium(ctx->opt.precision, b, ctx->lat[ctx->cur], ctx->stream));

@@ -64,6 +64,7 @@ constexpr int MAX_INTERIOR_ROWS = 2048;  // 128 chunks x 16 rows per tridiagonal
 // holds them in
 constexpr int REF_BLOCK = 64;
 constexpr int BLK_STRIDE = 4;
+constexpr int ROW_WAVE_NX = 256;  // widest rows whose means one wave takes
 
 struct ChanDesc {
   int nx, ny, nk, flags;        // nk = nx/2 + 1 spectral columns
@@ -154,6 +155,7 @@ struct StepBuffers {
   float* blocks;                // storage references along x, [ny][nb][BLK_STRIDE] per channel
   const int2* row_tiles;        // (channel, row) per row-means work-group
   int n_row_tiles;
+  int n_row_narrow;             // the first of them: rows of at most ROW_WAVE_NX nodes
   double* cprime;               // Thomas coefficient entering chunk j of mode k, [tri_C][nk] per channel
 };
 

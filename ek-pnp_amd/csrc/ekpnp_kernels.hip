@@ -2906,7 +2906,7 @@ __global__ __launch_bounds__(256) void k_reduce_final(StepBuffers b) {
 __global__ __launch_bounds__(256) void k_row_means(StepBuffers b, double* __restrict__ out,
                                                    float* __restrict__ blocks_out) {
   __shared__ double red[4][REF_ROWS];
-  const int2 t = b.row_tiles[blockIdx.x];
+  const int2 t = b.row_tiles[b.n_row_narrow + blockIdx.x];
   const ChanDesc* __restrict__ cd = b.chans + t.x;
   const int nx = cd->nx, y = t.y, nb = cd->nb;
   const long long rec = cd->ref_off + (long long)REF_STRIDE * y;
@@ -2964,6 +2964,73 @@ __global__ __launch_bounds__(256) void k_row_means(StepBuffers b, double* __rest
     // x-flux is not the row's macroscopic one: no flux reference there
     const bool wall = (y == 0 || y == cd->ny - 1);
     out[rec + i] = (i >= REF_ROWS || (wall && i >= 3)) ? 0.0 : s / (double)nx;
+  }
+}
+
+// a product that the sum behind it must not take in unrounded
+__device__ __forceinline__ double times_rounded(double a, double b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+__device__ __forceinline__ double wave_total(double v) {  // wave_sum in every lane
+  const long long i = __double_as_longlong(wave_sum(v));
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)i), hi = __builtin_amdgcn_readfirstlane((unsigned)(i >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The same for rows of at most ROW_WAVE_NX nodes, a wave each: the sums of a row's 64-node
+// blocks are the wave sums that k_row_means adds up, and its block records too.
+// A work-group per row keeps 4 to 64 lanes of 256 busy there: 512 channels of
+// n_x = 4 312 -> 74 us, the 256-channel sweep 619 -> 264.
+__global__ __launch_bounds__(256) void k_row_means_narrow(StepBuffers b, double* __restrict__ out,
+                                                          float* __restrict__ blocks_out) {
+  const int row = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= b.n_row_narrow) return;
+  const int2 t = b.row_tiles[row];
+  const ChanDesc* __restrict__ cd = b.chans + t.x;
+  const int nx = cd->nx, y = t.y, nb = cd->nb;  // nb <= 4
+  const long long rec = cd->ref_off + (long long)REF_STRIDE * y;
+  const long long kn0 = cd->blk_off + (long long)BLK_STRIDE * nb * y;
+  if (!cd->active) {
+    for (int i = lane; i < REF_STRIDE; i += 64) out[rec + i] = b.refs[rec + i];
+    for (int i = lane; i < BLK_STRIDE * nb; i += 64) blocks_out[kn0 + i] = b.blocks[kn0 + i];
+    return;
+  }
+  const long long o = cd->fld_off + (long long)y * nx, st = b.macro_stride;
+  static_assert(ROW_WAVE_NX == 4 * REF_BLOCK, "one block per round");
+  double f[4][4];  // rho, c+, c-, u_x of the wave's node of each block
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int x = REF_BLOCK * k + lane;
+    const bool on = x < nx;
+    f[k][0] = on ? b.macro[M_RHO * st + o + x] : 0.0;
+    f[k][1] = on ? b.macro[M_CP * st + o + x] : 0.0;
+    f[k][2] = on ? b.macro[M_CN * st + o + x] : 0.0;
+    f[k][3] = on ? b.macro[M_UX * st + o + x] : 0.0;
+  }
+  double red[4][REF_ROWS] = {};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (k >= nb) break;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      red[k][i] = wave_total(f[k][i]);
+      red[k][3 + i] = wave_total(times_rounded(f[k][i], f[k][3]));
+    }
+    if (lane < BLK_STRIDE) {
+      const double cnt = (double)min(REF_BLOCK, nx - REF_BLOCK * k);
+      blocks_out[kn0 + (long long)BLK_STRIDE * k + lane] =
+          lane == 3 ? 0.0f : (float)((lane == 0 ? red[k][0] : lane == 1 ? red[k][1] : red[k][2]) / cnt);
+    }
+  }
+  const bool wall = (y == 0 || y == cd->ny - 1);
+#pragma unroll
+  for (int i = 0; i < REF_STRIDE; ++i) {
+    const double s = i < REF_ROWS ? (red[0][min(i, REF_ROWS - 1)] + red[1][min(i, REF_ROWS - 1)]) +
+                                        (red[2][min(i, REF_ROWS - 1)] + red[3][min(i, REF_ROWS - 1)])
+                                  : 0.0;
+    if (lane == i) out[rec + i] = (i >= REF_ROWS || (wall && i >= 3)) ? 0.0 : s / (double)nx;
   }
 }
 
@@ -3369,7 +3436,10 @@ hipError_t launch_to_q(int precision, const StepBuffers& b, const void* src, voi
 }
 
 hipError_t launch_row_means(const StepBuffers& b, double* out, float* blocks_out, hipStream_t s) {
-  hipLaunchKernelGGL(k_row_means, dim3(b.n_row_tiles), dim3(256), 0, s, b, out, blocks_out);
+  if (b.n_row_narrow > 0)
+    hipLaunchKernelGGL(k_row_means_narrow, dim3((b.n_row_narrow + 3) / 4), dim3(256), 0, s, b, out, blocks_out);
+  if (b.n_row_tiles > b.n_row_narrow)
+    hipLaunchKernelGGL(k_row_means, dim3(b.n_row_tiles - b.n_row_narrow), dim3(256), 0, s, b, out, blocks_out);
   return hipGetLastError();
 }
 
