@@ -357,7 +357,9 @@ int ekpnp_set_poisson_plan(ekpnp_ctx* ctx, int fft_elems, int tri_rows, int fft_
  * 2048, 4096}, the three FFT kernel families and tri_rows in {8, 16} (reps solves
  * each, three passes over the candidates, HIP events on the context's
  * stream), keeps the fastest, and restores
- * psi.  out (may be NULL, else 4 doubles) receives {fft_elems, tri_rows, ms
+ * psi.  A small context of narrow rows, whose step runs the transforms inside
+ * its collide-stream launch, keeps to the persistent family that launch holds.
+ * out (may be NULL, else 4 doubles) receives {fft_elems, tri_rows, ms
  * per solve, fft_persistent}.  No counterpart in the reference (cuFFT plans are
  * fixed by main.cu:113). */
 int ekpnp_autotune(ekpnp_ctx* ctx, int reps, double* out);
@@ -404,7 +406,9 @@ size_t ekpnp_device_bytes(const ekpnp_ctx* ctx);
  * untimed replay, per step).  The
  * launches are those of the coupled step: when the plan puts the wall rows
  * on the tridiagonal launch (ekpnp_get_poisson_plan), [0] covers the other
- * rows and [2] includes the wall rows. */
+ * rows and [2] includes the wall rows; in a small context of narrow rows [0]
+ * includes the forward x-FFT ([1] is then the gap between two events), and in
+ * [4] the inverse one too. */
 int ekpnp_time_stages(ekpnp_ctx* ctx, int nsteps, double* ms_out);
 /* Measurement: a non-temporal float4 device copy of `bytes` bytes (a
  * multiple of 16) on `device`, grid work-groups of 256 lanes striding over
