@@ -93,7 +93,7 @@ struct GemmArgs {
   uint16_t* c;         // BF16 a_l or g_l [rows][N] (HIDDEN, LOSS, DGELU)
   uint16_t* ct;        // its transpose [N][ldt]    (HIDDEN while training, LOSS, DGELU; may be null)
   long long ldt;
-  float* partial;      // squared-error sum of each work-group (LOSS)
+  double* partial;     // squared-error sum of each work-group (LOSS)
   float scale;         // 1 / (M N)                 (LOSS)
 };
 
@@ -104,10 +104,12 @@ struct GemmArgs {
 // 4.5 - 12 us now).
 template <int EPI>
 __global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
-  __shared__ float red[MLP_WG / 64];
+  __shared__ double red[MLP_WG / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m0 = blockIdx.y * TILE, n0 = (blockIdx.x * (MLP_WG / 64) + wave) * TILE;
-  float e2 = 0.f;
+  // squared errors, summed in FP64: an FP32 sum over the work-group's 1024
+  // loses the small ones beside a large one
+  double e2 = 0.0;
   if (n0 < g.N) {
     const floatx4 acc = tile_product(g.A, g.K, g.B, g.K, m0, n0, g.K);
     const int n = n0 + (lane & 15), mr = m0 + (lane >> 4) * 4;
@@ -132,7 +134,7 @@ __global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
         g.g[o] = gv;
         h[r] = f2bf(gv);
         g.c[o] = h[r];
-        e2 += d * d;
+        e2 += (double)d * (double)d;
       } else {
         v *= dgelu(g.z[o]);
         g.g[o] = v;
@@ -301,7 +303,7 @@ struct ekpnp_mlp {
   std::vector<uint16_t*> wt;   // [L+2], W_l transposed [in_l][out_l], l >= 2
   float* t = nullptr;          // targets
   float* xin = nullptr;        // FP32 input staging
-  float* partial = nullptr;    // squared-error sums, written by the device into host memory
+  double* partial = nullptr;   // squared-error sums, written by the device into host memory
   Layer* layers = nullptr;     // layer table of the weight kernels, layers 1..L+1
   int n_wgrad = 0, n_update = 0;  // their work-groups
   std::vector<void*> bufs;     // every device allocation
@@ -502,7 +504,7 @@ int ekpnp_mlp_create(const ekpnp_mlp_config* cfg, ekpnp_mlp** out) {
     if (l >= 2) A(&m->wt[l], n * m->in_dim[l]);
   }
   const dim3 lg = gemm_grid(cfg->n_out, (int)R);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&m->partial, (size_t)lg.x * lg.y * sizeof(float), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&m->partial, (size_t)lg.x * lg.y * sizeof(double), hipHostMallocDefault);
   std::vector<Layer> tab(L + 1);
   for (int l = 1; l <= L + 1; ++l) {
     Layer& d = tab[l - 1];
