@@ -10,11 +10,14 @@
 #include <algorithm>
 #include <atomic>
 #include <cerrno>
+#include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <exception>
 #include <string>
 #include <thread>
@@ -65,9 +68,10 @@ int pow2_ceil(int v) {
 }
 
 // copy_to_host: bytes per staged piece, pieces in flight, copying threads,
-// and the size from which it uses several pieces and threads
+// the size from which it uses several pieces and threads, and how long a
+// thread spins for the next piece before it sleeps
 constexpr size_t STAGE_CHUNK = 8u << 20, STAGE_PARALLEL_MIN = 2u << 20;
-constexpr int STAGE_SLOTS = 3, STAGE_THREADS = 4;
+constexpr int STAGE_SLOTS = 3, STAGE_THREADS = 4, STAGE_SPIN_US = 50;
 
 struct ChannelTiles {
   int fft_first, fft_count;  // range in the FFT tile table
@@ -851,6 +855,30 @@ void map_pages(char* p, size_t bytes) {
 #endif
 }
 
+// A condition that another thread makes true with set().  It is expected within
+// microseconds while pieces follow each other, and anything later while the
+// stream works off the steps in front of the first: a short spin, then sleep.
+struct Gate {
+  std::mutex m;
+  std::condition_variable cv;
+  template <typename F>
+  void set(F change) {
+    {
+      std::lock_guard<std::mutex> lock(m);
+      change();
+    }
+    cv.notify_all();
+  }
+  template <typename F>
+  void wait(F ready) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(STAGE_SPIN_US);
+    while (std::chrono::steady_clock::now() < until)
+      if (ready()) return;
+    std::unique_lock<std::mutex> lock(m);
+    cv.wait(lock, ready);
+  }
+};
+
 // dst = bytes of device memory at src, once the stream's earlier work is done.
 // The runtime's copy to pageable memory moves a field at 10 GB/s (13 ms for the
 // 134 MB of 8192 x 2048): it copies and first touches the caller's pages on one
@@ -904,6 +932,7 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
   std::atomic<size_t> ready{0};
   std::atomic<int> left{0};
   std::atomic<bool> stop{false};
+  Gate announced, copied;
   const int threads = STAGE_THREADS;
   auto share = [&](int t, size_t i, bool map_only) {
     const size_t n = size_of(i), part = (n / threads + 4095) & ~(size_t)4095, a = std::min(n, part * t);
@@ -916,10 +945,10 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
       helpers.emplace_back([&, t] {
         for (size_t i = 0; i < pieces; ++i) {
           share(t, i, true);
-          while (ready.load(std::memory_order_acquire) <= i)
-            if (stop.load(std::memory_order_relaxed)) return;
+          announced.wait([&] { return ready.load() > i || stop.load(); });
+          if (ready.load() <= i) return;
           share(t, i, false);
-          left.fetch_sub(1, std::memory_order_release);
+          if (left.fetch_sub(1) == 1) copied.set([] {});
         }
       });
   } catch (const std::exception&) {
@@ -932,14 +961,13 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
     share(0, i, true);
     e = hipEventSynchronize(c->stage_ev[i % slots]);
     if (e != hipSuccess) break;
-    left.store(helping, std::memory_order_relaxed);
-    ready.store(i + 1, std::memory_order_release);
+    left.store(helping);
+    announced.set([&] { ready.store(i + 1); });
     for (int t = 0; t < threads; t = t == 0 ? helping + 1 : t + 1) share(t, i, false);
-    while (left.load(std::memory_order_acquire) > 0) {
-    }
+    copied.wait([&] { return left.load() == 0; });
     if (i + slots < pieces) e = issue(i + slots);
   }
-  stop.store(true);
+  announced.set([&] { stop.store(true); });
   for (auto& t : helpers) t.join();
   if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // no copy into the staging buffer stays in flight
   return e;
