@@ -86,6 +86,7 @@ struct GemmArgs {
   const uint16_t* A;   // [rows][K], rows a multiple of 32
   const uint16_t* B;   // [N][K]
   int M, N, K;         // M: rows that count; the transposes hold 0 from row M up to the next multiple of 32
+  int row_tiles;       // of M rounded up to that multiple
   const float* bias;   // [N]                       (HIDDEN, OUT, LOSS)
   float* z;            // pre-activation [M][N]: written (HIDDEN, OUT), read (DGELU)
   const float* t;      // targets [M][N]            (LOSS)
@@ -106,7 +107,9 @@ template <int EPI>
 __global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
   __shared__ double red[MLP_WG / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int m0 = blockIdx.y * TILE, n0 = (blockIdx.x * (MLP_WG / 64) + wave) * TILE;
+  const int row_tile = (int)(blockIdx.z * gridDim.y + blockIdx.y), m0 = row_tile * TILE;
+  if (row_tile >= g.row_tiles) return;  // the last z may hold fewer
+  const int n0 = (blockIdx.x * (MLP_WG / 64) + wave) * TILE;
   // squared errors, summed in FP64: an FP32 sum over the work-group's 1024
   // loses the small ones beside a large one
   double e2 = 0.0;
@@ -152,7 +155,7 @@ __global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
     if (lane == 0) red[wave] = e2;
     __syncthreads();
     if (threadIdx.x == 0)
-      g.partial[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+      g.partial[(size_t)row_tile * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
   }
 }
 
@@ -334,7 +337,15 @@ void release(ekpnp_mlp* m) {
 }
 
 int rows_of(int B) { return (B + KSTEP - 1) / KSTEP * KSTEP; }
-dim3 gemm_grid(int N, int rows) { return dim3((N / TILE + MLP_WG / 64 - 1) / (MLP_WG / 64), rows / TILE); }
+// x: columns; y and z: rows, which in y alone would end at 65535 (of a launch's
+// 65536) tiles, a batch of 1,048,560
+constexpr int MAX_GRID_Y = 65535;
+dim3 gemm_grid(int N, int rows) {
+  const int tiles = rows / TILE, z = (tiles + MAX_GRID_Y - 1) / MAX_GRID_Y;
+  return dim3((N / TILE + MLP_WG / 64 - 1) / (MLP_WG / 64), (tiles + z - 1) / z, z);
+}
+// squared-error sums of a batch of rows (k_gemm<EPI_LOSS>)
+size_t loss_partials(int N, int rows) { return (size_t)gemm_grid(N, rows).x * (rows / TILE); }
 
 // layers 1 .. last of the forward pass (hidden layers, or with L + 1 the
 // linear output too); train: the transposed activations are written as well
@@ -350,6 +361,7 @@ hipError_t forward(ekpnp_mlp* m, const float* x_host, int B, int last, bool trai
     g.A = m->a[l - 1];
     g.B = m->pbf + m->off_w[l];
     g.M = B;
+    g.row_tiles = rows / TILE;
     g.N = m->out_dim[l];
     g.K = m->in_dim[l];
     g.bias = m->p32 + m->off_b[l];
@@ -393,6 +405,7 @@ int loss_grad(ekpnp_mlp* m, const float* x_host, const float* t_host, int B) {
       g.z = m->z[l];
     }
     g.M = B;
+    g.row_tiles = rows / TILE;
     g.N = m->out_dim[l];
     g.g = m->g[l];
     g.c = m->gb[l];
@@ -409,9 +422,9 @@ int loss_grad(ekpnp_mlp* m, const float* x_host, const float* t_host, int B) {
 
 float loss_of(const ekpnp_mlp* m, int B) {
   const int no = m->cfg.n_out;
-  const dim3 grid = gemm_grid(no, rows_of(B));
+  const size_t n = loss_partials(no, rows_of(B));
   double s = 0.0;
-  for (unsigned i = 0; i < grid.x * grid.y; ++i) s += m->partial[i];
+  for (size_t i = 0; i < n; ++i) s += m->partial[i];
   return (float)(s / (double)(B * no));
 }
 
@@ -503,8 +516,8 @@ int ekpnp_mlp_create(const ekpnp_mlp_config* cfg, ekpnp_mlp** out) {
     if (l <= L) A(&m->at[l], R * n);
     if (l >= 2) A(&m->wt[l], n * m->in_dim[l]);
   }
-  const dim3 lg = gemm_grid(cfg->n_out, (int)R);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&m->partial, (size_t)lg.x * lg.y * sizeof(double), hipHostMallocDefault);
+  if (e == hipSuccess)
+    e = hipHostMalloc((void**)&m->partial, loss_partials(cfg->n_out, (int)R) * sizeof(double), hipHostMallocDefault);
   std::vector<Layer> tab(L + 1);
   for (int l = 1; l <= L + 1; ++l) {
     Layer& d = tab[l - 1];
