@@ -1165,6 +1165,14 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
   c->opt = o;
   c->nchan = n_channels;
   c->elem = (o.precision == EKPNP_POP_FP32) ? 4 : 8;
+  // the device's sizes, before anything is planned by them
+  int max_lds = 65536;
+  if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, o.device) != hipSuccess)
+    max_lds = 65536;
+  c->max_lds = max_lds;
+  int n_cu = 256;
+  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o.device) == hipSuccess && n_cu > 0)
+    c->n_cu = n_cu;
   c->params.assign(channels, channels + n_channels);
   c->desc.resize(n_channels);
   c->ctiles.resize(n_channels);
@@ -1330,13 +1338,6 @@ int ekpnp_create(const ekpnp_channel_params* channels, int n_channels, const ekp
     return EKPNP_ERR_HIP;
   }
   c->sb = make_buffers(c);
-  int max_lds = 65536;
-  if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, o.device) != hipSuccess)
-    max_lds = 65536;
-  c->max_lds = max_lds;
-  int n_cu = 256;
-  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o.device) == hipSuccess && n_cu > 0)
-    c->n_cu = n_cu;
   // default plan (ekpnp_autotune refines it): rows of nx = 4096 and 8192
   // run fastest in the row-pair kernels (two rows per work-group; when the
   // channels' widths differ, the one-tile kernels with as many rows as fit
