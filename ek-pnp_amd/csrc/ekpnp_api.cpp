@@ -450,11 +450,15 @@ int x_family(const ChanDesc& d) { return d.pow2 ? 0 : d.nx >= DFT_MIN_NX ? 1 : 2
 //   32 channels (32, 64)   576        35.2 -> 23.4
 //   64x128 x48 fp32       1536        41.5 -> 38.7    64x128 x56 fp32  1792  44.0 -> 44.7
 //   64x128 x40 fp64       1280        42.7 -> 40.4    64x128 x64 fp64  2048  56.4 -> 58.7
-//   32 wide x90           1010        34.3 -> 32.9    32 wide x120     1440  38.6 -> 39.6
-// and with rows below 24 nodes, FP32 storage:
+//   32 wide x90           1040        33.2 -> 32.0    32 wide x120     1448  37.2 -> 36.9, 36.4
+// (two draws of heights 64 and 128) and with rows below 24 nodes, FP32 storage:
 //   n_x = 4 x1100         2750        70.4 -> 63.1    n_x = 4 x1300    3250  89.3 -> 89.4
 //   n_x = 8 x450          2800        51.4 -> 50.6    12, 20 x400      4000  99.5 -> 100.6
-constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_NARROW = 12;
+// 16 nodes are not narrow: their transforms apart are the pipelined kernels'
+// (n_y = 128, and 60: the last tile of a channel partly empty):
+//   n_x = 16 x192         1536        38.2 -> 35.9    n_x = 16 x208    1664  39.0 -> 40.3
+//   n_x = 16, 60 x384     1536        38.5 -> 37.6    n_x = 16, 60 x416 1664 40.0 -> 43.7, x768 3072 54.9 -> 64.1
+constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_NARROW = 12, LBM_FWD_NARROW_POW2 = 8;
 // The inverse x-transforms of the step before are in that launch too, with FP64
 // storage while it is emptier still (each work-group transforms a row to either
 // side as well: half as much again at 4 rows a tile, three times at one).  Step
@@ -462,10 +466,21 @@ constexpr int LBM_FWD_TILES_PER_CU = 6, LBM_FWD_TILES_PER_CU_NARROW = 12;
 //   10x101 fp64     4 tiles  15.5 -> 13.5    32 channels (32, 64)  576  29.6 -> 23.4
 //   64x128 fp64    32        18.7 -> 16.3    n_x = 4 x512 fp32    1280  38.7 -> 35.2
 //   256x256 fp32  256        21.8 -> 18.6    64x128 x48 fp32      1536  41.0 -> 38.7
-//   256x512 fp64  512        29.1 -> 25.4    256 wide x15 fp32    1440  42.4 -> 42.9
-//   256x1000 fp64 1000       37.6 -> 38.4    n_x = 4 x900 fp32    2250  56.2 -> 54.6
+//   256x512 fp64  512        29.1 -> 25.4    256x96 x15 fp32      1440  40.5 -> 40.1
+//   256x1000 fp64 1000       37.6 -> 38.4
 //   64x128 x32 fp64 1024     35.4 -> 36.4
-constexpr int LBM_FWD_INV_TILES_PER_CU_FP64 = 3;
+// Narrow rows with FP32 storage: past LBM_FWD_TILES_PER_CU only with rows that hold whole
+// groups of 4 nodes (or at most 4), of 8 nodes up to LBM_FWD_INV_TILES_PER_CU_8; the others'
+// spectra, of an even number of modes a row or ragged tiles, lose:
+//   n_x = 4 x597         1791  44.9 -> 43.6    x939  2817  61.1 -> 59.3
+//   n_x = 12 x358        1790  41.3 -> 41.1    x614  3070  59.4 -> 58.9    x409  2045  46.4 -> 44.1
+//   n_x = 20 x138        1794  39.6 -> 39.0    x177  2301  45.9 -> 44.6    x217  2821  51.0 -> 52.2
+//   n_x = 8 x299         1794  41.8 -> 41.4    x384  2304  47.2 -> 47.4    x512  3072  55.3 -> 58.2
+//   n_x = 6 x384         1536  38.4 -> 37.7    x512  2048  45.4 -> 48.3    x704  2816  57.1 -> 61.5
+//   n_x = 7 x384         1536  37.8 -> 37.7    x448  1792  42.3 -> 43.9    x768  3072  58.2 -> 63.4
+//   n_x = 10 x307        1535  37.3 -> 35.9    x358  1790  39.6 -> 40.6    x614  3070  54.3 -> 58.1
+//   n_x = 18 x192        1536  36.6 -> 35.8    x224  1792  39.9 -> 41.2    x384  3072  56.6 -> 60.3
+constexpr int LBM_FWD_INV_TILES_PER_CU_FP64 = 3, LBM_FWD_INV_TILES_PER_CU_8 = 9;
 void build_lbm_fwd(ekpnp_ctx* c) {
   c->lbm_fwd.clear();
   for (auto& d : c->desc) d.lbm_span = d.nx <= LBM_WG ? LBM_WG / d.nx * d.nx : LBM_WG;
@@ -481,12 +496,19 @@ void build_lbm_fwd(ekpnp_ctx* c) {
     for (int n = 0; n < d.nx * d.ny; n += d.lbm_span) c->lbm_fwd.push_back(make_int2(i, n));
   }
   c->lbm_fwd_kind = n_rows == 0 ? FWD_GENERAL : n_rows == c->nchan ? FWD_ROWS : FWD_MIXED;
-  bool narrow = c->opt.precision == EKPNP_POP_FP32;
-  for (const auto& d : c->desc) narrow = narrow && d.nx < DFT_MIN_NX;
-  if (c->lbm_fwd.size() > (size_t)(narrow ? LBM_FWD_TILES_PER_CU_NARROW : LBM_FWD_TILES_PER_CU) * c->n_cu)
-    c->lbm_fwd.clear();
-  c->lbm_inv = !c->lbm_fwd.empty() && (c->opt.precision == EKPNP_POP_FP32 ||
-                                       c->lbm_fwd.size() <= (size_t)LBM_FWD_INV_TILES_PER_CU_FP64 * c->n_cu);
+  const bool fp64 = c->opt.precision == EKPNP_POP_FP64;
+  bool narrow = !fp64, groups = true, eight = false;
+  for (const auto& d : c->desc) {
+    narrow = narrow && d.nx < DFT_MIN_NX && (!d.pow2 || d.nx <= LBM_FWD_NARROW_POW2);
+    groups = groups && (d.nx <= 4 || d.nx % 4 == 0);
+    eight = eight || d.nx == LBM_FWD_NARROW_POW2;
+  }
+  const int most = narrow ? LBM_FWD_TILES_PER_CU_NARROW : LBM_FWD_TILES_PER_CU;
+  const int most_inv = fp64 ? LBM_FWD_INV_TILES_PER_CU_FP64
+                       : !(narrow && groups) ? LBM_FWD_TILES_PER_CU
+                       : eight ? LBM_FWD_INV_TILES_PER_CU_8 : most;
+  if (c->lbm_fwd.size() > (size_t)most * c->n_cu) c->lbm_fwd.clear();
+  c->lbm_inv = !c->lbm_fwd.empty() && c->lbm_fwd.size() <= (size_t)most_inv * c->n_cu;
 }
 
 // a new interior tile shape for the row kernel: table, buffers, graphs
