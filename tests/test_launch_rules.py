@@ -46,3 +46,31 @@ def test_one_launch_limits_follow_the_compute_units(so):
 def test_narrow_rows_leave_the_launch_where_it_loses(so, sizes, copies, want):
     got = fake_hip.launches(so, [(sizes * n, "fp32", {}) for n in copies])
     assert [fused(s) for s in got] == want
+
+
+def cached(steps):
+    """population planes that the collide-stream's last launch takes through the caches"""
+    k = [n for n in steps if n.startswith(("k_lbm<", "k_lbm_rows<false"))]
+    return int(k[-1].rstrip(">").split(", ")[-1])
+
+
+# both lattices of a context in MB beside each
+@pytest.mark.parametrize("sizes,precision,options,want", [
+    ([(1024, 800)], "fp64", {}, 13),           # 354
+    ([(1024, 1000)], "fp64", {}, 9),           # 442
+    ([(1024, 1300)], "fp64", {}, 9),           # 575
+    ([(1024, 2000)], "fp64", {}, 6),           # 885
+    ([(2048, 1024)], "fp64", {}, 4),           # 906
+    ([(4096, 640)], "fp64", {}, 4),            # 1132
+    ([(1024, 514)], "fp64", {}, 27),           # 227
+    ([(512, 256)], "fp64", {}, 0),             # 57
+    # the batches of test_gpu_lbm_cache.py, and the last narrow one below its limit
+    *[([(1024, 64)] * n, "fp32", {}, w) for n, w in ((5, 0), (6, 27), (11, 27), (12, 18), (16, 18), (20, 13), (30, 9),
+                                                     (45, 6), (70, 4), (100, 2), (160, 0))],
+    *[([(1000, 64)] * n, "fp32", {}, w) for n, w in ((16, 27), (17, 18), (24, 13), (45, 6), (90, 2))],
+    *[([(32, 256)] * n, "fp32", {}, w) for n, w in ((129, 27), (130, 0), (131, 0))],
+    *[([(1000, 64)] * n, "fp32", {"compute_fp64": False}, w) for n, w in ((16, 27), (17, 18))],
+    *[([(1024, 64)] * n, "fp64", {}, w) for n, w in ((2, 0), (3, 27), (8, 27), (9, 18), (12, 13), (35, 4))],
+])
+def test_cached_planes(so, sizes, precision, options, want):
+    assert cached(fake_hip.launches(so, [(sizes, precision, options)])[0]) == want
