@@ -91,10 +91,11 @@ def calibrate_copy():
 
 
 def measured_traffic(config, precision, wrows=0):
-    """HBM bytes per launch of the row kernel's interior rows, for the tile
-    shape the run used, from the committed counter summary of this workload
-    (FETCH_SIZE and WRITE_SIZE scaled by the copy calibration), or None when
-    no summary exists for it."""
+    """Bytes between L2 and the fabric per launch of the row kernel's interior
+    rows, for the tile shape the run used, from the committed counter summary of
+    this workload (FETCH_SIZE and WRITE_SIZE scaled by the copy calibration), or
+    None when no summary exists for it.  Reads that the Infinity Cache answers
+    are among them: HBM bytes only where every population plane is streamed."""
     path = os.path.join(ROOT, "profiles", f"k_lbm_{config}_{precision}_traffic.json")
     if not os.path.exists(path):
         return None

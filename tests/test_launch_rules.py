@@ -1,5 +1,8 @@
 """Which kernels a context of given channels launches (CPU only: the library on a
 HIP runtime without a device)."""
+import json
+import os
+
 import pytest
 
 import fake_hip
@@ -74,3 +77,13 @@ def cached(steps):
 ])
 def test_cached_planes(so, sizes, precision, options, want):
     assert cached(fake_hip.launches(so, [(sizes, precision, options)])[0]) == want
+
+
+@pytest.mark.parametrize("config,size", [("c1", (4096, 1024)), ("c4", (8192, 2048))])
+def test_traffic_summaries_are_of_the_kernel_that_runs(so, config, size):
+    with open(os.path.join(fake_hip.ROOT, "profiles", f"k_lbm_{config}_fp32_traffic.json")) as f:
+        d = json.load(f)
+    runs = {n for n in fake_hip.launches(so, [([size], "fp32", {})])[0] if n.startswith("k_lbm_rows<")}
+    named = {k.split("ekpnp::", 1)[1].split("(")[0] for k in [d["kernel"], *d["kernel_by_tile_rows"].values()]}
+    assert set(d["kernel_by_tile_rows"]) == set(d["bytes_per_launch_by_tile_rows"]) == {"0", "2", "4"}
+    assert named == runs
