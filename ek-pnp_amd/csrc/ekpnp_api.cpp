@@ -70,9 +70,9 @@ int pow2_ceil(int v) {
 // copy_to_host: bytes per staged piece, pieces in flight, copying threads,
 // the size from which it uses several pieces and threads, the size from which it
 // asks what the destination is, and how long a thread spins for the next piece
-// before it sleeps
+// before it sleeps (a piece's DMA takes 20 to 170 us)
 constexpr size_t STAGE_CHUNK = 8u << 20, STAGE_PARALLEL_MIN = 2u << 20, STAGE_ASK_MIN = 64u << 10;
-constexpr int STAGE_SLOTS = 3, STAGE_THREADS = 4, STAGE_SPIN_US = 50;
+constexpr int STAGE_SLOTS = 3, STAGE_THREADS = 4, STAGE_SPIN_US = 500;
 
 struct ChannelTiles {
   int fft_first, fft_count;  // range in the FFT tile table
@@ -158,7 +158,7 @@ struct ekpnp_ctx {
   // largest field read (at most STAGE_SLOTS x STAGE_CHUNK bytes)
   char* stage = nullptr;
   size_t stage_bytes = 0;
-  hipEvent_t stage_ev[STAGE_SLOTS] = {};
+  hipEvent_t stage_ev[STAGE_SLOTS + 1] = {};  // a piece has come; the work before the copy is done
   std::map<std::tuple<int, int, int, int>, hipGraphExec_t> graphs;
   std::string err;
 };
@@ -889,9 +889,7 @@ void map_pages(char* p, size_t bytes) {
 #endif
 }
 
-// A condition that another thread makes true with set().  It is expected within
-// microseconds while pieces follow each other, and anything later while the
-// stream works off the steps in front of the first: a short spin, then sleep.
+// A condition that another thread makes true with set()
 struct Gate {
   std::mutex m;
   std::condition_variable cv;
@@ -903,11 +901,13 @@ struct Gate {
     }
     cv.notify_all();
   }
+  // spins for spin_us, then sleeps
   template <typename F>
-  void wait(F ready) {
-    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(STAGE_SPIN_US);
-    while (std::chrono::steady_clock::now() < until)
+  void wait(int spin_us, F ready) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(spin_us);
+    do {
       if (ready()) return;
+    } while (std::chrono::steady_clock::now() < until);
     std::unique_lock<std::mutex> lock(m);
     cv.wait(lock, ready);
   }
@@ -947,7 +947,7 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
       (void)hipGetLastError();
     }
   }
-  for (size_t i = 0; i < slots && pieces > 1 && c->stage; ++i)
+  for (size_t i = 0; i <= STAGE_SLOTS && pieces > 1 && c->stage; ++i)
     if (!c->stage_ev[i] && hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming) != hipSuccess) {
       (void)hipGetLastError();
       c->stage_ev[i] = nullptr;
@@ -971,11 +971,17 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
                                   hipMemcpyDeviceToHost, c->stream);
     return e == hipSuccess ? hipEventRecord(c->stage_ev[i % slots], c->stream) : e;
   };
-  // helpers copy their share of each piece the main thread announces in `ready`
+  // The helpers sleep while the stream works off what is in front of the copy,
+  // wake when that is done, with the first piece's DMA under way, and copy their
+  // share of each piece the main thread announces in `ready`.
   std::atomic<size_t> ready{0};
   std::atomic<int> left{0};
   std::atomic<bool> stop{false};
-  Gate announced, copied;
+  const hipEvent_t begin = c->stage_ev[STAGE_SLOTS];
+  const bool idle = hipStreamQuery(c->stream) == hipSuccess;
+  if (!idle) (void)hipGetLastError();
+  std::atomic<bool> begun{idle};
+  Gate wake, announced, copied;
   const int threads = STAGE_THREADS;
   auto share = [&](int t, size_t i, bool map_only) {
     const size_t n = size_of(i), part = (n / threads + 4095) & ~(size_t)4095, a = std::min(n, part * t);
@@ -988,7 +994,8 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
       helpers.emplace_back([&, t] {
         for (size_t i = 0; i < pieces; ++i) {
           share(t, i, true);
-          announced.wait([&] { return ready.load() > i || stop.load(); });
+          if (i == 0) wake.wait(0, [&] { return begun.load() || stop.load(); });
+          announced.wait(STAGE_SPIN_US, [&] { return ready.load() > i || stop.load(); });
           if (ready.load() <= i) return;
           share(t, i, false);
           if (left.fetch_sub(1) == 1) copied.set([] {});
@@ -998,19 +1005,25 @@ hipError_t copy_to_host(ekpnp_ctx* c, void* dst, const void* src, size_t bytes) 
     // fewer threads than asked for: the caller's thread takes their shares
   }
   const int helping = (int)helpers.size();
-  hipError_t e = hipSuccess;
+  hipError_t e = idle ? hipSuccess : hipEventRecord(begin, c->stream);
   for (size_t i = 0; i < slots && e == hipSuccess; ++i) e = issue(i);
   for (size_t i = 0; i < pieces && e == hipSuccess; ++i) {
     share(0, i, true);
+    if (i == 0 && !idle) {
+      e = hipEventSynchronize(begin);
+      wake.set([&] { begun.store(true); });
+      if (e != hipSuccess) break;
+    }
     e = hipEventSynchronize(c->stage_ev[i % slots]);
     if (e != hipSuccess) break;
     left.store(helping);
     announced.set([&] { ready.store(i + 1); });
     for (int t = 0; t < threads; t = t == 0 ? helping + 1 : t + 1) share(t, i, false);
-    copied.wait([&] { return left.load() == 0; });
+    copied.wait(STAGE_SPIN_US, [&] { return left.load() == 0; });
     if (i + slots < pieces) e = issue(i + slots);
   }
-  announced.set([&] { stop.store(true); });
+  wake.set([&] { stop.store(true); });
+  announced.set([] {});
   for (auto& t : helpers) t.join();
   if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // no copy into the staging buffer stays in flight
   return e;

@@ -104,6 +104,7 @@ int hipGetLastError() { return 0; }
 const char* hipGetErrorString(int) { return "fake HIP"; }
 int hipDeviceSynchronize() { return 0; }
 int hipStreamSynchronize(void*) { return 0; }
+int hipStreamQuery(void*) { return 0; }
 int hipStreamDestroy(void*) { return 0; }
 int hipEventDestroy(void*) { return 0; }
 int hipEventRecord(void*, void*) { return 0; }
