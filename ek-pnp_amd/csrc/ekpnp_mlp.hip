@@ -86,7 +86,6 @@ struct GemmArgs {
   const uint16_t* A;   // [rows][K], rows a multiple of 32
   const uint16_t* B;   // [N][K]
   int M, N, K;         // M: rows that count; the transposes hold 0 from row M up to the next multiple of 32
-  int row_tiles;       // of M rounded up to that multiple
   const float* bias;   // [N]                       (HIDDEN, OUT, LOSS)
   float* z;            // pre-activation [M][N]: written (HIDDEN, OUT), read (DGELU)
   const float* t;      // targets [M][N]            (LOSS)
@@ -107,9 +106,7 @@ template <int EPI>
 __global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
   __shared__ double red[MLP_WG / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row_tile = (int)(blockIdx.z * gridDim.y + blockIdx.y), m0 = row_tile * TILE;
-  if (row_tile >= g.row_tiles) return;  // the last z may hold fewer
-  const int n0 = (blockIdx.x * (MLP_WG / 64) + wave) * TILE;
+  const int m0 = blockIdx.y * TILE, n0 = (blockIdx.x * (MLP_WG / 64) + wave) * TILE;
   // squared errors, summed in FP64: an FP32 sum over the work-group's 1024
   // loses the small ones beside a large one
   double e2 = 0.0;
@@ -155,7 +152,7 @@ __global__ __launch_bounds__(MLP_WG) void k_gemm(GemmArgs g) {
     if (lane == 0) red[wave] = e2;
     __syncthreads();
     if (threadIdx.x == 0)
-      g.partial[(size_t)row_tile * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+      g.partial[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
   }
 }
 
@@ -337,15 +334,34 @@ void release(ekpnp_mlp* m) {
 }
 
 int rows_of(int B) { return (B + KSTEP - 1) / KSTEP * KSTEP; }
-// x: columns; y and z: rows, which in y alone would end at 65535 (of a launch's
-// 65536) tiles, a batch of 1,048,560
-constexpr int MAX_GRID_Y = 65535;
-dim3 gemm_grid(int N, int rows) {
-  const int tiles = rows / TILE, z = (tiles + MAX_GRID_Y - 1) / MAX_GRID_Y;
-  return dim3((N / TILE + MLP_WG / 64 - 1) / (MLP_WG / 64), (tiles + z - 1) / z, z);
-}
+int gemm_columns(int N) { return (N / TILE + MLP_WG / 64 - 1) / (MLP_WG / 64); }  // work-groups a row of tiles
 // squared-error sums of a batch of rows (k_gemm<EPI_LOSS>)
-size_t loss_partials(int N, int rows) { return (size_t)gemm_grid(N, rows).x * (rows / TILE); }
+size_t loss_partials(int N, int rows) { return (size_t)gemm_columns(N) * (rows / TILE); }
+
+// k_gemm over rows (a multiple of 32) rows.  Row tiles lie on the grid's y, which
+// holds 65536: a larger batch, above 1,048,560, takes several launches, each
+// with its operands' first rows.  (The grid's z instead costs the launches of
+// ordinary batches 0.3 us each: reading the grid's size, a bound to check.)
+template <int EPI>
+void launch_gemm(GemmArgs g, int rows, hipStream_t s) {
+  constexpr int MOST = 65535 * TILE;
+  const int gx = gemm_columns(g.N);
+  for (;;) {
+    const int n = std::min(rows, MOST);
+    hipLaunchKernelGGL(k_gemm<EPI>, dim3(gx, n / TILE), dim3(MLP_WG), 0, s, g);
+    rows -= n;
+    if (rows == 0) return;
+    const size_t o = (size_t)n * g.N;
+    g.A += (size_t)n * g.K;
+    g.M -= n;
+    if (g.z) g.z += o;
+    if (g.t) g.t += o;
+    if (g.g) g.g += o;
+    if (g.c) g.c += o;
+    if (g.ct) g.ct += n;
+    if (g.partial) g.partial += loss_partials(g.N, n);
+  }
+}
 
 // layers 1 .. last of the forward pass (hidden layers, or with L + 1 the
 // linear output too); train: the transposed activations are written as well
@@ -361,19 +377,17 @@ hipError_t forward(ekpnp_mlp* m, const float* x_host, int B, int last, bool trai
     g.A = m->a[l - 1];
     g.B = m->pbf + m->off_w[l];
     g.M = B;
-    g.row_tiles = rows / TILE;
     g.N = m->out_dim[l];
     g.K = m->in_dim[l];
     g.bias = m->p32 + m->off_b[l];
     g.z = m->z[l];
-    const dim3 grid = gemm_grid(g.N, rows);
     if (l <= m->L) {
       g.c = m->a[l];
       g.ct = train ? m->at[l] : nullptr;
       g.ldt = m->rows;
-      hipLaunchKernelGGL(k_gemm<EPI_HIDDEN>, grid, dim3(MLP_WG), 0, m->stream, g);
+      launch_gemm<EPI_HIDDEN>(g, rows, m->stream);
     } else {
-      hipLaunchKernelGGL(k_gemm<EPI_OUT>, grid, dim3(MLP_WG), 0, m->stream, g);
+      launch_gemm<EPI_OUT>(g, rows, m->stream);
     }
   }
   return hipGetLastError();
@@ -405,15 +419,13 @@ int loss_grad(ekpnp_mlp* m, const float* x_host, const float* t_host, int B) {
       g.z = m->z[l];
     }
     g.M = B;
-    g.row_tiles = rows / TILE;
     g.N = m->out_dim[l];
     g.g = m->g[l];
     g.c = m->gb[l];
     g.ct = m->gt[l];
     g.ldt = m->rows;
-    const dim3 grid = gemm_grid(g.N, rows);
-    if (l == L + 1) hipLaunchKernelGGL(k_gemm<EPI_LOSS>, grid, dim3(MLP_WG), 0, m->stream, g);
-    else hipLaunchKernelGGL(k_gemm<EPI_DGELU>, grid, dim3(MLP_WG), 0, m->stream, g);
+    if (l == L + 1) launch_gemm<EPI_LOSS>(g, rows, m->stream);
+    else launch_gemm<EPI_DGELU>(g, rows, m->stream);
   }
   hipLaunchKernelGGL(k_wgrad, dim3(m->n_wgrad), dim3(MLP_WG), 0, m->stream, m->layers, L + 1, m->g32, m->rows, B);
   MHIP(m, hipGetLastError());

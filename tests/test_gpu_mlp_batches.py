@@ -10,7 +10,7 @@ from ekpnp import surrogate as S
 pytestmark = pytest.mark.gpu
 
 
-# 65535 row tiles (one z), 65538 (the last z not full), 67584
+# 65535 row tiles (one launch), 65538 and 67584 (two)
 @pytest.mark.parametrize("batch", [1048560, 1048600, 1081344])
 def test_more_row_tiles_than_a_launch_dimension(batch):
     net = S.MLP(n_in=5, n_hidden=32, n_layers=1, n_out=32, max_batch=batch, seed=3)
@@ -18,12 +18,13 @@ def test_more_row_tiles_than_a_launch_dimension(batch):
     rng = np.random.default_rng(1)
     x = rng.uniform(-1, 1, (batch, 5)).astype(np.float32)
     y = net.forward(x)
-    half = (batch + 31) // 32 * 16  # about where z = 1 begins
-    for a in (0, half - 2048, batch - 4096):  # a row's outputs depend on that row alone
+    half = (batch + 31) // 32 * 16
+    for a in (0, half - 2048, 1048560 - 4096, batch - 4096):  # a row's outputs depend on that row alone
         assert np.array_equal(y[a:a + 4096], ref.forward(x[a:a + 4096])), a
-    # targets that the network meets exactly but for 264 rows, on both sides of the
-    # boundary between the two z and at the end
-    rows = np.r_[half - 66:half + 66, batch - 132:batch]
+    # targets that the network meets exactly but for 264 rows, before (beyond one launch's: on
+    # both sides of) its last row and at the end
+    edge = min(1048560, batch - 198)
+    rows = np.r_[edge - 66:edge + 66, batch - 132:batch]
     t = y.copy()
     t[rows] += rng.standard_normal((264, 32)).astype(np.float32)
     loss, g = net.loss_grad(x, t)
