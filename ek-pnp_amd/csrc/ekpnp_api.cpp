@@ -277,8 +277,8 @@ ChanDesc make_desc(const ekpnp_channel_params& p, int precision) {
 // lie there a step later, and one that does not evicts psi and the spectrum for
 // nothing.  So as many planes as fit LBM_CACHE_BYTES: the largest count of
 // LBM_CACHED whose planes, both lattices of them (bytes: all 27), stay within
-// it (FP64 storage, whose nodes spend longer on a plane: LBM_CACHE_BYTES_FP64, but
-// for the first two planes).  k_lbm (the widths the row kernel does not take, FP64 storage) gains from
+// it (FP64 storage without narrow channels: LBM_CACHE_BYTES_FP64, but for the first
+// two planes).  k_lbm (the widths the row kernel does not take, FP64 storage) gains from
 // whole lattices a little longer, up to LBM_CACHE_BYTES_WHOLE, and with FP32
 // storage and narrow channels only from whole ones; the row kernel and FP64
 // storage stream what is below LBM_CACHE_BYTES_MIN, which the L2 caches serve
@@ -295,7 +295,8 @@ ChanDesc make_desc(const ekpnp_channel_params& p, int precision) {
 //   512x1800    fp64  398 MB  98.4 (13)                [105.8 with 9]
 //   1024x1300   fp64  575 MB  140.9 (9)                [146.0 with 6, 147.6 with 13]
 //   1000x1300   fp64  562 MB  332.7 (9)                [340.5 with 6]
-//   64x128 x150 fp64  531 MB  121.9 (9)                [121.3 with 6]
+//   64x128 x150 fp64  531 MB  121.3 (6)                [121.9 with 9]
+//   4x200 x700  fp64  242 MB  79.5 (13)                [81.2 with 18]
 //   1024x2000   fp64  885 MB  191.3 (6)                [205.8 with 4, 218.9 with 9]
 //   4096x640    fp64 1132 MB  282.1 -> 256.6 (4)       [262.4 with 2, 269.1 with 6]
 //   4096x1330   fp64 2353 MB  531.9 (0)                [540.0 with 2]
@@ -316,15 +317,15 @@ ChanDesc make_desc(const ekpnp_channel_params& p, int precision) {
 //   n_x = 8 x4000    1178 MB  418.6 (0)                [433.1 with 2]
 constexpr double LBM_CACHE_BYTES = 160e6, LBM_CACHE_BYTES_FP64 = 200e6, LBM_CACHE_BYTES_WHOLE = 230e6,
                  LBM_CACHE_BYTES_MIN = 80e6;
-constexpr int LBM_CACHE_PART_NX = 256;  // narrowest channel of FP32 storage k_lbm with a part of the planes cached
+// narrowest channel of k_lbm with a part (FP64 storage: a larger part) of the planes cached
+constexpr int LBM_CACHE_PART_NX = 256;
 
 int lbm_cached_planes(double bytes, bool fp64, bool rows, int min_nx) {
   if (!rows && bytes <= LBM_CACHE_BYTES_WHOLE && (!fp64 || bytes >= LBM_CACHE_BYTES_MIN)) return LBM_CACHED_ALL;
   if ((!rows && !fp64 && min_nx < LBM_CACHE_PART_NX) || bytes < LBM_CACHE_BYTES_MIN) return 0;
+  const double most = fp64 && min_nx >= LBM_CACHE_PART_NX ? LBM_CACHE_BYTES_FP64 : LBM_CACHE_BYTES;
   int i = 0;
-  while (i < LBM_CACHED_ALL &&
-         LBM_CACHED[i + 1] / 27.0 * bytes <= (fp64 && i > 0 ? LBM_CACHE_BYTES_FP64 : LBM_CACHE_BYTES))
-    ++i;
+  while (i < LBM_CACHED_ALL && LBM_CACHED[i + 1] / 27.0 * bytes <= (i > 0 ? most : LBM_CACHE_BYTES)) ++i;
   return i;
 }
 

@@ -1,8 +1,8 @@
 """The row collide-stream kernel against the general one (EKPNP_LBM_ROWS=0),
 each in its own launch: at the widths that a small context alone would take
-through the one-launch kernel, and on a large channel.  The kernels round the flux products of the storage references and one
-sum of squares differently, in FP64; a stored FP32 value may then differ by a unit in its
-last place."""
+through the one-launch kernel, and on a large channel.  The kernels round the
+flux products of the storage references and one sum of squares differently, in
+FP64; a stored FP32 value may then differ by a unit in its last place."""
 import numpy as np
 import pytest
 

@@ -67,6 +67,9 @@ def cached(steps):
     ([(4096, 640)], "fp64", {}, 4),            # 1132
     ([(1024, 514)], "fp64", {}, 27),           # 227
     ([(512, 256)], "fp64", {}, 0),             # 57
+    ([(256, 256)] * 14, "fp64", {}, 13),       # 396
+    ([(255, 256)] * 14, "fp64", {}, 9),        # 395: narrow channels keep to the smaller limit
+    ([(4, 200)] * 700, "fp64", {}, 13),        # 242
     # the batches of test_gpu_lbm_cache.py, and the last narrow one below its limit
     *[([(1024, 64)] * n, "fp32", {}, w) for n, w in ((5, 0), (6, 27), (11, 27), (12, 18), (16, 18), (20, 13), (30, 9),
                                                      (45, 6), (70, 4), (100, 2), (160, 0))],
